@@ -207,7 +207,6 @@ NepEngine::NepEngine(const std::string& path)
   dalloc(&params_, im.data.size(), "parameters");
   check(hipMemcpy(params_, im.data.data(), im.data.size() * sizeof(float), hipMemcpyHostToDevice),
         "upload parameters");
-  upload_angular_constants(derive_angular_constants());
   dm_.T = T;
   dm_.nR = m.nR;
   dm_.nA = m.nA;

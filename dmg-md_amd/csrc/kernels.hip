@@ -20,183 +20,11 @@
 //    ZBL, and writes FP64 force/virial.  No floating-point atomics anywhere:
 //    results are deterministic and independent of launch order.
 //  * Integrator and thermo in FP64, thermo sums compensated (two-sum).
-#include "device_common.hpp"
-
-#include <hip/hip_ext.h>
+#include "nep_math.hpp"
 
 #include <cmath>
 
 namespace dmgx {
-
-__constant__ float c_c3[(kMaxL + 1) * (kMaxL + 1) - 1];
-__constant__ float c_zc[kMaxL + 1][kMaxL + 1][kMaxL + 1];
-__constant__ float c_c4[5];
-__constant__ float c_c5;
-
-void upload_angular_constants(const AngularConstants& a)
-{
-  (void)hipMemcpyToSymbol(HIP_SYMBOL(c_c3), a.c3, sizeof(a.c3));
-  (void)hipMemcpyToSymbol(HIP_SYMBOL(c_zc), a.zc, sizeof(a.zc));
-  (void)hipMemcpyToSymbol(HIP_SYMBOL(c_c4), a.c4, sizeof(a.c4));
-  (void)hipMemcpyToSymbol(HIP_SYMBOL(c_c5), &a.c5, sizeof(a.c5));
-}
-
-// ---------------------------------------------------------------------------
-// helpers
-// ---------------------------------------------------------------------------
-
-// cosine cutoff (nep_utilities.cuh:317-342).  cos and sin of pi d/rc come
-// from the hardware sine/cosine (v_sin_f32 / v_cos_f32), whose argument is in
-// revolutions: 0.5 d/rc lies in [0, 0.5), far inside their [-256, 256]
-// domain, with absolute errors near 1e-7.
-__device__ __forceinline__ void cutoff_fc(float rc, float rcinv, float d, float& fc)
-{
-  fc = d < rc ? 0.5f * __builtin_amdgcn_cosf(0.5f * d * rcinv) + 0.5f : 0.0f;
-}
-__device__ __forceinline__ void cutoff_fc_fcp(float rc, float rcinv, float d, float& fc, float& fcp)
-{
-  if (d < rc) {
-    const float rev = 0.5f * d * rcinv;
-    const float sn = __builtin_amdgcn_sinf(rev), cs = __builtin_amdgcn_cosf(rev);
-    fc = 0.5f * cs + 0.5f;
-    fcp = -1.57079633f * sn * rcinv;
-  } else {
-    fc = 0.0f;
-    fcp = 0.0f;
-  }
-}
-
-// Chebyshev radial basis f_k = (T_k(x)+1)/2 fc, x = 2(d/rc-1)^2-1; entries
-// k >= kn are zero
-template <int K>
-__device__ __forceinline__ void cheb(int kn, float rcinv, float d, float fc, float* f)
-{
-  const float t = d * rcinv - 1.0f;
-  const float x = 2.0f * t * t - 1.0f;
-  const float hfc = 0.5f * fc;
-  float tm2 = 1.0f, tm1 = x;
-  f[0] = fc;
-  if (K > 1) f[1] = (x + 1.0f) * hfc;
-#pragma unroll
-  for (int k = 2; k < K; ++k) {
-    const float tk = 2.0f * x * tm1 - tm2;
-    tm2 = tm1;
-    tm1 = tk;
-    f[k] = k < kn ? (tk + 1.0f) * hfc : 0.0f;
-  }
-}
-
-// basis and d/dd (T_k' = k U_{k-1})
-template <int K>
-__device__ __forceinline__ void cheb_d(int kn, float rcinv, float d, float fc, float fcp, float* f, float* fp)
-{
-  const float t = d * rcinv - 1.0f;
-  const float x = 2.0f * t * t - 1.0f;
-  const float dx = 4.0f * t * rcinv;  // dx/dd
-  f[0] = fc;
-  fp[0] = fcp;
-  float tm2 = 1.0f, tm1 = x, um2 = 1.0f, um1 = 2.0f * x;
-  if (K > 1) {
-    const float v = 0.5f * (x + 1.0f);
-    f[1] = v * fc;
-    fp[1] = 0.5f * dx * fc + v * fcp;
-  }
-#pragma unroll
-  for (int k = 2; k < K; ++k) {
-    const float tk = 2.0f * x * tm1 - tm2;
-    const float v = 0.5f * (tk + 1.0f);
-    const float der = 0.5f * k * um1 * dx;  // (T_k'/2) dx/dd, T_k' = k U_{k-1}
-    f[k] = k < kn ? v * fc : 0.0f;
-    fp[k] = k < kn ? der * fc + v * fcp : 0.0f;
-    tm2 = tm1;
-    tm1 = tk;
-    const float uk = 2.0f * x * um1 - um2;
-    um2 = um1;
-    um1 = uk;
-  }
-}
-
-// real solid harmonics Y_{L,m}(u), L=1..LM, packed at L*L-1 (+2m-1 re, +2m im)
-template <int LM>
-__device__ __forceinline__ void harmonics(float ux, float uy, float uz, float* Y)
-{
-  float zp[LM + 1];
-  zp[0] = 1.0f;
-#pragma unroll
-  for (int k = 1; k <= LM; ++k) zp[k] = zp[k - 1] * uz;
-  float pr[LM + 1], pim[LM + 1];
-  pr[0] = 1.0f;
-  pim[0] = 0.0f;
-#pragma unroll
-  for (int k = 1; k <= LM; ++k) {
-    pr[k] = pr[k - 1] * ux - pim[k - 1] * uy;
-    pim[k] = pr[k - 1] * uy + pim[k - 1] * ux;
-  }
-#pragma unroll
-  for (int L = 1; L <= LM; ++L) {
-#pragma unroll
-    for (int m = 0; m <= L; ++m) {
-      float Z = 0.0f;
-#pragma unroll
-      for (int k = (L - m) & 1; k <= L - m; k += 2) Z += c_zc[L][m][k] * zp[k];
-      const int b = L * L - 1;
-      if (m == 0) {
-        Y[b] = Z;
-      } else {
-        Y[b + 2 * m - 1] = Z * pr[m];
-        Y[b + 2 * m] = Z * pim[m];
-      }
-    }
-  }
-}
-
-// Screened-Coulomb ZBL pair energy f(d) and df/dd with the cosine switch
-// between r_in and r_out (nep_utilities.cuh:347-433); zp is one pair's
-// {1/a, Zi Zj K_C, r_in, r_out, (c_k, d_k) x4} record.
-__device__ __forceinline__ void zbl_pair(const float* __restrict__ zp, float d, float dinv, float& f, float& fp)
-{
-  const float x = d * zp[0];
-  float phi = 0.0f, dphi = 0.0f;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const float t = zp[4 + 2 * k] * expf(-zp[5 + 2 * k] * x);
-    phi += t;
-    dphi -= zp[5 + 2 * k] * t;
-  }
-  const float vv = zp[1] * phi * dinv;
-  const float vp = zp[1] * dphi * zp[0] * dinv - vv * dinv;
-  const float r1 = zp[2], r2 = zp[3];
-  float fc = 0.0f, fcp = 0.0f;
-  if (d < r1) {
-    fc = 1.0f;
-  } else if (d < r2) {
-    const float wv = 3.14159265f / (r2 - r1);
-    float sn, cs;
-    sincosf(wv * (d - r1), &sn, &cs);
-    fc = 0.5f * cs + 0.5f;
-    fcp = -0.5f * wv * sn;
-  }
-  f = vv * fc;
-  fp = vp * fc + vv * fcp;
-}
-
-// Loads the first kp floats of a 16-byte aligned row as float4s into out[0..KP)
-// (kp <= KP, both multiples of 4); entries past kp are left as they are.
-template <int KP>
-__device__ __forceinline__ void load_row4(const float* __restrict__ row, int kp, float* out)
-{
-  const float4* q = reinterpret_cast<const float4*>(row);
-#pragma unroll
-  for (int c = 0; c < KP / 4; ++c) {
-    if (4 * c < kp) {
-      const float4 t = q[c];
-      out[4 * c] = t.x;
-      out[4 * c + 1] = t.y;
-      out[4 * c + 2] = t.z;
-      out[4 * c + 3] = t.w;
-    }
-  }
-}
 
 // ---------------------------------------------------------------------------
 // per-step typewise filter (nep.cu:503-561) into compact edge rows
@@ -223,12 +51,6 @@ __device__ __forceinline__ void load_row4(const float* __restrict__ row, int kp,
 #ifndef DMGX_GATHER_BATCH
 #define DMGX_GATHER_BATCH 2
 #endif
-// the fused descriptor kernel's workgroup (256: three workgroups per CU by
-// LDS; 512, which would allow four wavefronts per SIMD, measured no faster)
-#ifndef DMGX_DESC_BLOCK
-#define DMGX_DESC_BLOCK 256
-#endif
-constexpr int kDescBlock = DMGX_DESC_BLOCK;
 constexpr int kFilterLanes = DMGX_FILTER_LANES;
 constexpr int kFilterBatch = DMGX_FILTER_BATCH;
 constexpr int kGatherLanes = DMGX_GATHER_LANES;
@@ -405,948 +227,6 @@ __global__ __launch_bounds__(kBlock) void k_split_reverse(int c1, int c2, int nb
       }
     }
     w.cq[arow + a] = v;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// fused descriptor + ANN + adjoint + angular partial forces
-// ---------------------------------------------------------------------------
-
-// ANN modes of the descriptor kernel
-enum : int { kAnnValu = 0, kAnnMfma32 = 1, kAnnMfmaBf16 = 2, kAnnMfmaSplit = 3 };
-
-// multi-type models with at most this many types keep their coefficient
-// blocks in LDS
-constexpr int kTypesLds = 4;
-// multi-type models with at most this many types run their ANN on the
-// matrix cores: every type's weights staged in LDS, one GEMM pass per type
-// present in the wavefront, each atom taking the pass of its own type
-constexpr int kTypesMfma = 2;
-
-template <int NR, int KR, int NA, int KA, int LM, bool Q222, bool Q1111, bool ONE, bool EXACT, int ANN = kAnnValu,
-          bool CL = false>
-struct Cfg {
-  static constexpr int nr = NR, kr = KR, na = NA, ka = KA, lm = LM, ann = ANN;
-  static constexpr bool q222 = Q222, q1111 = Q1111, one = ONE, exact = EXACT;
-  static constexpr bool cl = CL && EXACT && !ONE;  // coefficient blocks in LDS (T <= kTypesLds)
-  // type pairs of the LDS tables: every pair of up to kMaxTypes types, or
-  // the types an LDS-table instance serves (kTypesMfma with the matrix-core
-  // ANN, which stages every type's weights too)
-  static constexpr int ltypes = !cl ? kMaxTypes : (ANN != kAnnValu ? kTypesMfma : kTypesLds);
-  static constexpr int nabc = (LM + 1) * (LM + 1) - 1;
-  static constexpr int numl = LM + (Q222 ? 1 : 0) + (Q1111 ? 1 : 0);
-  static constexpr int dim = NR + NA * numl;
-};
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-
-// float -> bfloat16, round to nearest even (inputs are finite)
-__device__ __forceinline__ short to_bf16(float x)
-{
-  unsigned u = __float_as_uint(x);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (short)(u >> 16);
-}
-
-// LDS floats per wavefront of the matrix-core ANN: 64 rows of DMAX+1 (odd
-// stride), then 64 energies
-template <int DMAX>
-constexpr int ann_lds_floats() { return 64 * (DMAX + 1) + 128; }
-
-// ANN of the 64 atoms of a wavefront on the matrix cores (single-type
-// model, H <= 64).  Lane l holds atom l's scaled descriptor q[0..D).
-//   GEMM 1: Z^T[h][atom] = sum_d W0[h][d] Q[atom][d]   (A = W0, B = Q^T)
-//   x = tanh(Z - b0), E = sum_h w1 x, G = w1 (1 - x^2)
-//   GEMM 2: Fp[atom][d] = sum_h G[atom][h] W0[h][d]     (A = G, B = W0)
-// With the 16x16 output layout (lane l, register r) -> (row 4(l/16)+r,
-// column l%16), the GEMM-1 accumulator of lane l holds atom 16nt + l%16 at
-// hidden units 16mt + 4(l/16) + r; ordering GEMM 2's contraction index as
-// (mt, r) makes those registers its A operand as they are.  Fp rows and the
-// energies go back to their lanes through LDS.  BF16 rounds Q, W0 and G to
-// bfloat16 (16x16x16 bf16 MFMA, FP32 accumulation); FP32 uses the 16x16x4
-// FP32 MFMA (exact products).
-// LDS copy of one type's ANN weights for the matrix-core path: W0 rows
-// padded to 64 hidden units with an odd row stride (no bank conflicts), then
-// b0 and w1 (zero past H)
-template <int DMAX>
-constexpr int ann_w_stride() { return DMAX + 1; }
-// floats of W0 rows: 64 x WS floats, or with SPLIT three bfloat16 parts of
-// 64 x WS shorts each (96 x WS floats); then b0 and w1
-template <int DMAX, bool SPLIT = false>
-constexpr int ann_w_floats() { return (SPLIT ? 96 : 64) * ann_w_stride<DMAX>() + 128; }
-
-// bfloat16 -> float (exact)
-__device__ __forceinline__ float from_bf16(short b) { return __uint_as_float(((unsigned)(unsigned short)b) << 16); }
-
-// x = hi + mid + lo + r with hi = bf16(x), mid = bf16(x - hi),
-// lo = bf16(x - hi - mid) (each difference exact in FP32), |r| <= 2^-27 |x|
-struct Bf16Split {
-  short hi, mid, lo;
-};
-__device__ __forceinline__ Bf16Split split_bf16(float x)
-{
-  const short hi = to_bf16(x);
-  const float r1 = x - from_bf16(hi);
-  const short mid = to_bf16(r1);
-  return Bf16Split{hi, mid, to_bf16(r1 - from_bf16(mid))};
-}
-
-// SPLIT: W0 is stored as its three bfloat16 parts, shorts [64][WS] each
-// (hi, then mid, then lo), in place of the float rows
-template <int DMAX, bool SPLIT = false>
-__device__ __forceinline__ void stage_ann_weights(const DevModel& m, int D, float* __restrict__ ws, int t = 0)
-{
-  constexpr int WS = ann_w_stride<DMAX>();
-  const int H = m.H;
-  const float* __restrict__ w0 = m.w0 + (size_t)t * H * D;
-  const float* __restrict__ b0 = m.b0 + (size_t)t * H;
-  const float* __restrict__ w1 = m.w1 + (size_t)t * H;
-  short* __restrict__ whl = reinterpret_cast<short*>(ws);
-  for (int k = threadIdx.x; k < 64 * WS; k += blockDim.x) {
-    const int h = k / WS, d = k % WS;
-    const float x = (h < H && d < D) ? w0[h * D + d] : 0.0f;
-    if (SPLIT) {
-      const Bf16Split p = split_bf16(x);
-      whl[k] = p.hi;
-      whl[64 * WS + k] = p.mid;
-      whl[128 * WS + k] = p.lo;
-    } else {
-      ws[k] = x;
-    }
-  }
-  for (int h = threadIdx.x; h < 64; h += blockDim.x) {
-    constexpr int bo = (SPLIT ? 96 : 64) * WS;
-    ws[bo + h] = h < H ? b0[h] : 0.0f;
-    ws[bo + 64 + h] = h < H ? w1[h] : 0.0f;
-  }
-}
-
-
-// orders this wavefront's LDS writes before its later LDS reads (each
-// wavefront works in its own LDS region, so no workgroup barrier is needed)
-__device__ __forceinline__ void wave_lds_sync()
-{
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// MT: multi-type (ti is the lane's type, T the number of types <=
-// kTypesMfma, ws holds the types' weight blocks one after another): per
-// type present in the wavefront one pass over the hidden tiles whose
-// activation gradients and energies count only for atoms of that type.
-template <int DMAX, int MODE, bool MT = false>
-__device__ __forceinline__ void ann_mfma(const DevModel& m, int D, const float* q, float* Fp, float& E,
-                                         float* __restrict__ lds, const float* __restrict__ ws, int ti = 0,
-                                         int T = 1)
-{
-  // MODE kAnnMfma32: FP32 operands (16x16x4 FP32 MFMA, exact products);
-  // kAnnMfmaBf16: bfloat16 operands; kAnnMfmaSplit: every operand split
-  // into three bfloat16 parts (hi + mid + lo) and each product formed from
-  // the six part products of relative size above 2^-24 (hi*hi, hi*mid,
-  // mid*hi, mid*mid, hi*lo, lo*hi; 16x16x16 bf16 MFMAs, FP32 accumulation,
-  // smallest first): FP32 accuracy from bfloat16 products, the "bf16x6"
-  // method of Henry, Tang and Heinecke (ARITH 2019)
-  constexpr bool BF16 = MODE == kAnnMfmaBf16;
-  constexpr bool X3 = MODE == kAnnMfmaSplit;
-  constexpr int DS = DMAX + 1;
-  constexpr int DT = (DMAX + 15) / 16;
-  const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
-  float* Qs = lds;
-  float* Es = lds + 64 * DS;
-  int* Ts = reinterpret_cast<int*>(lds + 64 * DS + 64);
-#pragma unroll
-  for (int d = 0; d < DMAX; ++d) Qs[lane * DS + d] = d < D ? q[d] : 0.0f;
-  unsigned present = 1u;
-  if (MT) {
-    Ts[lane] = ti;
-    present = 0u;
-    for (int t = 0; t < T; ++t)
-      if (__any(ti == t)) present |= 1u << t;
-  }
-  wave_lds_sync();
-  const int H = m.H, HT = (H + 15) >> 4;
-  constexpr int WS = ann_w_stride<DMAX>();
-#pragma unroll 1
-  for (int nt = 0; nt < 4; ++nt) {
-    const float* qrow = Qs + (16 * nt + lr) * DS;
-    // split descriptor operands of this atom tile, reused by every hidden tile
-    s16x4 qh[X3 ? DT : 1], qm[X3 ? DT : 1], ql[X3 ? DT : 1];
-    if (X3) {
-#pragma unroll
-      for (int ks = 0; ks < DT; ++ks)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int d = 16 * ks + 4 * lg + c;
-          const Bf16Split p = split_bf16(d < D ? qrow[d] : 0.0f);
-          qh[ks][c] = p.hi;
-          qm[ks][c] = p.mid;
-          ql[ks][c] = p.lo;
-        }
-    }
-    f32x4 facc[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) facc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float ep = 0.0f;
-    const int at = MT ? Ts[16 * nt + lr] : 0;  // type of this lane's atom in the tile
-    // the type loop is unrolled over its compile-time bound: a runtime-bounded
-    // loop that skips absent types gave wrong accumulators in GEMM 2 here
-    // (forces off by 5% with exact energies), the unrolled form does not
-#pragma unroll
-    for (int t = 0; t < (MT ? kTypesMfma : 1); ++t) {
-      if (t >= T || !((present >> t) & 1u)) continue;
-      const bool mine = !MT || at == t;
-      // [64][WS] floats (or three [64][WS] bfloat16 parts), zero-padded
-      const float* __restrict__ W0 = ws + (size_t)t * ann_w_floats<DMAX, X3>();
-      const float* __restrict__ b0 = W0 + (X3 ? 96 : 64) * WS;
-      const float* __restrict__ w1 = b0 + 64;
-      // one tile of 16 hidden units at a time: GEMM 1, activation, and its
-      // share of GEMM 2, so that only one accumulator tile is live
-#pragma unroll 1
-      for (int mt = 0; mt < HT; ++mt) {
-        f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-        const int ha = 16 * mt + lr;
-        const short* __restrict__ Wh = reinterpret_cast<const short*>(W0);
-        const short* __restrict__ Wm = Wh + 64 * WS;
-        const short* __restrict__ Wl = Wh + 128 * WS;
-        if (X3) {
-#pragma unroll
-          for (int ks = 0; ks < DT; ++ks) {
-            s16x4 ah, am, al;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-              // columns past the row stride would read the next row or, past
-              // the last row, the float biases as bfloat16 pairs (possibly
-              // NaN patterns): they hold zeros
-              const int d = 16 * ks + 4 * lg + c;
-              ah[c] = d < WS ? Wh[ha * WS + d] : (short)0;
-              am[c] = d < WS ? Wm[ha * WS + d] : (short)0;
-              al[c] = d < WS ? Wl[ha * WS + d] : (short)0;
-            }
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(al, qh[ks], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ah, ql[ks], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(am, qm[ks], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(am, qh[ks], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ah, qm[ks], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ah, qh[ks], acc, 0, 0, 0);
-          }
-        } else if (!BF16) {
-#pragma unroll
-          for (int ks = 0; ks < (DMAX + 3) / 4; ++ks) {
-            const int d = 4 * ks + lg;
-            const float bq = d < D ? qrow[d] : 0.0f;
-            const float a = W0[ha * WS + d];
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bq, acc, 0, 0, 0);
-          }
-        } else {
-#pragma unroll
-          for (int ks = 0; ks < (DMAX + 15) / 16; ++ks) {
-            s16x4 bq, a;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-              const int d = 16 * ks + 4 * lg + c;
-              bq[c] = to_bf16(d < D ? qrow[d] : 0.0f);
-              a[c] = to_bf16(W0[ha * WS + d]);
-            }
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bq, acc, 0, 0, 0);
-          }
-        }
-        float G[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int h = 16 * mt + 4 * lg + r;
-          G[r] = 0.0f;
-          if (h < H && mine) {
-            const float x = tanhf(acc[r] - b0[h]);
-            ep += w1[h] * x;
-            G[r] = w1[h] * (1.0f - x * x);
-          }
-        }
-        if (X3) {
-          s16x4 gh, gm, gl;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const Bf16Split p = split_bf16(G[r]);
-            gh[r] = p.hi;
-            gm[r] = p.mid;
-            gl[r] = p.lo;
-          }
-#pragma unroll
-          for (int dt = 0; dt < DT; ++dt) {
-            const int d = 16 * dt + lr;
-            s16x4 bh, bm, bl;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-              const int h = 16 * mt + 4 * lg + c;
-              bh[c] = d < WS ? Wh[h * WS + d] : (short)0;
-              bm[c] = d < WS ? Wm[h * WS + d] : (short)0;
-              bl[c] = d < WS ? Wl[h * WS + d] : (short)0;
-            }
-            facc[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(gl, bh, facc[dt], 0, 0, 0);
-            facc[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(gh, bl, facc[dt], 0, 0, 0);
-            facc[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(gm, bm, facc[dt], 0, 0, 0);
-            facc[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(gm, bh, facc[dt], 0, 0, 0);
-            facc[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(gh, bm, facc[dt], 0, 0, 0);
-            facc[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(gh, bh, facc[dt], 0, 0, 0);
-          }
-        } else if (!BF16) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int h = 16 * mt + 4 * lg + r;
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) {
-              const int d = 16 * dt + lr;
-              const float bw = W0[h * WS + d];
-              facc[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(G[r], bw, facc[dt], 0, 0, 0);
-            }
-          }
-        } else {
-          s16x4 a;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) a[r] = to_bf16(G[r]);
-#pragma unroll
-          for (int dt = 0; dt < DT; ++dt) {
-            const int d = 16 * dt + lr;
-            s16x4 bw;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-              const int h = 16 * mt + 4 * lg + c;
-              bw[c] = to_bf16(W0[h * WS + d]);
-            }
-            facc[dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bw, facc[dt], 0, 0, 0);
-          }
-        }
-      }
-    }  // types
-    ep += __shfl_xor(ep, 16);
-    ep += __shfl_xor(ep, 32);
-    if (lg == 0) Es[16 * nt + lr] = ep;
-    // this tile's Fp rows replace its (already consumed) Q rows
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int d = 16 * dt + lr;
-        if (d < DMAX) Qs[(16 * nt + 4 * lg + r) * DS + d] = facc[dt][r];
-      }
-  }
-  wave_lds_sync();
-#pragma unroll
-  for (int d = 0; d < DMAX; ++d) Fp[d] = d < D ? Qs[lane * DS + d] : 0.0f;
-  E = Es[lane];
-}
-
-// Static LDS of a descriptor instance: pair tables, coefficient blocks, ANN
-// weights and the per-wavefront ANN staging.  Instances stay within
-// kDescLdsMax per workgroup; where the matrix-core ANN would not, the vector
-// ANN runs.
-constexpr int kDescLdsMax = 96 * 1024;
-template <class C>
-constexpr int desc_lds_bytes()
-{
-  const int pairs = C::ltypes * C::ltypes;
-  const int pcut = C::one ? 1 + 2 : 4 * pairs + 4 * pairs;  // float cutoffs, then the FP64 squares
-  const int ctab = C::cl ? pairs * (C::nr * C::kr + C::na * C::ka) : 1;
-  const int mfma = C::ann != kAnnValu;
-  const int annw = mfma ? (C::one ? 1 : kTypesMfma) * ann_w_floats<C::dim, C::ann == kAnnMfmaSplit>() : 1;
-  const int annl = mfma ? (kDescBlock / 64) * ann_lds_floats<C::dim>() : 0;
-  return 4 * (pcut + ctab + annw + annl);
-}
-
-template <int NR, int KR, int NA, int KA, bool Q2, bool Q1, bool ONE, int ANN = kAnnMfma32>
-constexpr bool mfma_ann_fits()
-{
-  // single-type instances reach two wavefronts per SIMD, so they keep two
-  // workgroups per CU (64 KiB each); multi-type ones run one either way
-  return desc_lds_bytes<Cfg<NR, KR, NA, KA, 4, Q2, Q1, ONE, true, ANN, !ONE>>() <=
-         (ONE ? 64 * 1024 : kDescLdsMax);
-}
-
-// sum of v over the P consecutive lanes of a lane group (every lane gets it)
-template <int P>
-__device__ __forceinline__ float group_sum(float v)
-{
-#pragma unroll
-  for (int off = 1; off < P; off <<= 1) v += __shfl_xor(v, off, P);
-  return v;
-}
-
-// CAND: the edges come from the candidate rows (DevWork::split).  edge, vsa
-// and eq are w.edge, w.vsa and w.eq, passed as restrict parameters: with
-// candidate rows this kernel writes them, and only through them, so the
-// model's tables stay provably unmodified (scalar loads).
-// P: lanes per atom.  With P > 1 (systems too small to fill the GPU with one
-// lane per atom) a group of P lanes shares an atom: each takes every P-th
-// edge and every P-th hidden neuron of the (vector-ALU) ANN, and the partial
-// sums are combined across the group, so every lane holds the atom's
-// descriptor, moments and derivatives.
-template <class C, bool CAND, int P = 1>
-__global__ __launch_bounds__(kDescBlock) void k_descriptor(DevBox b, DevModel m, int N, int c1, int c2, int nblocks,
-                                                       const int* __restrict__ type, double* __restrict__ pe,
-                                                       float4* __restrict__ edge, int* __restrict__ vsa,
-                                                       int* __restrict__ eq, int accumulate, DevWork w)
-{
-  constexpr int NR = C::nr, KR = C::kr, NA = C::na, KA = C::ka, LM = C::lm, NABC = C::nabc, DMAX = C::dim;
-  static_assert(P == 1 || (P == 4 && !CAND && C::ann == kAnnValu), "lane groups: the filter's rows, vector ANN");
-  const int lr = P == 1 ? 0 : (int)(threadIdx.x & (P - 1));  // lane within the atom's group
-  const int i0 = c1 + xcd_tile(nblocks) * (int)(blockDim.x / P) + (int)(threadIdx.x / P);
-  const bool active = i0 < c2;
-  // the matrix-core ANN needs every lane of the wavefront: lanes past the
-  // range carry an empty row of a valid atom and write nothing
-  const int i = active ? i0 : c1;
-  // multi-type: per type pair the float cutoffs and their inverses (radial,
-  // angular; the FP64 pair mean rounded once) and, with C::cl, the
-  // coefficient blocks [pair][n][k] (radial, then angular), staged in LDS
-  constexpr int kPairs = C::ltypes * C::ltypes;
-  static_assert(desc_lds_bytes<C>() <= kDescLdsMax, "descriptor LDS above its bound per workgroup");
-  __shared__ float pcut[C::one ? 1 : 4 * kPairs];
-  __shared__ double pcut2[C::one ? 1 : 2 * kPairs];  // FP64 squared pair cutoffs (candidate rows)
-  __shared__ float ctab[C::cl ? kPairs * (NR * KR + NA * KA) : 1];
-  if (!C::one) {
-    const int T = m.T;
-    for (int k = threadIdx.x; k < T * T; k += blockDim.x) {
-      const int p = k / T, q = k % T;
-      const double rrd = (m.rcR[p] + m.rcR[q]) * 0.5, rad = (m.rcA[p] + m.rcA[q]) * 0.5;
-      const float rr = (float)rrd, ra = (float)rad;
-      pcut[k] = rr;
-      pcut[kPairs + k] = 1.0f / rr;
-      pcut[2 * kPairs + k] = ra;
-      pcut[3 * kPairs + k] = 1.0f / ra;
-      pcut2[k] = rrd * rrd;
-      pcut2[kPairs + k] = rad * rad;
-    }
-    if (C::cl) {
-      const int nrad = T * T * NR * KR, nang = T * T * NA * KA;
-      for (int k = threadIdx.x; k < nrad + nang; k += blockDim.x) ctab[k] = k < nrad ? m.cR[k] : m.cA[k - nrad];
-    }
-    __syncthreads();
-  }
-  // candidate rows: the rebuild kernels of this step ran before this launch
-  // (the only descriptor launch of the evaluation), which closes the request
-  if (CAND && blockIdx.x == 0 && threadIdx.x == 0 && w.flags[kFlagRebuild]) {
-    w.flags[kFlagRebuild] = 0;
-    w.flags[kFlagRebuildCount] += 1;
-  }
-  if (C::ann == kAnnValu && !active) return;
-  __shared__ float ann_w[C::ann != kAnnValu ? (C::one ? 1 : kTypesMfma) * ann_w_floats<DMAX, C::ann == kAnnMfmaSplit>()
-                                           : 1];
-  if (C::ann != kAnnValu) {
-    // every type's weights (at most kTypesMfma types), staged once per workgroup
-    for (int t = 0; t < (C::one ? 1 : m.T); ++t)
-      stage_ann_weights<DMAX, C::ann == kAnnMfmaSplit>(
-          m, C::exact ? DMAX : m.D, ann_w + t * ann_w_floats<DMAX, C::ann == kAnnMfmaSplit>(), t);
-    __syncthreads();
-  }
-  const int nR = C::exact ? NR : m.nR, nA = C::exact ? NA : m.nA;
-  // 3-body order: components L <= Lm, then the 4-/5-body blocks
-  const int Lm = C::exact ? LM : m.L;
-  const int kR = C::exact ? KR : m.kR, kA = C::exact ? KA : m.kA;
-  const bool h222 = C::exact ? C::q222 : (m.has222 != 0);
-  const bool h1111 = C::exact ? C::q1111 : (m.has1111 != 0);
-  const int D = C::exact ? DMAX : m.D;
-  const int T = C::one ? 1 : m.T;
-  const int ti = C::one ? 0 : safe_type(type[i], T);
-  float rcRf[kMaxTypes], rcAf[kMaxTypes];
-  // per-type float cutoffs (the FP64 values rounded once)
-  if (C::one) {
-    rcRf[0] = (float)m.rcR[0];
-    rcAf[0] = (float)m.rcA[0];
-  }
-  int nr = 0, na = 0;
-  if (active && !CAND) {
-    nr = w.nr[i];
-    na = w.na[i];
-  }
-  // with candidate rows this kernel writes the angular edges it reads back
-  const float4* erow = edge + (size_t)i * w.MR;
-  float4* __restrict__ frow = w.f12 + (size_t)i * w.MA;
-  float q[DMAX];
-#pragma unroll
-  for (int d = 0; d < DMAX; ++d) q[d] = 0.0f;
-
-  // ---- radial descriptor: q_n = sum_j sum_k c[ti,tj,n,k] f_k(r_ij)
-  // The basis values are summed per neighbour type and contracted with the
-  // coefficients once per atom (single type: one sum; up to C::ltypes types:
-  // one per type); more types contract per edge.
-  float Fs[KR];
-#pragma unroll
-  for (int k = 0; k < KR; ++k) Fs[k] = 0.0f;
-  float Ft[C::cl ? C::ltypes : 1][KR];
-#pragma unroll
-  for (int t = 0; t < (C::cl ? C::ltypes : 1); ++t)
-#pragma unroll
-    for (int k = 0; k < KR; ++k) Ft[t][k] = 0.0f;
-  // the radial loop keeps kAhead edge records in flight (its work per edge
-  // is short); the angular loops below load the next record before using
-  // the current one and the first record of the next 128-byte line a line
-  // ahead
-  constexpr int kAhead = 8;
-  auto radial_edge = [&](const float4 r, const int tj) {
-    const float d2 = r.x * r.x + r.y * r.y + r.z * r.z;
-    const float d = d2 * __builtin_amdgcn_rsqf(d2);  // edges have d > 0
-    const float rc = C::one ? rcRf[0] : pcut[ti * T + tj];
-    const float rcinv = C::one ? 1.0f / rc : pcut[kPairs + ti * T + tj];
-    float fc;
-    cutoff_fc(rc, rcinv, d, fc);
-    float f[KR];
-    cheb<KR>(kR, rcinv, d, fc, f);
-    if (C::one) {
-#pragma unroll
-      for (int k = 0; k < KR; ++k)
-        if (k < kR) Fs[k] += f[k];
-    } else if (C::cl) {
-#pragma unroll
-      for (int t = 0; t < C::ltypes; ++t) {
-        if (t < T) {
-          const float wt = tj == t ? 1.0f : 0.0f;
-#pragma unroll
-          for (int k = 0; k < KR; ++k) Ft[t][k] = fmaf(wt, f[k], Ft[t][k]);
-        }
-      }
-    } else {
-      const float* c = m.cR + (size_t)(ti * T + tj) * nR * kR;
-#pragma unroll
-      for (int n = 0; n < NR; ++n) {
-        if (n < nR) {
-          float g = 0.0f;
-#pragma unroll
-          for (int k = 0; k < KR; ++k)
-            if (k < kR) g += c[n * kR + k] * f[k];
-          q[n] += g;
-        }
-      }
-    }
-  };
-  if (!CAND) {
-    auto ridx = [&](int e) { return e < na ? e : w.MR - 1 - (e - na); };
-    float4 ring[kAhead];
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u)
-      ring[u] = u * P + lr < nr ? erow[ridx(u * P + lr)] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (int e0 = lr; e0 < nr; e0 += kAhead * P)
-#pragma unroll
-      for (int u = 0; u < kAhead; ++u) {
-        const int e = e0 + u * P;
-        if (e >= nr) break;
-        const float4 r = ring[u];
-        if (e + kAhead * P < nr) ring[u] = erow[ridx(e + kAhead * P)];
-        radial_edge(r, C::one ? 0 : safe_type(type[__float_as_int(r.w)], T));
-      }
-    if (P > 1) {
-      // the group's partial radial sums
-      if (C::one) {
-#pragma unroll
-        for (int k = 0; k < KR; ++k) Fs[k] = group_sum<P>(Fs[k]);
-      } else if (C::cl) {
-#pragma unroll
-        for (int t = 0; t < (C::cl ? C::ltypes : 1); ++t)
-#pragma unroll
-          for (int k = 0; k < KR; ++k) Ft[t][k] = group_sum<P>(Ft[t][k]);
-      } else {
-#pragma unroll
-        for (int n = 0; n < NR; ++n) q[n] = group_sum<P>(q[n]);
-      }
-    }
-  } else {
-    // candidate rows: the FP64 minimum-image distance of every candidate
-    // (the filter's expressions, so the same edges pass), the radial sum over
-    // those within the pair's radial cutoff, and the step's angular edges
-    // (in candidate order) with their reverse indices and the candidates'
-    // slot status for the gather.  Slot indices are read eight candidates
-    // ahead, the packed positions four.
-    const int nrc = active ? w.nrc[i] : 0, nac = active ? w.nac[i] : 0;
-    const size_t vrow = (size_t)i * w.MV, arow = (size_t)i * w.MA;
-    const int* __restrict__ crow = w.cl + vrow;
-    float4* ew = edge + (size_t)i * w.MR;
-    const double4 pi = w.xq[i];
-    double cr1 = 0.0, ca1 = 0.0;
-    if (C::one) {
-      const double rr = (m.rcR[0] + m.rcR[0]) * 0.5, ra = (m.rcA[0] + m.rcA[0]) * 0.5;
-      cr1 = rr * rr;
-      ca1 = ra * ra;
-    }
-    auto cidx = [&](int e) { return e < nac ? e : w.MV - 1 - (e - nac); };
-    constexpr int kSplitAhead = 4;
-    int jr[2 * kSplitAhead];
-    double4 pr[kSplitAhead];
-#pragma unroll
-    for (int u = 0; u < 2 * kSplitAhead; ++u) jr[u] = u < nrc ? crow[cidx(u)] : 0;
-#pragma unroll
-    for (int u = 0; u < kSplitAhead; ++u) pr[u] = u < nrc ? w.xq[jr[u]] : make_double4(0.0, 0.0, 0.0, 0.0);
-    int nin = 0;
-    for (int e0 = 0; e0 < nrc; e0 += 2 * kSplitAhead)
-#pragma unroll
-      for (int u = 0; u < 2 * kSplitAhead; ++u) {
-        const int e = e0 + u;
-        if (e >= nrc) break;
-        const int j = jr[u];
-        const double4 pj = pr[u % kSplitAhead];
-        if (e + kSplitAhead < nrc) pr[u % kSplitAhead] = w.xq[jr[(u + kSplitAhead) % (2 * kSplitAhead)]];
-        if (e + 2 * kSplitAhead < nrc) jr[u] = crow[cidx(e + 2 * kSplitAhead)];
-        double x = pj.x - pi.x, y = pj.y - pi.y, z = pj.z - pi.z;
-        mic(b, x, y, z);
-        const double d2 = dist2(x, y, z);
-        int tj = 0;
-        double cr = cr1, ca = ca1;
-        if (!C::one) {
-          tj = safe_type((int)__double_as_longlong(pj.w), T);
-          cr = pcut2[ti * T + tj];
-          ca = pcut2[kPairs + ti * T + tj];
-        }
-        const bool in_r = d2 < cr;
-        const int jo = w.map.owner ? w.map.owner[j] : j;
-        const float4 r = make_float4((float)x, (float)y, (float)z, __int_as_float(jo));
-        if (e < nac) {
-          const bool in_a = in_r && d2 < ca;
-          vsa[arow + e] = in_a ? na : -1;
-          if (in_a) {
-            ew[na] = r;
-            eq[arow + na] = w.cq[arow + e];
-            ++na;
-          }
-        }
-        if (in_r) {
-          ++nin;
-          radial_edge(r, tj);
-        }
-      }
-    if (active) {
-      w.nr[i] = nin;
-      w.na[i] = na;
-    }
-  }
-  if (C::one) {
-#pragma unroll
-    for (int n = 0; n < NR; ++n) {
-      if (n < nR) {
-        float g = 0.0f;
-#pragma unroll
-        for (int k = 0; k < KR; ++k)
-          if (k < kR) g += m.cR[n * kR + k] * Fs[k];
-        q[n] = g;
-      }
-    }
-  } else if (C::cl) {
-#pragma unroll
-    for (int n = 0; n < NR; ++n) {
-      float g = 0.0f;
-#pragma unroll
-      for (int t = 0; t < C::ltypes; ++t) {
-        if (t < T) {
-          const float* c = ctab + (ti * T + t) * NR * KR + n * KR;
-#pragma unroll
-          for (int k = 0; k < KR; ++k) g += c[k] * Ft[t][k];
-        }
-      }
-      q[n] = g;
-    }
-  }
-
-  // ---- angular moments s[n][lm] = sum_j g_n(r_ij) Y_lm(u_ij)
-  float s[NA][NABC];
-#pragma unroll
-  for (int n = 0; n < NA; ++n)
-#pragma unroll
-    for (int a = 0; a < NABC; ++a) s[n][a] = 0.0f;
-  float zpe = 0.0f;
-  // each lane takes every P-th edge; the next record is loaded before the
-  // current one is used, and the first record of the next 128-byte line
-  // (eight of the lane's records) a line ahead
-  float4 rn = erow[lr < na ? lr : 0];
-  float4 ahead = erow[lr + 8 * P < na ? lr + 8 * P : 0];
-  for (int e = lr; e < na; e += P) {
-    const float4 r = rn;
-    const int en = e + P;
-    if (en < na) {
-      if ((((en - lr) / P) & 7) == 0) {
-        rn = ahead;
-        if (en + 8 * P < na) ahead = erow[en + 8 * P];
-      } else {
-        rn = erow[en];
-      }
-    }
-    const float d2 = r.x * r.x + r.y * r.y + r.z * r.z;
-    const float dinv = __builtin_amdgcn_rsqf(d2);  // hardware 1/sqrt (1 ulp); edges have d > 0
-    const float d = d2 * dinv;
-    float rc;
-    int tj = 0;
-    if (C::one) {
-      rc = rcAf[0];
-    } else {
-      tj = safe_type(type[__float_as_int(r.w)], T);
-      rc = pcut[2 * kPairs + ti * T + tj];
-    }
-    if (m.zbl) {
-      // half of each ZBL pair energy belongs to the centre; ZBL pairs are
-      // taken from the angular rows, as the reference's ZBL pass does
-      float zf, zfp;
-      zbl_pair(m.zblp + (size_t)(ti * m.T + tj) * 12, d, dinv, zf, zfp);
-      zpe += 0.5f * zf;
-    }
-    const float rcinv = C::one ? 1.0f / rc : pcut[3 * kPairs + ti * T + tj];
-    float fc;
-    cutoff_fc(rc, rcinv, d, fc);
-    float f[KA];
-    cheb<KA>(kA, rcinv, d, fc, f);
-    const float* c = C::cl ? ctab + T * T * NR * KR + (ti * T + tj) * NA * KA
-                           : m.cA + (size_t)(ti * T + tj) * nA * kA;
-    float g[NA];
-#pragma unroll
-    for (int n = 0; n < NA; ++n) {
-      g[n] = 0.0f;
-      if (n < nA) {
-#pragma unroll
-        for (int k = 0; k < KA; ++k)
-          if (k < kA) g[n] += c[n * kA + k] * f[k];
-      }
-    }
-    float Y[NABC];
-    harmonics<LM>(r.x * dinv, r.y * dinv, r.z * dinv, Y);
-#pragma unroll
-    for (int n = 0; n < NA; ++n)
-#pragma unroll
-      for (int a = 0; a < NABC; ++a) s[n][a] += g[n] * Y[a];
-  }
-  if (P > 1) {
-    // the group's partial moments and ZBL energies
-#pragma unroll
-    for (int n = 0; n < NA; ++n)
-#pragma unroll
-      for (int a = 0; a < NABC; ++a) s[n][a] = group_sum<P>(s[n][a]);
-    zpe = group_sum<P>(zpe);
-  }
-
-  // ---- invariants
-#pragma unroll
-  for (int n = 0; n < NA; ++n) {
-    if (n >= nA) break;
-#pragma unroll
-    for (int L = 1; L <= LM; ++L) {
-      float v = 0.0f;
-#pragma unroll
-      for (int a = L * L - 1; a < (L + 1) * (L + 1) - 1; ++a) v += c_c3[a] * s[n][a] * s[n][a];
-      if (L <= Lm) q[nR + (L - 1) * nA + n] = v;
-    }
-    int li = Lm;
-    if (h222) {
-      const float* x = &s[n][3];
-      q[nR + li * nA + n] = c_c4[0] * x[0] * x[0] * x[0] + c_c4[1] * x[0] * (x[1] * x[1] + x[2] * x[2]) +
-                            c_c4[2] * x[0] * (x[3] * x[3] + x[4] * x[4]) +
-                            c_c4[3] * x[3] * (x[2] * x[2] - x[1] * x[1]) + c_c4[4] * x[1] * x[2] * x[4];
-      ++li;
-    }
-    if (h1111) {
-      const float r2 = s[n][0] * s[n][0] + s[n][1] * s[n][1] + s[n][2] * s[n][2];
-      q[nR + li * nA + n] = c_c5 * r2 * r2;
-    }
-  }
-
-  // ---- ANN (nep_utilities.cuh:209-310): E = sum_h w1 tanh(w0.q - b0) - bias
-#pragma unroll
-  for (int d = 0; d < DMAX; ++d)
-    if (d < D) q[d] *= m.qs[d];
-  float Fp[DMAX];
-  float E = 0.0f;
-  if (C::ann != kAnnValu) {
-    __shared__ float ann_lds[kDescBlock / 64][ann_lds_floats<DMAX>()];
-    ann_mfma<DMAX, C::ann, !C::one>(m, D, q, Fp, E, ann_lds[threadIdx.x >> 6], ann_w, ti, T);
-  } else {
-    const int H = m.H;
-    const float* w0 = m.w0 + (size_t)ti * H * D;
-    const float* b0 = m.b0 + (size_t)ti * H;
-    const float* w1 = m.w1 + (size_t)ti * H;
-#pragma unroll
-    for (int d = 0; d < DMAX; ++d) Fp[d] = 0.0f;
-    for (int h = lr; h < H; h += P) {
-      const float* wr = w0 + (size_t)h * D;
-      float a = 0.0f;
-#pragma unroll
-      for (int d = 0; d < DMAX; ++d)
-        if (d < D) a += wr[d] * q[d];
-      const float x = tanhf(a - b0[h]);
-      E += w1[h] * x;
-      const float gq = w1[h] * (1.0f - x * x);
-#pragma unroll
-      for (int d = 0; d < DMAX; ++d)
-        if (d < D) Fp[d] += gq * wr[d];
-    }
-    if (P > 1) {
-      // the group's hidden neurons
-      E = group_sum<P>(E);
-#pragma unroll
-      for (int d = 0; d < DMAX; ++d) Fp[d] = group_sum<P>(Fp[d]);
-    }
-  }
-  E -= m.b1[0];
-  if (m.version == 5) E -= m.w1x[ti];
-#pragma unroll
-  for (int d = 0; d < DMAX; ++d)
-    if (d < D) Fp[d] *= m.qs[d];
-  const double etot = (double)E + (double)zpe;
-  if (active && lr == 0) pe[i] = accumulate ? pe[i] + etot : etot;
-
-  // ---- radial adjoint in basis space: bR[i][t][k] = sum_n Fp_n c[ti,t,n,k]
-  for (int t = 0; t < T; ++t) {
-    const float* c = C::cl ? ctab + (ti * T + t) * NR * KR : m.cR + (size_t)(ti * T + t) * nR * kR;
-    float* out = w.bR + ((size_t)i * T + t) * m.kRp;
-    if (!active) break;
-#pragma unroll
-    for (int k = 0; k < ((KR + 3) & ~3); ++k) {
-      float v = 0.0f;
-      if (k < kR) {
-#pragma unroll
-        for (int n = 0; n < NR; ++n)
-          if (n < nR) v += Fp[n] * c[n * kR + k];
-      }
-      if (k < m.kRp && (P == 1 || (k & (P - 1)) == lr)) out[k] = v;
-    }
-  }
-
-  // ---- angular adjoint a[n][lm] = dE/ds[n][lm], written over s
-#pragma unroll
-  for (int n = 0; n < NA; ++n) {
-    if (n >= nA) break;
-    float extra[8];
-#pragma unroll
-    for (int a = 0; a < 8; ++a) extra[a] = 0.0f;
-    int li = Lm;
-    if (h222) {
-      const float F = Fp[nR + li * nA + n];
-      const float* x = &s[n][3];
-      extra[3] = F * (3.0f * c_c4[0] * x[0] * x[0] + c_c4[1] * (x[1] * x[1] + x[2] * x[2]) +
-                      c_c4[2] * (x[3] * x[3] + x[4] * x[4]));
-      extra[4] = F * (2.0f * c_c4[1] * x[0] * x[1] - 2.0f * c_c4[3] * x[3] * x[1] + c_c4[4] * x[2] * x[4]);
-      extra[5] = F * (2.0f * c_c4[1] * x[0] * x[2] + 2.0f * c_c4[3] * x[3] * x[2] + c_c4[4] * x[1] * x[4]);
-      extra[6] = F * (2.0f * c_c4[2] * x[0] * x[3] + c_c4[3] * (x[2] * x[2] - x[1] * x[1]));
-      extra[7] = F * (2.0f * c_c4[2] * x[0] * x[4] + c_c4[4] * x[1] * x[2]);
-      ++li;
-    }
-    if (h1111) {
-      const float F = Fp[nR + li * nA + n];
-      const float r2 = s[n][0] * s[n][0] + s[n][1] * s[n][1] + s[n][2] * s[n][2];
-      const float k5 = 4.0f * c_c5 * F * r2;
-      extra[0] = k5 * s[n][0];
-      extra[1] = k5 * s[n][1];
-      extra[2] = k5 * s[n][2];
-    }
-#pragma unroll
-    for (int L = 1; L <= LM; ++L) {
-      const float F2 = L <= Lm ? 2.0f * Fp[nR + (L - 1) * nA + n] : 0.0f;  // no adjoint above the order
-#pragma unroll
-      for (int a = L * L - 1; a < (L + 1) * (L + 1) - 1; ++a) {
-        float v = F2 * c_c3[a] * s[n][a];
-        if (a < 8) v += extra[a];
-        s[n][a] = v;
-      }
-    }
-  }
-
-  // ---- angular partial forces dE_i/dr_ij (the edges of the moments loop)
-  rn = erow[lr < na ? lr : 0];
-  ahead = erow[lr + 8 * P < na ? lr + 8 * P : 0];
-  for (int e = lr; e < na; e += P) {
-    const float4 r = rn;
-    const int en = e + P;
-    if (en < na) {
-      if ((((en - lr) / P) & 7) == 0) {
-        rn = ahead;
-        if (en + 8 * P < na) ahead = erow[en + 8 * P];
-      } else {
-        rn = erow[en];
-      }
-    }
-    const int j = __float_as_int(r.w);
-    const float d2 = r.x * r.x + r.y * r.y + r.z * r.z;
-    const float dinv = __builtin_amdgcn_rsqf(d2);  // hardware 1/sqrt (1 ulp); edges have d > 0
-    const float d = d2 * dinv;
-    const float ux = r.x * dinv, uy = r.y * dinv, uz = r.z * dinv;
-    float rc;
-    int tj = 0;
-    if (C::one) {
-      rc = rcAf[0];
-    } else {
-      tj = safe_type(type[j], T);
-      rc = pcut[2 * kPairs + ti * T + tj];
-    }
-    const float rcinv = C::one ? 1.0f / rc : pcut[3 * kPairs + ti * T + tj];
-    float fc, fcp;
-    cutoff_fc_fcp(rc, rcinv, d, fc, fcp);
-    float f[KA], fp[KA];
-    cheb_d<KA>(kA, rcinv, d, fc, fcp, f, fp);
-    const float* c = C::cl ? ctab + T * T * NR * KR + (ti * T + tj) * NA * KA
-                           : m.cA + (size_t)(ti * T + tj) * nA * kA;
-    float g[NA], gp[NA];
-#pragma unroll
-    for (int n = 0; n < NA; ++n) {
-      g[n] = 0.0f;
-      gp[n] = 0.0f;
-      if (n < nA) {
-#pragma unroll
-        for (int k = 0; k < KA; ++k)
-          if (k < kA) {
-            g[n] += c[n * kA + k] * f[k];
-            gp[n] += c[n * kA + k] * fp[k];
-          }
-      }
-    }
-    // contract the adjoint with the basis: A = sum_n a g_n, B = sum_n a g'_n,
-    // then Pr = sum B Y and G = sum A dY/du (Y = Z(uz) Re/Im (ux+i uy)^m)
-    float zp[LM + 1];
-    zp[0] = 1.0f;
-#pragma unroll
-    for (int k = 1; k <= LM; ++k) zp[k] = zp[k - 1] * uz;
-    float pr[LM + 1], pim[LM + 1];
-    pr[0] = 1.0f;
-    pim[0] = 0.0f;
-#pragma unroll
-    for (int k = 1; k <= LM; ++k) {
-      pr[k] = pr[k - 1] * ux - pim[k - 1] * uy;
-      pim[k] = pr[k - 1] * uy + pim[k - 1] * ux;
-    }
-    float Pr = 0.0f, Gx = 0.0f, Gy = 0.0f, Gz = 0.0f;
-#pragma unroll
-    for (int L = 1; L <= LM; ++L) {
-#pragma unroll
-      for (int mm = 0; mm <= L; ++mm) {
-        float Z = 0.0f, dZ = 0.0f;
-#pragma unroll
-        for (int k = (L - mm) & 1; k <= L - mm; k += 2) {
-          Z += c_zc[L][mm][k] * zp[k];
-          if (k > 0) dZ += c_zc[L][mm][k] * (float)k * zp[k - 1];
-        }
-        const int b = L * L - 1;
-        if (mm == 0) {
-          float A = 0.0f, B = 0.0f;
-#pragma unroll
-          for (int n = 0; n < NA; ++n) {
-            A += s[n][b] * g[n];
-            B += s[n][b] * gp[n];
-          }
-          Pr += B * Z;
-          Gz += A * dZ;
-        } else {
-          const int ir = b + 2 * mm - 1, ii = b + 2 * mm;
-          float Ar = 0.0f, Ai = 0.0f, Br = 0.0f, Bi = 0.0f;
-#pragma unroll
-          for (int n = 0; n < NA; ++n) {
-            Ar += s[n][ir] * g[n];
-            Ai += s[n][ii] * g[n];
-            Br += s[n][ir] * gp[n];
-            Bi += s[n][ii] * gp[n];
-          }
-          Pr += Z * (Br * pr[mm] + Bi * pim[mm]);
-          const float mz = (float)mm * Z;
-          Gx += mz * (Ar * pr[mm - 1] + Ai * pim[mm - 1]);
-          Gy += mz * (Ai * pr[mm - 1] - Ar * pim[mm - 1]);
-          Gz += dZ * (Ar * pr[mm] + Ai * pim[mm]);
-        }
-      }
-    }
-    const float gu = Gx * ux + Gy * uy + Gz * uz;
-    const float4 fo = make_float4(Pr * ux + (Gx - gu * ux) * dinv, Pr * uy + (Gy - gu * uy) * dinv,
-                                  Pr * uz + (Gz - gu * uz) * dinv, 0.0f);
-    frow[e] = fo;
   }
 }
 
@@ -2005,172 +885,6 @@ hipError_t launch_filter(const DevBox& b, const DevModel& m, int c1, int c2, Dev
   } else if (close) {
     k_close_request<<<1, 1, 0, s>>>(w.flags);
   }
-  return hipGetLastError();
-}
-
-template <class C>
-static void run_descriptor(const DevBox& b, const DevModel& m, int N, int c1, int c2, const int* type, double* pe,
-                           bool acc, DevWork& w, hipStream_t s, hipEvent_t e0, hipEvent_t e1, int lanes = 1)
-{
-  if constexpr (C::ann == kAnnValu) {
-    if (lanes == 4 && !w.split) {
-      constexpr int per = kDescBlock / 4;
-      const int nb = (c2 - c1 + per - 1) / per;
-      auto k = k_descriptor<C, false, 4>;
-      if (e0 || e1)
-        hipExtLaunchKernelGGL(k, dim3(xcd_grid(nb)), dim3(kDescBlock), 0, s, e0, e1, 0, b, m, N, c1, c2, nb, type,
-                              pe, w.edge, w.vsa, w.eq, acc ? 1 : 0, w);
-      else
-        k<<<xcd_grid(nb), kDescBlock, 0, s>>>(b, m, N, c1, c2, nb, type, pe, w.edge, w.vsa, w.eq, acc ? 1 : 0, w);
-      return;
-    }
-  }
-  const int nb = (c2 - c1 + kDescBlock - 1) / kDescBlock;
-  auto k = w.split ? k_descriptor<C, true> : k_descriptor<C, false>;
-  if (e0 || e1)
-    hipExtLaunchKernelGGL(k, dim3(xcd_grid(nb)), dim3(kDescBlock), 0, s, e0, e1, 0, b, m, N, c1, c2, nb, type, pe,
-                          w.edge, w.vsa, w.eq, acc ? 1 : 0, w);
-  else
-    k<<<xcd_grid(nb), kDescBlock, 0, s>>>(b, m, N, c1, c2, nb, type, pe, w.edge, w.vsa, w.eq, acc ? 1 : 0, w);
-}
-
-// single-type exact configuration with the ANN mode picked at run time:
-// matrix cores for H <= 64 (FP32 or BF16 operands), vector ALUs otherwise
-template <int NR, int KR, int NA, int KA, bool Q2, bool Q1>
-static void run_single(const DevBox& b, const DevModel& m, int N, int c1, int c2, const int* type, double* pe, bool acc, int ann,
-                       DevWork& w, hipStream_t s, hipEvent_t e0, hipEvent_t e1, int lanes)
-{
-  const int mode = (m.H <= 64 && !(lanes == 4 && !w.split)) ? ann : kAnnValu;
-  if constexpr (mfma_ann_fits<NR, KR, NA, KA, Q2, Q1, true>()) {
-    if (mode == kAnnMfma32) {
-      run_descriptor<Cfg<NR, KR, NA, KA, 4, Q2, Q1, true, true, kAnnMfma32>>(b, m, N, c1, c2, type, pe, acc, w, s, e0,
-                                                                            e1);
-      return;
-    }
-    if (mode == kAnnMfmaBf16) {
-      run_descriptor<Cfg<NR, KR, NA, KA, 4, Q2, Q1, true, true, kAnnMfmaBf16>>(b, m, N, c1, c2, type, pe, acc, w, s, e0,
-                                                                              e1);
-      return;
-    }
-    if constexpr (mfma_ann_fits<NR, KR, NA, KA, Q2, Q1, true, kAnnMfmaSplit>()) {
-      if (mode == kAnnMfmaSplit) {
-        run_descriptor<Cfg<NR, KR, NA, KA, 4, Q2, Q1, true, true, kAnnMfmaSplit>>(b, m, N, c1, c2, type, pe, acc, w, s,
-                                                                                  e0, e1);
-        return;
-      }
-    }
-  }
-  run_descriptor<Cfg<NR, KR, NA, KA, 4, Q2, Q1, true, true, kAnnValu>>(b, m, N, c1, c2, type, pe, acc, w, s, e0, e1,
-                                                                      lanes);
-}
-
-template <int NR, int KR, int NA, int KA, bool Q2, bool Q1>
-static void run_multi(const DevBox& b, const DevModel& m, int N, int c1, int c2, const int* type, double* pe, bool acc, int ann,
-                      DevWork& w, hipStream_t s, hipEvent_t e0, hipEvent_t e1, int lanes)
-{
-  const int mode = (m.H <= 64 && m.T <= kTypesMfma && !(lanes == 4 && !w.split)) ? ann : kAnnValu;
-  if constexpr (mfma_ann_fits<NR, KR, NA, KA, Q2, Q1, false>()) {
-    if (mode == kAnnMfma32) {
-      run_descriptor<Cfg<NR, KR, NA, KA, 4, Q2, Q1, false, true, kAnnMfma32, true>>(b, m, N, c1, c2, type, pe, acc, w,
-                                                                                   s, e0, e1);
-      return;
-    }
-    if (mode == kAnnMfmaBf16) {
-      run_descriptor<Cfg<NR, KR, NA, KA, 4, Q2, Q1, false, true, kAnnMfmaBf16, true>>(b, m, N, c1, c2, type, pe, acc,
-                                                                                     w, s, e0, e1);
-      return;
-    }
-    if constexpr (mfma_ann_fits<NR, KR, NA, KA, Q2, Q1, false, kAnnMfmaSplit>()) {
-      if (mode == kAnnMfmaSplit) {
-        run_descriptor<Cfg<NR, KR, NA, KA, 4, Q2, Q1, false, true, kAnnMfmaSplit, true>>(b, m, N, c1, c2, type, pe,
-                                                                                         acc, w, s, e0, e1);
-        return;
-      }
-    }
-  }
-  if (m.T <= kTypesLds)
-    run_descriptor<Cfg<NR, KR, NA, KA, 4, Q2, Q1, false, true, kAnnValu, true>>(b, m, N, c1, c2, type, pe, acc, w, s,
-                                                                               e0, e1, lanes);
-  else
-    run_descriptor<Cfg<NR, KR, NA, KA, 4, Q2, Q1, false, true>>(b, m, N, c1, c2, type, pe, acc, w, s, e0, e1, lanes);
-}
-
-namespace {
-bool model_is(const DevModel& m, int nr, int kr, int na, int ka, int L, bool a, bool b, bool one)
-{
-  return m.nR == nr && m.kR == kr && m.nA == na && m.kA == ka && m.L == L && (m.has222 != 0) == a &&
-         (m.has1111 != 0) == b && (m.T == 1) == one;
-}
-
-// sizes of the exactly instantiated configurations (nR, kR, nA, kA, q222,
-// q1111, single type); the bounded sizes below come after them
-struct ExactCfg {
-  int nr, kr, na, ka;
-  bool q2, q1, one;
-};
-constexpr ExactCfg kExact[] = {
-    {5, 9, 5, 9, true, true, true},     {7, 9, 5, 9, true, false, true},   {13, 17, 9, 13, true, true, true},
-    {7, 11, 7, 11, true, true, false},  {5, 9, 5, 9, true, false, false},  {9, 9, 7, 9, false, false, false},
-    {7, 9, 5, 9, true, true, true},     {7, 9, 5, 9, true, true, false},   {9, 13, 7, 13, true, true, true},
-    {9, 13, 7, 13, true, true, false}};
-constexpr int kBuckets[][4] = {{7, 9, 5, 9}, {9, 13, 7, 13}};
-}  // namespace
-
-bool descriptor_bucket(const DevModel& m, int dims[4])
-{
-  for (const ExactCfg& c : kExact)
-    if (model_is(m, c.nr, c.kr, c.na, c.ka, 4, c.q2, c.q1, c.one)) return false;
-  if (m.L > 4) return false;
-  for (const auto& b : kBuckets)
-    if (m.nR <= b[0] && m.kR <= b[1] && m.nA <= b[2] && m.kA <= b[3]) {
-      for (int k = 0; k < 4; ++k) dims[k] = b[k];
-      return true;
-    }
-  return false;
-}
-
-hipError_t launch_descriptor(const DevBox& b, const DevModel& m, int N, int c1, int c2, const int* type, double* pe,
-                             bool acc, int ann, DevWork& w, hipStream_t s, hipEvent_t e0, hipEvent_t e1, int lanes)
-{
-  if (lanes != 1 && lanes != 4) return hipErrorInvalidValue;
-  if (c2 <= c1) return hipSuccess;
-  const bool one = m.T == 1;
-  const bool q2 = m.has222 != 0, q1 = m.has1111 != 0;
-  auto is = [&](int nr, int kr, int na, int ka, int L, bool a, bool b, bool o) {
-    return model_is(m, nr, kr, na, ka, L, a, b, o);
-  };
-  // exact instantiations: the configurations in use, and the bounded sizes
-  // that other models are padded to (descriptor_bucket); generic otherwise
-  if (is(5, 9, 5, 9, 4, true, true, true))
-    run_single<5, 9, 5, 9, true, true>(b, m, N, c1, c2, type, pe, acc, ann, w, s, e0, e1, lanes);
-  else if (is(7, 9, 5, 9, 4, true, false, true))
-    run_single<7, 9, 5, 9, true, false>(b, m, N, c1, c2, type, pe, acc, ann, w, s, e0, e1, lanes);
-  else if (is(13, 17, 9, 13, 4, true, true, true))
-    run_descriptor<Cfg<13, 17, 9, 13, 4, true, true, true, true>>(b, m, N, c1, c2, type, pe, acc, w, s, e0, e1, lanes);
-  else if (is(7, 11, 7, 11, 4, true, true, false))
-    run_multi<7, 11, 7, 11, true, true>(b, m, N, c1, c2, type, pe, acc, ann, w, s, e0, e1, lanes);
-  else if (is(5, 9, 5, 9, 4, true, false, false))
-    run_multi<5, 9, 5, 9, true, false>(b, m, N, c1, c2, type, pe, acc, ann, w, s, e0, e1, lanes);
-  else if (is(9, 9, 7, 9, 4, false, false, false))
-    run_multi<9, 9, 7, 9, false, false>(b, m, N, c1, c2, type, pe, acc, ann, w, s, e0, e1, lanes);
-  else if (is(7, 9, 5, 9, 4, true, true, true))
-    run_single<7, 9, 5, 9, true, true>(b, m, N, c1, c2, type, pe, acc, ann, w, s, e0, e1, lanes);
-  else if (is(7, 9, 5, 9, 4, true, true, false))
-    run_multi<7, 9, 5, 9, true, true>(b, m, N, c1, c2, type, pe, acc, ann, w, s, e0, e1, lanes);
-  else if (is(9, 13, 7, 13, 4, true, true, true))
-    run_single<9, 13, 7, 13, true, true>(b, m, N, c1, c2, type, pe, acc, ann, w, s, e0, e1, lanes);
-  else if (is(9, 13, 7, 13, 4, true, true, false))
-    run_multi<9, 13, 7, 13, true, true>(b, m, N, c1, c2, type, pe, acc, ann, w, s, e0, e1, lanes);
-  else if (m.L <= kPadL && m.nR <= kMaxNR && m.kR <= kMaxK && m.nA <= kMaxNA && m.kA <= kMaxK)
-    run_descriptor<Cfg<kMaxNR, kMaxK, kMaxNA, kMaxK, kPadL, true, true, false, false>>(b, m, N, c1, c2, type, pe, acc,
-                                                                                      w, s, e0, e1, lanes);
-  else if (m.L <= kMaxL && m.nR <= kMaxNR && m.kR <= kMaxK && m.nA <= kMaxNA && m.kA <= kMaxK)
-    // 3-body orders 5..8 (80 angular moments per radial function): the
-    // generic instance at order 8, its per-atom arrays partly in scratch
-    run_descriptor<Cfg<kMaxNR, kMaxK, kMaxNA, kMaxK, kMaxL, true, true, false, false>>(b, m, N, c1, c2, type, pe, acc,
-                                                                                      w, s, e0, e1, lanes);
-  else
-    return hipErrorInvalidValue;
   return hipGetLastError();
 }
 

@@ -168,8 +168,6 @@ enum : int {
   kNumFlags = 16,
 };
 
-void upload_angular_constants(const AngularConstants& a);
-
 // Neighbour build (neighbor.hip).  launch_pack packs (x, y, z, type) for
 // the step, validates types and, unless `forced`, sets flags[kFlagRebuild]
 // when an atom moved more than skin/2 (and, with a request map, marks the

@@ -14,7 +14,6 @@
 #include <cmath>
 #include <fstream>
 #include <iterator>
-#include <numeric>
 #include <sstream>
 #include <stdexcept>
 
@@ -232,57 +231,6 @@ NepModel::Image NepModel::device_image() const
   for (int d = 0; d < D; ++d) v[im.off_qs + d] = (float)p[num_para_ann + num_para_desc + d];
   for (size_t i = 0; i < zbl_para.size(); ++i) v[im.off_zbl + i] = (float)zbl_para[i];
   return im;
-}
-
-AngularConstants derive_angular_constants()
-{
-  AngularConstants a{};
-  const double pi = 3.14159265358979323846;
-  for (int L = 1; L <= kMaxL; ++L) {
-    // 2^L P_L(z) = sum_k (-1)^k C(L,k) C(2L-2k,L) z^(L-2k)
-    long long base[kMaxL + 1] = {};
-    auto binom = [](int n, int k) {
-      long long r = 1;
-      for (int i = 1; i <= k; ++i) r = r * (n - k + i) / i;
-      return r;
-    };
-    for (int k = 0; 2 * k <= L; ++k) {
-      long long val = binom(L, k) * binom(2 * L - 2 * k, L);
-      base[L - 2 * k] = (k % 2) ? -val : val;
-    }
-    for (int m = 0; m <= L; ++m) {
-      long long d[kMaxL + 1] = {};
-      for (int p = m; p <= L; ++p) {
-        long long f = 1;
-        for (int s = 0; s < m; ++s) f *= (p - s);
-        d[p - m] = base[p] * f;
-      }
-      long long g = 0;
-      for (int p = 0; p <= L - m; ++p)
-        if (d[p]) g = std::gcd(g, d[p] < 0 ? -d[p] : d[p]);
-      for (int p = 0; p <= L - m; ++p) a.zc[L][m][p] = (float)(d[p] / g);
-      const double alpha = (double)g / std::ldexp(1.0, L);
-      double fr = 1.0;
-      for (int s = L - m + 1; s <= L + m; ++s) fr /= (double)s;
-      const double w = (2.0 * L + 1.0) / (4.0 * pi) * fr * alpha * alpha;
-      const int b = L * L - 1;
-      if (m == 0) {
-        a.c3[b] = (float)w;
-      } else {
-        a.c3[b + 2 * m - 1] = (float)(2.0 * w);
-        a.c3[b + 2 * m] = (float)(2.0 * w);
-      }
-    }
-  }
-  // q_222: Wigner-3j (2 2 2; m1 m2 m3) coupling of three l=2 moments, weights
-  // k*sqrt(14)/(448 pi^1.5) for s3^3, s3(s4^2+s5^2), s3(s6^2+s7^2),
-  // s6(s5^2-s4^2), s4 s5 s7.
-  const double u4 = std::sqrt(14.0) / (448.0 * std::pow(pi, 1.5));
-  const double k4[5] = {-5.0, -90.0, 45.0, 270.0, -540.0};
-  for (int i = 0; i < 5; ++i) a.c4[i] = (float)(k4[i] * u4);
-  // q_1111: sum over intermediate L of (1 1 L)(L 1 1) couplings = 21/(80 pi^2) |s_1|^4
-  a.c5 = (float)(21.0 / (80.0 * pi * pi));
-  return a;
 }
 
 }  // namespace dmgx
