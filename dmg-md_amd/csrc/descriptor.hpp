@@ -16,9 +16,6 @@ constexpr int kDescBlock = 256;
 // ANN modes of the descriptor kernel
 enum : int { kAnnValu = 0, kAnnMfma32 = 1, kAnnMfmaBf16 = 2, kAnnMfmaSplit = 3 };
 
-// multi-type models with at most this many types keep their coefficient
-// blocks in LDS
-constexpr int kTypesLds = 4;
 // multi-type models with at most this many types run their ANN on the
 // matrix cores: every type's weights staged in LDS, one GEMM pass per type
 // present in the wavefront, each atom taking the pass of its own type
@@ -132,15 +129,6 @@ __device__ __forceinline__ void stage_ann_weights(const DevModel& m, int D, floa
   }
 }
 
-
-// orders this wavefront's LDS writes before its later LDS reads (each
-// wavefront works in its own LDS region, so no workgroup barrier is needed)
-__device__ __forceinline__ void wave_lds_sync()
-{
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // MT: multi-type (ti is the lane's type, T the number of types <=
 // kTypesMfma, ws holds the types' weight blocks one after another): per
@@ -481,29 +469,6 @@ constexpr bool mfma_ann_fits()
          (ONE ? 64 * 1024 : kDescLdsMax);
 }
 
-// sum of v over the P consecutive lanes of a lane group (every lane gets the
-// same bits: each stage adds two partners that hold each other's value), with
-// the lane permutations of the DPP adds (one instruction per stage)
-template <int CTRL>
-__device__ __forceinline__ float dpp_move(float v)
-{
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
-}
-template <int P>
-__device__ __forceinline__ float group_sum(float v)
-{
-  static_assert(P == 1 || P == 4 || P == 16, "lane groups of 4 or 16");
-  if (P >= 4) {
-    v += dpp_move<0xB1>(v);  // quad_perm [1,0,3,2]
-    v += dpp_move<0x4E>(v);  // quad_perm [2,3,0,1]
-  }
-  if (P >= 16) {
-    v += dpp_move<0x141>(v);  // row_half_mirror
-    v += dpp_move<0x140>(v);  // row_mirror
-  }
-  return v;
-}
-
 // What bounds it: vector instruction issue, most of it in the two loops over
 // the angular edges (about 240 and 500 instructions per edge and wavefront at
 // n_max 4, basis 8, order 4).  The angular coefficients are literals, the
@@ -530,13 +495,14 @@ template <class C, bool CAND, int P = 1>
 __global__ __launch_bounds__(kDescBlock, C::waves) void k_descriptor(DevBox b, DevModel m, int N, int c1, int c2, int nblocks,
                                                        const int* __restrict__ type, double* __restrict__ pe,
                                                        float4* __restrict__ edge, int* __restrict__ vsa,
-                                                       int* __restrict__ eq, int accumulate, DevWork w)
+                                                       short* __restrict__ eq, int accumulate, DevWork w)
 {
   constexpr int NR = C::nr, KR = C::kr, NA = C::na, KA = C::ka, LM = C::lm, NABC = C::nabc, DMAX = C::dim;
   static_assert(P == 1 || ((P == 4 || P == 16) && !CAND && C::ann == kAnnValu), "lane groups: the filter's rows, vector ANN");
   const int lr = P == 1 ? 0 : (int)(threadIdx.x & (P - 1));  // lane within the atom's group
-  const int i0 = c1 + xcd_tile(nblocks) * (int)(blockDim.x / P) + (int)(threadIdx.x / P);
-  const bool active = i0 < c2;
+  // blocks start at a row tile's first centre, so a wavefront reads whole tiles
+  const int i0 = (c1 & ~(kTile - 1)) + xcd_tile(nblocks) * (int)(blockDim.x / P) + (int)(threadIdx.x / P);
+  const bool active = i0 >= c1 && i0 < c2;
   // the matrix-core ANN needs every lane of the wavefront: lanes past the
   // range carry an empty row of a valid atom and write nothing
   const int i = active ? i0 : c1;
@@ -604,11 +570,13 @@ __global__ __launch_bounds__(kDescBlock, C::waves) void k_descriptor(DevBox b, D
     na = w.na[i];
   }
   // with candidate rows this kernel writes the angular edges it reads back
-  const float4* erow = edge + (size_t)i * w.MR;
-  float4* __restrict__ frow = w.f12 + (size_t)i * w.MA;
+  const float4* erow = edge + row_begin(i, w.MR);
+  float3* __restrict__ frow = w.f12 + row_begin(i, w.MA);
   float q[DMAX];
 #pragma unroll
   for (int d = 0; d < DMAX; ++d) q[d] = 0.0f;
+
+  auto type_of = [&](const float4& r) { return C::one ? 0 : edge_type(w, type, __float_as_int(r.w), T); };
 
   // ---- radial descriptor: q_n = sum_j sum_k c[ti,tj,n,k] f_k(r_ij),
   // f_k = (T_k(x) + 1) fc / 2.  The scaled polynomials t_k = (fc / 2) T_k are
@@ -662,21 +630,21 @@ __global__ __launch_bounds__(kDescBlock, C::waves) void k_descriptor(DevBox b, D
     // radial-only edges, stored from the row's end downward; kAhead records
     // in flight (the work per edge is short).  The angular edges' radial terms
     // are summed in the loop over the angular moments.
-    constexpr int kAhead = 4;
+    constexpr int kAhead = 12;
     const int nro = nr - na;
     float4 ring[kAhead];
 #pragma unroll
     for (int u = 0; u < kAhead; ++u)
-      ring[u] = u * P + lr < nro ? erow[w.MR - 1 - (u * P + lr)] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      ring[u] = u * P + lr < nro ? erow[(size_t)(w.MR - 1 - (u * P + lr)) * kTile] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     for (int e0 = lr; e0 < nro; e0 += kAhead * P)
 #pragma unroll
       for (int u = 0; u < kAhead; ++u) {
         const int e = e0 + u * P;
         if (e >= nro) break;
         const float4 r = ring[u];
-        if (e + kAhead * P < nro) ring[u] = erow[w.MR - 1 - (e + kAhead * P)];
+        if (e + kAhead * P < nro) ring[u] = erow[(size_t)(w.MR - 1 - (e + kAhead * P)) * kTile];
         const float d2 = r.x * r.x + r.y * r.y + r.z * r.z;
-        radial_edge(d2 * __builtin_amdgcn_rsqf(d2), C::one ? 0 : safe_type(type[__float_as_int(r.w)], T));
+        radial_edge(d2 * __builtin_amdgcn_rsqf(d2), type_of(r));
       }
   } else {
     // candidate rows: the FP64 minimum-image distance of every candidate
@@ -688,7 +656,8 @@ __global__ __launch_bounds__(kDescBlock, C::waves) void k_descriptor(DevBox b, D
     const int nrc = active ? w.nrc[i] : 0, nac = active ? w.nac[i] : 0;
     const size_t vrow = (size_t)i * w.MV, arow = (size_t)i * w.MA;
     const int* __restrict__ crow = w.cl + vrow;
-    float4* ew = edge + (size_t)i * w.MR;
+    float4* ew = edge + row_begin(i, w.MR);
+    short* qw = eq + row_begin(i, w.MA);
     const double4 pi = w.xq[i];
     double cr1 = 0.0, ca1 = 0.0;
     if (C::one) {
@@ -726,13 +695,14 @@ __global__ __launch_bounds__(kDescBlock, C::waves) void k_descriptor(DevBox b, D
         }
         const bool in_r = d2 < cr;
         const int jo = w.map.owner ? w.map.owner[j] : j;
-        const float4 r = make_float4((float)x, (float)y, (float)z, __int_as_float(jo));
+        const float4 r =
+            make_float4((float)x, (float)y, (float)z, __int_as_float(C::one ? jo : edge_word(w.typed, jo, tj)));
         if (e < nac) {
           const bool in_a = in_r && d2 < ca;
           vsa[arow + e] = in_a ? na : -1;
           if (in_a) {
-            ew[na] = r;
-            eq[arow + na] = w.cq[arow + e];
+            ew[(size_t)na * kTile] = r;
+            qw[(size_t)na * kTile] = (short)w.cq[arow + e];
             ++na;
           }
         }
@@ -755,26 +725,29 @@ __global__ __launch_bounds__(kDescBlock, C::waves) void k_descriptor(DevBox b, D
 #pragma unroll
     for (int a = 0; a < NABC; ++a) s[n][a] = 0.0f;
   float zpe = 0.0f;
-  // each lane takes every P-th edge; the next record is loaded before the
-  // current one is used, and the first record of the next 128-byte line
-  // (eight of the lane's records) a line ahead
-  float4 rn = erow[lr < na ? lr : 0];
-  float4 ahead = erow[lr + 8 * P < na ? lr + 8 * P : 0];
-  for (int e = lr; e < na; e += P) {
-    const float4 r = rn;
-    const int en = e + P;
-    if (en < na) {
-      if ((((en - lr) / P) & 7) == 0) {
-        rn = ahead;
-        if (en + 8 * P < na) ahead = erow[en + 8 * P];
-      } else {
-        rn = erow[en];
-      }
-    }
+  // each lane takes every P-th edge with kRing records in flight: a record
+  // comes from beyond L1, and an edge's arithmetic covers a fraction of that
+  // (one ahead: 171 us on 256,000 Cu atoms, four: 165)
+  constexpr int kRing = 4;
+  auto edge_at = [&](int e) { return erow[(size_t)e * kTile]; };
+  float4 ring[kRing];
+  auto fill_ring = [&]() {
+#pragma unroll
+    for (int u = 0; u < kRing; ++u)
+      ring[u] = lr + u * P < na ? edge_at(lr + u * P) : make_float4(1.0f, 0.0f, 0.0f, 0.0f);
+  };
+  fill_ring();
+  for (int e0 = lr; e0 < na; e0 += kRing * P)
+#pragma unroll
+  for (int u = 0; u < kRing; ++u) {
+    const int e = e0 + u * P;
+    if (e >= na) break;
+    const float4 r = ring[u];
+    if (e + kRing * P < na) ring[u] = edge_at(e + kRing * P);
+    const int tj = type_of(r);
     const float d2 = r.x * r.x + r.y * r.y + r.z * r.z;
     const float dinv = __builtin_amdgcn_rsqf(d2);  // hardware 1/sqrt (1 ulp); edges have d > 0
     const float d = d2 * dinv;
-    const int tj = C::one ? 0 : safe_type(type[__float_as_int(r.w)], T);
     if (!CAND) radial_edge(d, tj);
     const float rc = C::one ? rcAf[0] : pcut[2 * kPairs + ti * T + tj];
     const float rcinv = C::one ? 1.0f / rc : pcut[3 * kPairs + ti * T + tj];
@@ -986,24 +959,19 @@ __global__ __launch_bounds__(kDescBlock, C::waves) void k_descriptor(DevBox b, D
   }
 
   // ---- angular partial forces dE_i/dr_ij (the edges of the moments loop)
-  rn = erow[lr < na ? lr : 0];
-  ahead = erow[lr + 8 * P < na ? lr + 8 * P : 0];
-  for (int e = lr; e < na; e += P) {
-    const float4 r = rn;
-    const int en = e + P;
-    if (en < na) {
-      if ((((en - lr) / P) & 7) == 0) {
-        rn = ahead;
-        if (en + 8 * P < na) ahead = erow[en + 8 * P];
-      } else {
-        rn = erow[en];
-      }
-    }
+  fill_ring();
+  for (int e0 = lr; e0 < na; e0 += kRing * P)
+#pragma unroll
+  for (int u = 0; u < kRing; ++u) {
+    const int e = e0 + u * P;
+    if (e >= na) break;
+    const float4 r = ring[u];
+    if (e + kRing * P < na) ring[u] = edge_at(e + kRing * P);
+    const int tj = type_of(r);
     const float d2 = r.x * r.x + r.y * r.y + r.z * r.z;
     const float dinv = __builtin_amdgcn_rsqf(d2);  // hardware 1/sqrt (1 ulp); edges have d > 0
     const float d = d2 * dinv;
     const float ux = r.x * dinv, uy = r.y * dinv, uz = r.z * dinv;
-    const int tj = C::one ? 0 : safe_type(type[__float_as_int(r.w)], T);
     const float rc = C::one ? rcAf[0] : pcut[2 * kPairs + ti * T + tj];
     const float rcinv = C::one ? 1.0f / rc : pcut[3 * kPairs + ti * T + tj];
     float fc, fcp;
@@ -1103,9 +1071,9 @@ __global__ __launch_bounds__(kDescBlock, C::waves) void k_descriptor(DevBox b, D
       if constexpr (M < LM) Gz += dR * pw.re[M] + dI * pw.im[M];
     });
     const float gu = Gx * ux + Gy * uy + Gz * uz;
-    const float4 fo = make_float4(Pr * ux + (Gx - gu * ux) * dinv, Pr * uy + (Gy - gu * uy) * dinv,
-                                  Pr * uz + (Gz - gu * uz) * dinv, 0.0f);
-    frow[e] = fo;
+    const float3 fo = make_float3(Pr * ux + (Gx - gu * ux) * dinv, Pr * uy + (Gy - gu * uy) * dinv,
+                                  Pr * uz + (Gz - gu * uz) * dinv);
+    frow[(size_t)e * kTile] = fo;
   }
 }
 
@@ -1126,7 +1094,7 @@ template <class C, bool CAND, int P>
 void launch_instance(const DescriptorCall& a)
 {
   constexpr int per = kDescBlock / P;
-  const int nb = (a.c2 - a.c1 + per - 1) / per;
+  const int nb = (a.c2 - (a.c1 & ~(kTile - 1)) + per - 1) / per;
   auto k = k_descriptor<C, CAND, P>;
   if (a.e0 || a.e1)
     hipExtLaunchKernelGGL(k, dim3(xcd_grid(nb)), dim3(kDescBlock), 0, a.s, a.e0, a.e1, 0, a.b, a.m, a.N, a.c1, a.c2, nb,

@@ -85,4 +85,10 @@ __device__ __forceinline__ bool cell_coords(const DevBox& b, double x, double y,
 // type index clamped into [0, T) (invalid caller types are flagged by the filter)
 __device__ __forceinline__ int safe_type(int t, int T) { return (t < 0 || t >= T) ? 0 : t; }
 
+// the neighbour's type from an edge record's word
+__device__ __forceinline__ int edge_type(const DevWork& w, const int* __restrict__ type, int v, int T)
+{
+  return w.typed ? v >> kEdgeSlotBits : safe_type(type[v], T);
+}
+
 }  // namespace dmgx

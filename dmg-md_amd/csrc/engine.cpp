@@ -371,7 +371,7 @@ int NepEngine::padded_rows(int mv, int layout) const
 // edge reverse, angular partial force and an angular bit; and with
 // candidate rows the candidate slot, its angular slot, its position and
 // reverse index
-constexpr double kRowEntryBytes = 4 + 4 + 16 + 4 + 16 + 4.0 / 32.0;
+constexpr double kRowEntryBytes = 4 + 2 + 16 + 2 + 12 + 4.0 / 32.0;
 constexpr double kSplitEntryBytes = 4 + 4 + 4 + 4;
 
 void NepEngine::allocate(int capacity, int mv, int centres)
@@ -391,16 +391,17 @@ void NepEngine::allocate(int capacity, int mv, int centres)
   dalloc(&w_.xs, cap, "cell-ordered positions");
   dalloc(&w_.x0, 3 * cap, "x0");
   dalloc(&w_.vn, rc, "vn");
+  const size_t tiles = row_entries(rc, mv);
   dalloc(&w_.vl, rows, "verlet rows");
   dalloc(&w_.vrev, rows, "verlet reverse");
   dalloc(&w_.nr, rc, "nr");
   dalloc(&w_.na, rc, "na");
-  dalloc(&w_.edge, rows, "edges");
-  dalloc(&w_.eq, rows, "edge reverse");
+  dalloc(&w_.edge, tiles, "edges");
+  dalloc(&w_.eq, tiles, "edge reverse");
   dalloc(&w_.amask, rc * (size_t)((mv + 31) / 32), "angular bits");
   dfree(&w_.vsa);  // candidate rows only
   dalloc(&w_.bR, rc * model_.num_types * (size_t)((model_.kR + 3) & ~3), "radial adjoint");
-  dalloc(&w_.f12, rows, "angular partials");
+  dalloc(&w_.f12, tiles, "angular partials");
   w_.cap = (int)cap;
   w_.rcap = (int)rc;
   w_.MV = mv;
@@ -538,6 +539,7 @@ NepEngine::Plan NepEngine::plan(const Box& box, int N, int n1, int n2, int nd1, 
              im.image != last_map_.image || im.gstart != last_map_.gstart;
   if (p.forced) scale_since_build_ = 1.0;  // this evaluation rebuilds from the current positions
   p.empty = false;
+  w_.typed = N <= 1 << kEdgeSlotBits;
   w_.map = im;
   if (w_.split) {
     // candidate rows are remade for every centre at a rebuild: no request map
@@ -614,7 +616,7 @@ void NepEngine::launch_key(std::vector<long long>& k) const
   const DevWork& w = w_;
   auto p = [&](const void* q) { k.push_back((long long)(uintptr_t)q); };
   for (long long v : {(long long)w.cap, (long long)w.rcap, (long long)w.MV, (long long)w.MR, (long long)w.MA,
-                      (long long)w.ncell_cap, (long long)w.split, (long long)w.map.n_owned, (long long)w.map.n_req})
+                      (long long)w.ncell_cap, (long long)w.split, (long long)w.typed, (long long)w.map.n_owned, (long long)w.map.n_req})
     k.push_back(v);
   for (const void* q : {(const void*)w.xq, (const void*)w.cell_of, (const void*)w.cell_rank,
                         (const void*)w.cell_count, (const void*)w.cell_start, (const void*)w.cell_atoms,
@@ -1052,7 +1054,7 @@ DevWork carve_work(char* base, int cap, int mv, long long ncell, int T, int kRp,
 {
   Carver c{base};
   DevWork w{};
-  const size_t n = (size_t)cap, rows = n * (size_t)mv;
+  const size_t n = (size_t)cap, rows = n * (size_t)mv, tiles = row_entries(n, mv);
   w.flags = c.take<int>(kNumFlags);
   w.cell_count = c.take<int>((size_t)ncell);
   w.cell_start = c.take<int>((size_t)ncell + 1);
@@ -1068,11 +1070,11 @@ DevWork carve_work(char* base, int cap, int mv, long long ncell, int T, int kRp,
   w.x0 = c.take<double>(3 * n);
   w.bR = c.take<float>(n * (size_t)T * (size_t)kRp);
   w.vl = c.take<int>(rows);
-  w.vrev = c.take<int>(rows);
-  w.eq = c.take<int>(rows);
+  w.vrev = c.take<short>(rows);
+  w.eq = c.take<short>(tiles);
   w.amask = c.take<unsigned>(n * (size_t)((mv + 31) / 32));
-  w.edge = c.take<float4>(rows);
-  w.f12 = c.take<float4>(rows);
+  w.edge = c.take<float4>(tiles);
+  w.f12 = c.take<float3>(tiles);
   if (split) {
     w.split = 1;
     w.cl = c.take<int>(rows);
@@ -1119,10 +1121,10 @@ void NepEngine::compute_in(void* ws, size_t ws_bytes, const Box& box, int N, int
   const bool split = tune_.split != 0;
   carve_work(nullptr, N, mv, ncell, model_.num_types, kRp, split, &need);
   if (need > ws_bytes) {
-    size_t one = 0, none = 0;
-    carve_work(nullptr, 1, mv, ncell, model_.num_types, kRp, split, &one);
+    size_t one = 0, none = 0;  // of a tile of slots, and of none
+    carve_work(nullptr, kTile, mv, ncell, model_.num_types, kRp, split, &one);
     carve_work(nullptr, 0, mv, ncell, model_.num_types, kRp, split, &none);
-    const size_t per_atom = std::max<size_t>(one - none, 1);
+    const size_t per_atom = std::max<size_t>((one - none) / kTile, 1);
     throw std::invalid_argument("the system needs " + std::to_string(need) + " bytes of workspace (" +
                                 std::to_string(N) + " slots, rows of " + std::to_string(mv) + ", " +
                                 std::to_string(ncell) + " cells); the fixed workspace holds " +
@@ -1131,6 +1133,7 @@ void NepEngine::compute_in(void* ws, size_t ws_bytes, const Box& box, int N, int
                                 " slots of this model in this box)");
   }
   DevWork w = carve_work(static_cast<char*>(ws), N, mv, ncell, model_.num_types, kRp, split, &need);
+  w.typed = N <= 1 << kEdgeSlotBits;
   // the workspace keeps the previous call's contents: clear the status words
   // and the cell counts (the cell scan expects them at zero) with a kernel
   check(launch_clear_ints(w.flags, kNumFlags, s), "clear status words");
@@ -1224,10 +1227,9 @@ void NepEngine::copy_verlet_rows(int c1, int c2, int max_nb, int* counts, int* r
 {
   if (!have_list_) throw std::runtime_error("no neighbour list yet");
   if (c1 < last_c1_ || c2 > last_c2_ || c2 < c1) throw std::invalid_argument("rows outside the centre range");
-  const int N = last_N_stats_;
   check(hipDeviceSynchronize(), "sync");
-  std::vector<int> vn(N), vl((size_t)w_.MV * N);
-  check(hipMemcpy(vn.data(), w_.vn, N * sizeof(int), hipMemcpyDeviceToHost), "copy");
+  std::vector<int> vn(c2), vl((size_t)w_.MV * c2);
+  check(hipMemcpy(vn.data(), w_.vn, c2 * sizeof(int), hipMemcpyDeviceToHost), "copy");
   check(hipMemcpy(vl.data(), w_.vl, vl.size() * sizeof(int), hipMemcpyDeviceToHost), "copy");
   for (int i = c1; i < c2; ++i) {
     const int n = std::min(vn[i], w_.MV);
@@ -1241,17 +1243,16 @@ void NepEngine::copy_pair_rows(int which, int c1, int c2, int max_nb, int* count
 {
   if (!have_list_) throw std::runtime_error("no neighbour list yet");
   if (c1 < last_c1_ || c2 > last_c2_ || c2 < c1) throw std::invalid_argument("rows outside the centre range");
-  const int N = last_N_stats_;
   // candidate rows keep the step's angular rows (written by the descriptor)
   // but no radial rows: for those the filter pass runs once on the last
   // evaluation's positions
   if (w_.split && which == 0)
     check(launch_filter(last_box_, dm_, last_c1_, last_c2_, w_, nullptr, tune_.filter_lanes, false), "filter");
   check(hipDeviceSynchronize(), "sync");
-  std::vector<int> nr(N), na(N);
-  std::vector<float4> e((size_t)w_.MR * N);
-  check(hipMemcpy(nr.data(), w_.nr, N * sizeof(int), hipMemcpyDeviceToHost), "copy");
-  check(hipMemcpy(na.data(), w_.na, N * sizeof(int), hipMemcpyDeviceToHost), "copy");
+  std::vector<int> nr(c2), na(c2);
+  std::vector<float4> e(row_entries(c2, w_.MR));
+  check(hipMemcpy(nr.data(), w_.nr, c2 * sizeof(int), hipMemcpyDeviceToHost), "copy");
+  check(hipMemcpy(na.data(), w_.na, c2 * sizeof(int), hipMemcpyDeviceToHost), "copy");
   check(hipMemcpy(e.data(), w_.edge, e.size() * sizeof(float4), hipMemcpyDeviceToHost), "copy");
   for (int i = c1; i < c2; ++i) {
     const int n = which == 0 ? nr[i] : na[i];
@@ -1260,10 +1261,10 @@ void NepEngine::copy_pair_rows(int which, int c1, int c2, int max_nb, int* count
     std::vector<int> r(n);
     for (int k = 0; k < n; ++k) {
       const int slot = k < na[i] ? k : w_.MR - 1 - (k - na[i]);
-      float w = e[(size_t)i * w_.MR + slot].w;
+      float w = e[row_begin(i, w_.MR) + (size_t)slot * kTile].w;
       int j;
       std::memcpy(&j, &w, sizeof(int));
-      r[k] = j;
+      r[k] = model_.num_types > 1 ? edge_slot(w_.typed, j) : j;
     }
     std::sort(r.begin(), r.end());
     std::copy(r.begin(), r.end(), rows + (size_t)(i - c1) * max_nb);

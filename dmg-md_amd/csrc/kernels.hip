@@ -43,18 +43,14 @@ namespace dmgx {
 #define DMGX_FILTER_LANES 16
 #endif
 #ifndef DMGX_FILTER_BATCH
-#define DMGX_FILTER_BATCH 7
+#define DMGX_FILTER_BATCH 5
 #endif
 #ifndef DMGX_GATHER_LANES
 #define DMGX_GATHER_LANES 8
 #endif
-#ifndef DMGX_GATHER_BATCH
-#define DMGX_GATHER_BATCH 2
-#endif
 constexpr int kFilterLanes = DMGX_FILTER_LANES;
 constexpr int kFilterBatch = DMGX_FILTER_BATCH;
 constexpr int kGatherLanes = DMGX_GATHER_LANES;
-constexpr int kGatherBatch = DMGX_GATHER_BATCH;  // radial edges per lane per batch (kR <= 9)
 
 // CAND: the rebuild-time split of the rows into candidate rows instead (the
 // same pass with every cutoff widened by the skin, writing slot indices
@@ -91,7 +87,8 @@ __global__ __launch_bounds__(kBlock) void k_filter(DevBox b, DevModel m, int c1,
     w.flags[kFlagRebuildCount] += 1;
   }
   const int g = threadIdx.x / G, lg = threadIdx.x % G, gw = g % (64 / G);
-  const int i = c1 + xcd_tile(nblocks) * PER + g;
+  const int first = c1 + xcd_tile(nblocks) * PER;  // the workgroup's centres: PER consecutive ones
+  const int i = first + g;
   const bool active = i < c2;
   double4 pi = make_double4(0, 0, 0, 0);
   int ti = 0, nv = 0;
@@ -100,8 +97,23 @@ __global__ __launch_bounds__(kBlock) void k_filter(DevBox b, DevModel m, int c1,
     ti = ONE ? 0 : safe_type((int)__double_as_longlong(pi.w), T);
     nv = min(w.vn[i], w.MV);
   }
-  const size_t vrow = (size_t)i * w.MV, erow = (size_t)i * w.MR, arow = (size_t)i * w.MA;
+  const size_t vrow = (size_t)i * w.MV;
   const unsigned below = (1u << lg) - 1u;
+  // The kept edges of a pass of G * RB entries are compacted in LDS (angular
+  // ones from the front of a centre's stage, radial-only ones from its end) and
+  // stored to the interleaved rows slot by slot: consecutive threads store one
+  // slot of the workgroup's consecutive centres, 16 * PER contiguous bytes.
+  // (Stored directly, each record is a line access of its own: 154 us against
+  // 115 on 256,000 Cu atoms; row-major rows, with shorter loads in the
+  // descriptor's way, 122.  One lane per centre, without ballots, reads the
+  // neighbours' positions from 64 lines at a time: 204 us.)  The odd record
+  // count keeps the store's reads free of bank conflicts.
+  constexpr int kStage = G * RB;
+  __shared__ float4 stage[CAND ? 1 : PER * (kStage + 1)];
+  __shared__ short stage_q[CAND ? 1 : PER * (kStage + 2)];
+  __shared__ int4 counts[CAND ? 1 : PER];  // angular / radial-only edges before the pass, and in it
+  float4* const st = stage + g * (kStage + 1);
+  short* const sq = stage_q + g * (kStage + 2);
   int na = 0, nro = 0;
   // the row's angular bits, assembled a 32-bit word at a time by the
   // group's first lane (a chunk of G consecutive entries never straddles
@@ -109,7 +121,7 @@ __global__ __launch_bounds__(kBlock) void k_filter(DevBox b, DevModel m, int c1,
   unsigned* const mrow = CAND ? nullptr : w.amask + (size_t)i * ((w.MV + 31) >> 5);
   unsigned mword = 0u;
   int mcur = 0;
-  for (int p0 = 0; __any(p0 < nv); p0 += G * RB) {
+  for (int p0 = 0; CAND ? __any(p0 < nv) : __syncthreads_or(p0 < nv); p0 += G * RB) {
     int jj[RB], qq[RB], jo[RB];
     double4 pj[RB];
 #pragma unroll
@@ -129,6 +141,7 @@ __global__ __launch_bounds__(kBlock) void k_filter(DevBox b, DevModel m, int c1,
       pj[r] = jj[r] >= 0 ? w.xq[jj[r]] : make_double4(0, 0, 0, 0);
       jo[r] = (MAP && jj[r] >= 0) ? w.map.owner[jj[r]] : jj[r];
     }
+    int pa = 0, pr = 0;  // angular and radial-only edges of this pass
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
       const int p = p0 + r * G + lg;
@@ -139,33 +152,30 @@ __global__ __launch_bounds__(kBlock) void k_filter(DevBox b, DevModel m, int c1,
         mic(b, x, y, z);
         const double d2 = dist2(x, y, z);
         double cr = rr2, ca = ra2;
+        int tj = 0;
         if (!ONE) {
-          const int tj = safe_type((int)__double_as_longlong(pj[r].w), T);
+          tj = safe_type((int)__double_as_longlong(pj[r].w), T);
           cr = cut2[ti * T + tj];
           ca = cut2[T * T + ti * T + tj];
         }
         if (d2 < cr) {
           isA = d2 < ca;
           isR = !isA;
-          rec = make_float4((float)x, (float)y, (float)z, __int_as_float(jo[r]));
+          rec = make_float4((float)x, (float)y, (float)z, __int_as_float(ONE ? jo[r] : edge_word(w.typed, jo[r], tj)));
         }
       }
       const unsigned gA = (unsigned)((__ballot(isA) >> (gw * G)) & gmask);
       const unsigned gR = (unsigned)((__ballot(isR) >> (gw * G)) & gmask);
-      // every row entry gets its angular slot or -1: one contiguous store
-      const int a = na + __popc(gA & below);
+      const int a = pa + __popc(gA & below), q = pr + __popc(gR & below);
       if (CAND) {
         // candidate rows hold the slot itself (its position is read every
         // step); the reverse index becomes a candidate slot in k_split_reverse
-        if (jj[r] >= 0) w.cpos[vrow + p] = (isA && a < w.MA) ? a : -1;
-        if (isA && a < w.MA) {
-          w.cl[vrow + a] = jj[r];
-          w.cq[arow + a] = qq[r] >= 0 ? jo[r] * w.MV + qq[r] : -1;
+        if (jj[r] >= 0) w.cpos[vrow + p] = isA ? na + a : -1;
+        if (isA) {
+          w.cl[vrow + na + a] = jj[r];
+          w.cq[vrow + na + a] = qq[r] >= 0 ? jo[r] * w.MV + qq[r] : -1;
         }
-        if (isR) {
-          const int slot = w.MV - 1 - (nro + __popc(gR & below));
-          if (slot >= 0) w.cl[vrow + slot] = jj[r];
-        }
+        if (isR) w.cl[vrow + w.MV - 1 - (nro + q)] = jj[r];
       } else {
         const int base = p0 + r * G;
         if (lg == 0 && base < nv) {
@@ -176,35 +186,50 @@ __global__ __launch_bounds__(kBlock) void k_filter(DevBox b, DevModel m, int c1,
           }
           mword |= gA << (base & 31);
         }
-        if (isA && a < w.MA) {
-          w.edge[erow + a] = rec;
-          w.eq[arow + a] = qq[r] >= 0 ? jo[r] * w.MV + qq[r] : -1;
+        if (isA) {
+          st[a] = rec;
+          sq[a] = (short)qq[r];
         }
-        if (isR) {
-          const int slot = w.MR - 1 - (nro + __popc(gR & below));
-          if (slot >= 0) w.edge[erow + slot] = rec;
-        }
+        if (isR) st[kStage - 1 - q] = rec;
       }
-      na += __popc(gA);
-      nro += __popc(gR);
+      pa += __popc(gA);
+      pr += __popc(gR);
     }
+    if (!CAND) {
+      if (lg == 0) counts[g] = make_int4(na, nro, pa, pr);
+      __syncthreads();
+      const int c = threadIdx.x % PER;
+      const int4 n = counts[c];
+      float4* const erow = w.edge + row_begin(first + c, w.MR);
+      short* const qrow = w.eq + row_begin(first + c, w.MA);
+      for (int k = threadIdx.x / PER; k < n.z; k += G) {
+        erow[(size_t)(n.x + k) * kTile] = stage[c * (kStage + 1) + k];
+        qrow[(size_t)(n.x + k) * kTile] = stage_q[c * (kStage + 2) + k];
+      }
+      for (int k = threadIdx.x / PER; k < n.w; k += G)
+        erow[(size_t)(w.MR - 1 - (n.y + k)) * kTile] = stage[c * (kStage + 1) + kStage - 1 - k];
+      // the next pass's first barrier (the loop condition's) keeps its stage
+      // writes behind these reads
+    }
+    na += pa;
+    nro += pr;
   }
   // na + nro <= nv <= MV = MR = MA: the two ends of a row never meet
   if (!CAND && active && lg == 0 && nv > 0) mrow[mcur] = mword;
   if (active && lg == 0) {
     if (CAND) {
-      w.nrc[i] = min(na + nro, w.MV);
-      w.nac[i] = min(na, w.MA);
+      w.nrc[i] = na + nro;
+      w.nac[i] = na;
     } else {
-      w.nr[i] = min(na + nro, w.MR);
-      w.na[i] = min(na, w.MA);
+      w.nr[i] = na + nro;
+      w.na[i] = na;
     }
   }
 }
 
 // Rebuild-time reverse of the candidate rows: an angular candidate i->j's
-// Verlet reverse index j*MV + q becomes j*MA + (i's angular candidate slot
-// in j's row), or -1 where j has no row in [c1, c2) or i is not one of its
+// Verlet reverse index j*MV + q becomes i's angular candidate slot in j's
+// row, or -1 where j has no row in [c1, c2) or i is not one of its
 // angular candidates.
 template <int G>
 __global__ __launch_bounds__(kBlock) void k_split_reverse(int c1, int c2, int nblocks, DevWork w)
@@ -223,7 +248,7 @@ __global__ __launch_bounds__(kBlock) void k_split_reverse(int c1, int c2, int nb
       const int j = q / w.MV;
       if (j >= c1 && j < c2) {
         const int c = w.cpos[q];
-        if (c >= 0) v = j * w.MA + c;
+        if (c >= 0) v = c;
       }
     }
     w.cq[arow + a] = v;
@@ -234,25 +259,111 @@ __global__ __launch_bounds__(kBlock) void k_split_reverse(int c1, int c2, int nb
 // gather: radial pair force, angular partials, ZBL -> FP64 force/virial
 // ---------------------------------------------------------------------------
 
-// CAND: the radial edges come from the candidate rows (DevWork::split)
+// Radial pair force of one edge: f'_k = (fc/2) x' k U_{k-1} + (fc'/2) (T_k + 1),
+// from recurrences scaled by (fc/2) x' and fc'/2; Gi = sum_k b_i f'_k and Gj
+// with the neighbour's adjoint.
+template <int KR>
+__device__ __forceinline__ void radial_pair(float rcinv, float d, float fc, float fcp, const float* bi, const float* bj,
+                                            float& Gi, float& Gj)
+{
+  const float t = d * rcinv - 1.0f, x = 2.0f * t * t - 1.0f, x2 = 2.0f * x;
+  const float A = 0.5f * fc * (4.0f * t * rcinv), B = 0.5f * fcp;
+  float T0 = B, T1 = x * B, U0 = 0.0f, U1 = A;  // U1 = A U_{k-1}
+  Gi = bi[0] * fcp;
+  Gj = bj[0] * fcp;
+#pragma unroll
+  for (int k = 1; k < KR; ++k) {
+    const float fp = fmaf((float)k, U1, T1 + B);
+    Gi = fmaf(bi[k], fp, Gi);
+    Gj = fmaf(bj[k], fp, Gj);
+    const float T2 = fmaf(x2, T1, -T0), U2 = fmaf(x2, U1, -U0);
+    T0 = T1;
+    T1 = T2;
+    U0 = U1;
+    U1 = U2;
+  }
+}
+
+// FP64 force and virial sums of a lane, each product formed and added by one
+// FP64 FMA (full rate on this chip; an FP32 product, its conversion and an
+// addition are three instructions).  A radial pair's virial is symmetric
+// (r (x) r): its off-diagonal terms are summed once and added to both at the
+// end.
+struct PairSums {
+  double fx = 0.0, fy = 0.0, fz = 0.0;
+  double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  double sxy = 0.0, sxz = 0.0, syz = 0.0;
+  // F_i += (Gi + Gj) r/d; virial_i += r (x) dE_j/dr_ji = r (x) (-Gj r/d)
+  __device__ __forceinline__ void radial(const float4& q, float dinv, float Gi, float Gj)
+  {
+    const double x = q.x, y = q.y, z = q.z, sc = (Gi + Gj) * dinv, gj = -Gj * dinv;
+    fx = fma(sc, x, fx);
+    fy = fma(sc, y, fy);
+    fz = fma(sc, z, fz);
+    const double wx = gj * x, wy = gj * y, wz = gj * z;
+    v[0] = fma(x, wx, v[0]);
+    v[1] = fma(y, wy, v[1]);
+    v[2] = fma(z, wz, v[2]);
+    sxy = fma(x, wy, sxy);
+    sxz = fma(x, wz, sxz);
+    syz = fma(y, wz, syz);
+  }
+  __device__ __forceinline__ void angular(const float4& q, float gx, float gy, float gz, float bx, float by, float bz)
+  {
+    const double x = q.x, y = q.y, z = q.z, wx = bx, wy = by, wz = bz;
+    fx += (double)gx;
+    fy += (double)gy;
+    fz += (double)gz;
+    v[0] = fma(x, wx, v[0]);
+    v[1] = fma(y, wy, v[1]);
+    v[2] = fma(z, wz, v[2]);
+    v[3] = fma(x, wy, v[3]);
+    v[4] = fma(x, wz, v[4]);
+    v[5] = fma(y, wz, v[5]);
+    v[6] = fma(y, wx, v[6]);
+    v[7] = fma(z, wx, v[7]);
+    v[8] = fma(z, wy, v[8]);
+  }
+  __device__ __forceinline__ void fold()
+  {
+    v[3] += sxy;
+    v[6] += sxy;
+    v[4] += sxz;
+    v[7] += sxz;
+    v[5] += syz;
+    v[8] += syz;
+  }
+};
+
+// G lanes per atom share its edges (interleaved rows: the lanes of
+// consecutive atoms read contiguous records); the per-lane FP64 sums are
+// combined with a butterfly over the group at the end.  Each lane takes its
+// edges a batch at a time: the edge records are loaded, then the neighbours'
+// adjoint rows (angular loop: their reverse partials), then all of them are
+// used, so the loads of a batch overlap.
+// What bounds it: about equal parts of vector issue (60% of the cycles on
+// 256,000 Cu atoms) and L1 accesses (three per neighbour row; reading a row's
+// chunks with four lanes and passing them on through LDS saved a fifth of the
+// accesses for as much more vector work: 128 us against 119).  Scaled
+// recurrences (radial_pair), FP64 FMAs (PairSums), DPP sums and, with several
+// types, the atom's own rows in LDS take it from 126 to 112 us there and from
+// 43 to 36 us on 5,832 atoms with 17 basis functions; HBM reads fell from 614
+// to 363 MB with the interleaved edge rows.  One lane per atom takes 141 us.
+// CAND: the radial edges come from the candidate rows (DevWork::split).
 template <int KR, bool ONE, int G, bool CAND>
-__global__ __launch_bounds__(kBlock) void k_gather(DevBox b, DevModel m, int n1, int n2, int nd1, int nd2,
+__global__ __launch_bounds__(kBlock, 4) void k_gather(DevBox b, DevModel m, int n1, int n2, int nd1, int nd2,
                                                    int nblocks, const int* __restrict__ type, int N,
                                                    double* __restrict__ force, double* __restrict__ virial,
                                                    int accumulate, DevWork w)
 {
-  // G lanes per atom share its edges; the per-lane FP64 sums are combined
-  // with a butterfly over the group at the end.  Each lane takes its edges
-  // RB at a time: the RB edge records are loaded, then the RB neighbour
-  // adjoint rows, then all of them are used, so the loads of a batch overlap.
   constexpr int PER = kBlock / G;
-  constexpr int RB = KR <= 9 ? kGatherBatch : 2;
+  constexpr int RB = 2, AB = 3;  // radial, angular edges per batch
   static_assert(G >= 1 && G <= 64 && (G & (G - 1)) == 0, "gather lanes: a power of two");
   const int g = threadIdx.x / G, lg = threadIdx.x % G;
-  const int i = n1 + xcd_tile(nblocks) * PER + g;
-  const bool active = i < n2;
+  const int i0 = (n1 & ~(kTile - 1)) + xcd_tile(nblocks) * PER + g;
+  const bool active = i0 >= n1 && i0 < n2;
+  const int i = active ? i0 : n1;
   const int T = ONE ? 1 : m.T;
-  const int kR = m.kR;
   int ti = 0, nr = 0, na = 0, nac = 0;
   double4 pi = make_double4(0.0, 0.0, 0.0, 0.0);
   if (active) {
@@ -268,21 +379,58 @@ __global__ __launch_bounds__(kBlock) void k_gather(DevBox b, DevModel m, int n1,
       nr = w.nr[i];
     }
   }
-  const int* __restrict__ crow = w.cl + (size_t)i * w.MV;
   constexpr int KP = (KR + 3) & ~3;  // padded row: KP/4 float4 loads
   const int kRp = m.kRp;
-  const float4* __restrict__ erow = w.edge + (size_t)i * w.MR;
-  const float4* __restrict__ frow = w.f12 + (size_t)i * w.MA;
-  const int* __restrict__ qrow = w.eq + (size_t)i * w.MA;
+  const float4* __restrict__ erow = w.edge + row_begin(i, w.MR);
+  const float3* __restrict__ frow = w.f12 + row_begin(i, w.MA);
+  const short* __restrict__ qrow = w.eq + row_begin(i, w.MA);
   const float* __restrict__ bR = w.bR;
-  double fx = 0.0, fy = 0.0, fz = 0.0;
-  double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  PairSums sum;
   float bi[KP];
 #pragma unroll
   for (int k = 0; k < KP; ++k) bi[k] = 0.0f;
   if (ONE && active) load_row4<KP>(bR + (size_t)i * kRp, kRp, bi);
   const float rcR0 = (float)((m.rcR[0] + m.rcR[0]) * 0.5);
-  // radial: F_i += (G_i + G_j) r_ij/d with G_c = sum_k b_c[k] f'_k(d)
+  // radial term of one edge (jj >= 0) with the neighbour's adjoint bj
+  constexpr int NC = KP / 4;  // 16-byte chunks of an adjoint row
+  // several types: the atom's own rows, one per neighbour type
+  __shared__ float4 own[ONE ? 1 : PER][ONE ? 1 : kTypesLds][ONE ? 1 : NC];
+  const bool own_lds = !ONE && T <= kTypesLds;
+  if (!ONE && own_lds) {
+    for (int k = lg; k < T * NC; k += G) {
+      const int t = k / NC, c = k % NC;
+      if (active && 4 * c < kRp) own[g][t][c] = reinterpret_cast<const float4*>(bR + ((size_t)i * T + t) * kRp)[c];
+      else own[g][t][c] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    wave_lds_sync();  // an atom's lanes lie in one wavefront
+  }
+  auto radial = [&](const float4& q, float dinv, float d, int tj, const float* bj) {
+    const float rc = ONE ? rcR0 : (float)((m.rcR[ti] + m.rcR[tj]) * 0.5);
+    const float rcinv = 1.0f / rc;
+    float fc, fcp, Gi, Gj;
+    cutoff_fc_fcp(rc, rcinv, d, fc, fcp);
+    if (ONE) {
+      radial_pair<KR>(rcinv, d, fc, fcp, bi, bj, Gi, Gj);
+    } else {
+      float bo[KP];
+      if (own_lds) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) reinterpret_cast<float4*>(bo)[c] = own[g][tj][c];
+      } else {
+#pragma unroll
+        for (int k = 0; k < KP; ++k) bo[k] = 0.0f;
+        load_row4<KP>(bR + ((size_t)i * T + tj) * kRp, kRp, bo);
+      }
+      radial_pair<KR>(rcinv, d, fc, fcp, bo, bj, Gi, Gj);
+    }
+    sum.radial(q, dinv, Gi, Gj);
+  };
+  auto load_adjoint = [&](int j, float* bj) {
+#pragma unroll
+    for (int k = 0; k < KP; ++k) bj[k] = 0.0f;
+    if (j >= nd1 && j < nd2) load_row4<KP>(bR + ((size_t)j * T + ti) * kRp, kRp, bj);
+  };
+  // every edge within the radial cutoff: F_i += (G_i + G_j) r_ij/d
   for (int e0 = lg; e0 < nr; e0 += G * RB) {
     float4 rr[RB];
     int jj[RB], tt[RB];
@@ -290,14 +438,20 @@ __global__ __launch_bounds__(kBlock) void k_gather(DevBox b, DevModel m, int n1,
 #pragma unroll
       for (int r = 0; r < RB; ++r) {
         const int e = e0 + r * G;
-        rr[r] = make_float4(0.f, 0.f, 0.f, 0.f);
         jj[r] = -1;
+        tt[r] = 0;
+        rr[r] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (e < nr) {
-          rr[r] = erow[e < na ? e : w.MR - 1 - (e - na)];
+          rr[r] = erow[(size_t)(e < na ? e : w.MR - 1 - (e - na)) * kTile];
           jj[r] = __float_as_int(rr[r].w);
+          if (!ONE) {
+            tt[r] = edge_type(w, type, jj[r], T);
+            jj[r] = edge_slot(w.typed, jj[r]);
+          }
         }
       }
     } else {
+      const int* __restrict__ crow = w.cl + (size_t)i * w.MV;
       int jc[RB];
       double4 pj[RB];
 #pragma unroll
@@ -311,12 +465,16 @@ __global__ __launch_bounds__(kBlock) void k_gather(DevBox b, DevModel m, int n1,
       for (int r = 0; r < RB; ++r) {
         rr[r] = make_float4(0.f, 0.f, 0.f, 0.f);
         jj[r] = -1;
+        tt[r] = 0;
         if (jc[r] >= 0) {
           double x = pj[r].x - pi.x, y = pj[r].y - pi.y, z = pj[r].z - pi.z;
           mic(b, x, y, z);
           const double d2 = dist2(x, y, z);
           double rc = (m.rcR[0] + m.rcR[0]) * 0.5;
-          if (!ONE) rc = (m.rcR[ti] + m.rcR[safe_type((int)__double_as_longlong(pj[r].w), T)]) * 0.5;
+          if (!ONE) {
+            tt[r] = safe_type((int)__double_as_longlong(pj[r].w), T);
+            rc = (m.rcR[ti] + m.rcR[tt[r]]) * 0.5;
+          }
           if (d2 < rc * rc) {
             jj[r] = w.map.owner ? w.map.owner[jc[r]] : jc[r];
             rr[r] = make_float4((float)x, (float)y, (float)z, __int_as_float(jj[r]));
@@ -324,86 +482,54 @@ __global__ __launch_bounds__(kBlock) void k_gather(DevBox b, DevModel m, int n1,
         }
       }
     }
+    float bj[RB][KP];
 #pragma unroll
-    for (int r = 0; r < RB; ++r) tt[r] = (ONE || jj[r] < 0) ? 0 : safe_type(type[jj[r]], T);
-    float bj[RB][KP], bo[ONE ? 1 : RB][KP];
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-#pragma unroll
-      for (int k = 0; k < KP; ++k) bj[r][k] = 0.0f;
-      if (jj[r] >= nd1 && jj[r] < nd2) load_row4<KP>(bR + ((size_t)jj[r] * T + ti) * kRp, kRp, bj[r]);
-      if (!ONE) {
-#pragma unroll
-        for (int k = 0; k < KP; ++k) bo[ONE ? 0 : r][k] = 0.0f;
-        if (jj[r] >= 0) load_row4<KP>(bR + ((size_t)i * T + tt[r]) * kRp, kRp, bo[ONE ? 0 : r]);
-      }
-    }
+    for (int r = 0; r < RB; ++r) load_adjoint(jj[r], bj[r]);
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
       const float4 q = rr[r];
-      // lanes past the row end carry r = 0: d = 0 and 1/d = 0 there
+      // lanes past the row end carry r = 0: d = 0 and 1/d = 0 there, so every term is zero
       const float d2 = q.x * q.x + q.y * q.y + q.z * q.z;
       const float dinv = jj[r] >= 0 ? __builtin_amdgcn_rsqf(d2) : 0.0f;
-      const float d = d2 * dinv;
-      const float rc = ONE ? rcR0 : (float)((m.rcR[ti] + m.rcR[tt[r]]) * 0.5);
-      const float rcinv = 1.0f / rc;
-      float fc, fcp;
-      cutoff_fc_fcp(rc, rcinv, d, fc, fcp);
-      float f[KR], fp[KR];
-      cheb_d<KR>(kR, rcinv, d, fc, fcp, f, fp);
-      float Gi = 0.0f, Gj = 0.0f;
-#pragma unroll
-      for (int k = 0; k < KR; ++k) {
-        Gi += (ONE ? bi[k] : bo[ONE ? 0 : r][k]) * fp[k];
-        Gj += bj[r][k] * fp[k];
-      }
-      const float sc = (Gi + Gj) * dinv;  // zero past the row end
-      fx += (double)(sc * q.x);
-      fy += (double)(sc * q.y);
-      fz += (double)(sc * q.z);
-      // virial_i += r_ij (x) dE_j/dr_ji,  dE_j/dr_ji = -Gj r_ij/d
-      const float gj = -Gj * dinv;
-      const float fjx = gj * q.x, fjy = gj * q.y, fjz = gj * q.z;
-      v[0] += (double)(q.x * fjx);
-      v[1] += (double)(q.y * fjy);
-      v[2] += (double)(q.z * fjz);
-      v[3] += (double)(q.x * fjy);
-      v[4] += (double)(q.x * fjz);
-      v[5] += (double)(q.y * fjz);
-      v[6] += (double)(q.y * fjx);
-      v[7] += (double)(q.z * fjx);
-      v[8] += (double)(q.z * fjy);
+      radial(q, dinv, d2 * dinv, tt[r], bj[r]);
     }
   }
-  // angular: F_i += dE_i/dr_ij - dE_j/dr_ji; the second term is read from
-  // j's row at the slot where i sits (Verlet reverse position -> angular slot)
-  constexpr int AB = 3;
+  // angular edges: F_i += dE_i/dr_ij - dE_j/dr_ji (the second term is read
+  // from j's row at the slot where i sits: Verlet reverse position -> angular
+  // slot), and ZBL
   for (int e0 = lg; e0 < na; e0 += G * AB) {
-    float4 rr[AB], aa[AB], bb[AB];
-    int jj[AB], qv[AB], e2[AB];
+    float4 rr[AB];
+    float3 aa[AB], bb[AB];
+    int jj[AB], qv[AB], tt[AB];
 #pragma unroll
     for (int r = 0; r < AB; ++r) {
       const int e = e0 + r * G;
-      rr[r] = aa[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+      rr[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+      aa[r] = make_float3(0.f, 0.f, 0.f);
       jj[r] = qv[r] = -1;
+      tt[r] = 0;
       if (e < na) {
-        rr[r] = erow[e];
-        aa[r] = frow[e];
-        qv[r] = qrow[e];
+        rr[r] = erow[(size_t)e * kTile];
+        aa[r] = frow[(size_t)e * kTile];
+        qv[r] = qrow[(size_t)e * kTile];
         jj[r] = __float_as_int(rr[r].w);
+        if (!ONE) {
+          tt[r] = edge_type(w, type, jj[r], T);
+          jj[r] = edge_slot(w.typed, jj[r]);
+        }
       }
     }
-    const int lim = w.rcap * w.MV;
 #pragma unroll
     for (int r = 0; r < AB; ++r) {
-      e2[r] = -1;
-      if (jj[r] >= nd1 && jj[r] < nd2 && qv[r] >= 0 && qv[r] < lim) {
+      bb[r] = make_float3(0.f, 0.f, 0.f);
+      int e2 = -1;
+      const int q = qv[r];
+      if (jj[r] >= nd1 && jj[r] < nd2 && q >= 0 && q < w.MV) {
         if (CAND) {
-          e2[r] = w.vsa[qv[r]];
+          e2 = w.vsa[(size_t)jj[r] * w.MA + q];
         } else {
-          // i's Verlet position q in j's row (qv = j MV + q); its angular
-          // slot is the number of angular entries of j's row before it
-          const int q = qv[r] - jj[r] * w.MV;
+          // i's Verlet position q in j's row; its angular slot is the number
+          // of angular entries of j's row before it
           const int mw = (w.MV + 31) >> 5;
           const unsigned* mk = w.amask + (size_t)jj[r] * mw;
           if (mw == 4) {
@@ -415,23 +541,19 @@ __global__ __launch_bounds__(kBlock) void k_gather(DevBox b, DevModel m, int n1,
             if ((word >> (q & 31)) & 1u) {
               int c = __popc(word & ((1u << (q & 31)) - 1u));
               c += (wq > 0 ? __popc(m4.x) : 0) + (wq > 1 ? __popc(m4.y) : 0) + (wq > 2 ? __popc(m4.z) : 0);
-              e2[r] = c;
+              e2 = c;
             }
           } else {
             const unsigned word = mk[q >> 5];
             if ((word >> (q & 31)) & 1u) {
               int c = __popc(word & ((1u << (q & 31)) - 1u));
               for (int k = 0; k < (q >> 5); ++k) c += __popc(mk[k]);
-              e2[r] = c;
+              e2 = c;
             }
           }
         }
       }
-    }
-#pragma unroll
-    for (int r = 0; r < AB; ++r) {
-      bb[r] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (e2[r] >= 0 && e2[r] < w.MA) bb[r] = w.f12[(size_t)jj[r] * w.MA + e2[r]];
+      if (e2 >= 0 && e2 < w.MA) bb[r] = w.f12[row_begin(jj[r], w.MA) + (size_t)e2 * kTile];
     }
 #pragma unroll
     for (int r = 0; r < AB; ++r) {
@@ -442,11 +564,10 @@ __global__ __launch_bounds__(kBlock) void k_gather(DevBox b, DevModel m, int n1,
       if (m.zbl && jj[r] >= 0) {
         // each directed pair carries half of the ZBL pair gradient
         // (nep_utilities.cuh:347-433 switch, nep.cu ZBL pass)
-        const int tj = ONE ? 0 : safe_type(type[jj[r]], T);
         const float d = sqrtf(q.x * q.x + q.y * q.y + q.z * q.z);
         const float dinv = 1.0f / d;
         float zf, zfp;
-        zbl_pair(m.zblp + (size_t)(ti * m.T + tj) * 12, d, dinv, zf, zfp);
+        zbl_pair(m.zblp + (size_t)(ti * m.T + tt[r]) * 12, d, dinv, zf, zfp);
         const float h = 0.5f * zfp * dinv;  // dE_i/dr_ij = h r_ij
         const float c = jdep ? 2.0f * h : h;
         gx += c * q.x;
@@ -458,41 +579,28 @@ __global__ __launch_bounds__(kBlock) void k_gather(DevBox b, DevModel m, int n1,
           bz -= h * q.z;
         }
       }
-      fx += (double)gx;
-      fy += (double)gy;
-      fz += (double)gz;
-      v[0] += (double)(q.x * bx);
-      v[1] += (double)(q.y * by);
-      v[2] += (double)(q.z * bz);
-      v[3] += (double)(q.x * by);
-      v[4] += (double)(q.x * bz);
-      v[5] += (double)(q.y * bz);
-      v[6] += (double)(q.y * bx);
-      v[7] += (double)(q.z * bx);
-      v[8] += (double)(q.z * by);
+      sum.angular(q, gx, gy, gz, bx, by, bz);
     }
   }
+  sum.fold();
+  sum.fx = group_sum<G>(sum.fx);
+  sum.fy = group_sum<G>(sum.fy);
+  sum.fz = group_sum<G>(sum.fz);
 #pragma unroll
-  for (int off = 1; off < G; off <<= 1) {
-    fx += __shfl_xor(fx, off, G);
-    fy += __shfl_xor(fy, off, G);
-    fz += __shfl_xor(fz, off, G);
-#pragma unroll
-    for (int c = 0; c < 9; ++c) v[c] += __shfl_xor(v[c], off, G);
-  }
+  for (int c = 0; c < 9; ++c) sum.v[c] = group_sum<G>(sum.v[c]);
   if (!active || lg != 0) return;
   if (accumulate) {
-    force[i] += fx;
-    force[N + i] += fy;
-    force[2 * N + i] += fz;
+    force[i] += sum.fx;
+    force[N + i] += sum.fy;
+    force[2 * N + i] += sum.fz;
 #pragma unroll
-    for (int c = 0; c < 9; ++c) virial[(size_t)c * N + i] += v[c];
+    for (int c = 0; c < 9; ++c) virial[(size_t)c * N + i] += sum.v[c];
   } else {
-    force[i] = fx;
-    force[N + i] = fy;
-    force[2 * N + i] = fz;
+    force[i] = sum.fx;
+    force[N + i] = sum.fy;
+    force[2 * N + i] = sum.fz;
 #pragma unroll
-    for (int c = 0; c < 9; ++c) virial[(size_t)c * N + i] = v[c];
+    for (int c = 0; c < 9; ++c) virial[(size_t)c * N + i] = sum.v[c];
   }
 }
 
@@ -865,7 +973,7 @@ hipError_t launch_split(const DevBox& b, const DevModel& m, int c1, int c2, DevW
 {
   if (!w.split || !w.cl) return hipErrorInvalidValue;
   if (c2 > c1) {
-    if (lanes == 8) run_filter<8, kFilterBatch, true>(b, m, c1, c2, 0, w, s);
+    if (lanes == 8) run_filter<8, 7, true>(b, m, c1, c2, 0, w, s);
     else if (lanes == 32) run_filter<32, 4, true>(b, m, c1, c2, 0, w, s);
     else run_filter<kFilterLanes, kFilterBatch, true>(b, m, c1, c2, 0, w, s);
   } else {
@@ -879,7 +987,7 @@ hipError_t launch_filter(const DevBox& b, const DevModel& m, int c1, int c2, Dev
 {
   if (c2 > c1) {
     const int cl = close ? 1 : 0;
-    if (lanes == 8) run_filter<8, kFilterBatch>(b, m, c1, c2, cl, w, s);
+    if (lanes == 8) run_filter<8, 7>(b, m, c1, c2, cl, w, s);
     else if (lanes == 32) run_filter<32, 4>(b, m, c1, c2, cl, w, s);
     else run_filter<kFilterLanes, kFilterBatch>(b, m, c1, c2, cl, w, s);
   } else if (close) {
@@ -893,7 +1001,7 @@ static void run_gather(const DevBox& b, const DevModel& m, int N, int n1, int n2
                        double* force, double* virial, int a, DevWork& w, hipStream_t s)
 {
   constexpr int per = kBlock / G;
-  const int nb = (n2 - n1 + per - 1) / per;
+  const int nb = (n2 - (n1 & ~(kTile - 1)) + per - 1) / per;
   const int g = xcd_grid(nb);
   auto pick = [&](auto k_rows, auto k_cand) { return w.split ? k_cand : k_rows; };
   decltype(&k_gather<9, true, G, false>) k;
@@ -1187,7 +1295,7 @@ __device__ __forceinline__ int serve_request_of(int R, const ServeSlots* __restr
 constexpr int kCarryLanes = 16;  // lanes per row in k_serve_carry_rows
 
 __global__ void k_serve_carry_rows(int R, const ServeSlots* __restrict__ req, int old_no, int o_keep,
-                                   const int* __restrict__ vl0, const int* __restrict__ vrev0,
+                                   const int* __restrict__ vl0, const short* __restrict__ vrev0,
                                    const int* __restrict__ vn0, DevWork w)
 {
   const int s = blockIdx.x * (blockDim.x / kCarryLanes) + threadIdx.x / kCarryLanes;
@@ -1297,7 +1405,7 @@ hipError_t launch_serve_assemble(int R, const ServeSlots* req, const ServeLayout
 }
 
 hipError_t launch_serve_carry_rows(int R_keep, const ServeSlots* req, int old_no, int old_nt, int new_no, int new_nt,
-                                   int o_keep, int g_keep, const int* vl0, const int* vrev0, const int* vn0,
+                                   int o_keep, int g_keep, const int* vl0, const short* vrev0, const int* vn0,
                                    const double* x0_0, DevWork& w, hipStream_t s)
 {
   if (R_keep <= 0) return hipSuccess;

@@ -101,8 +101,18 @@ __host__ __device__ inline int image_neg(int code)
 
 // Per-atom / per-edge workspaces (device pointers), sized for `cap` slots;
 // the per-centre arrays (rows, row lengths, radial adjoints) for the first
-// `rcap` slots, the ones that can be centres.  Row arrays are row-major:
-// entry p of centre i lives at [i*M + p].
+// `rcap` slots, the ones that can be centres.  The edge rows (edge, eq, f12)
+// are interleaved by tiles of 64 centres, the atoms of a wavefront of the
+// descriptor: entry p of centre i lives at row_begin(i, M) + p * kTile, so that
+// the wavefront's 64 entries p are contiguous (16-byte records: eight full
+// lines per load, where row-major rows touch 64) and no line of a row's unused
+// middle is moved.  The other row arrays are row-major, [i*M + p]: the filter
+// reads them with a group of lanes per centre.
+constexpr int kTile = 64;
+static_assert(sizeof(float3) == 12, "angular partials are packed");
+__host__ __device__ inline size_t row_begin(int i, int M) { return (size_t)(i >> 6) * M * kTile + (i & 63); }
+// entries of an interleaved row array for rc centres
+inline size_t row_entries(size_t rc, int M) { return (rc + kTile - 1) / kTile * kTile * (size_t)M; }
 // (Every field is part of NepEngine::launch_key: a captured launch takes
 // the struct by value.)
 struct DevWork {
@@ -120,20 +130,24 @@ struct DevWork {
   int* cell_tiles = nullptr;   // [2 (ncell/4096 + 2) + 8] tile sums, then (16-byte aligned) offsets, of the multi-block scan
   int* vn = nullptr;           // [cap] Verlet row length
   int* vl = nullptr;           // [cap*MV] Verlet rows
-  int* vrev = nullptr;         // [cap*MV] position of the centre in the neighbour's row
+  short* vrev = nullptr;       // [cap*MV] position of the centre in the neighbour's row (rows hold
+                               // at most 4096 entries), -1 if the neighbour has no row
   double* x0 = nullptr;        // [3*cap] positions at the last rebuild
   int* nr = nullptr;           // [cap] radial row length
   int* na = nullptr;           // [cap] angular row length
-  float4* edge = nullptr;      // [cap*MR] (rx, ry, rz, bits(j)): angular edges at
+  float4* edge = nullptr;      // [tiles*MR*64] (rx, ry, rz, bits(edge_word)): angular edges at
                                // 0..na-1, radial-only edges at MR-1 downward
-  int* eq = nullptr;           // [cap*MA] of an angular edge i->j: j*MV + (position of i in
-                               // j's Verlet row), whose angular bit gives i's slot in j's
+  // 1: an edge's word holds the neighbour's type above its slot (every slot
+  // fits kEdgeSlotBits), so its readers need no gather of types
+  int typed = 0;
+  short* eq = nullptr;         // [tiles*MA*64] of an angular edge i->j: the position of i in
+                               // j's Verlet row, whose angular bit gives i's slot in j's
                                // angular row; -1 if j has no row
   int* vsa = nullptr;          // [cap*MV] with candidate rows only: candidate slot -> angular slot, -1 if none
   unsigned* amask = nullptr;   // [cap*ceil(MV/32)] per-step filter: bit p of row i set when Verlet
                                // entry p is angular (its angular slot: the set bits below p)
   float* bR = nullptr;         // [cap*T*kRp] radial adjoint in basis space
-  float4* f12 = nullptr;       // [cap*MA] dE_i/dr_ij of angular edges
+  float3* f12 = nullptr;       // [tiles*MA*64] dE_i/dr_ij of angular edges
   // Rows split by type pair at rebuild time (split != 0): the step has no
   // filter pass; the descriptor and the gather read candidate rows, form the
   // FP64 distances themselves, and the descriptor writes the step's angular
@@ -144,8 +158,8 @@ struct DevWork {
                                // rc + skin, angular candidates (rcA + skin) at 0..nac-1,
                                // radial-only ones at MV-1 downward
   int* cpos = nullptr;         // [cap*MV] Verlet position -> angular candidate slot, -1 if none
-  int* cq = nullptr;           // [cap*MA] of an angular candidate i->j: j*MA + (i's angular
-                               // candidate slot in j's row), an index into vsa; -1 if none
+  int* cq = nullptr;           // [cap*MA] of an angular candidate i->j: i's angular candidate
+                               // slot in j's row; -1 if none
   int* nrc = nullptr;          // [cap] candidates
   int* nac = nullptr;          // [cap] angular candidates
   ImageMap map;                // periodic-image map of the current call (empty: none)
@@ -153,6 +167,13 @@ struct DevWork {
   double* partial = nullptr;   // thermo block partials
   double* thermo = nullptr;    // [8]
 };
+
+// The fourth word of an edge record: the neighbour's slot (the owner's, under
+// an image map) and, in typed rows, its type above kEdgeSlotBits.
+constexpr int kEdgeSlotBits = 27;
+static_assert(kMaxTypes <= 1 << (31 - kEdgeSlotBits), "a type index fits above the slot");
+__host__ __device__ inline int edge_word(int typed, int j, int t) { return typed ? j | (t << kEdgeSlotBits) : j; }
+__host__ __device__ inline int edge_slot(int typed, int v) { return typed ? v & ((1 << kEdgeSlotBits) - 1) : v; }
 
 // Status words in DevWork::flags
 enum : int {
@@ -334,7 +355,7 @@ hipError_t launch_serve_drift(int n_owned, int Nt, const int* atom_req, const do
 // old_nt) plus the translation, in w.x0 (stride new_nt).
 // Their owned slots are [0, o_keep), their ghosts [new_no, g_keep).
 hipError_t launch_serve_carry_rows(int R_keep, const ServeSlots* req, int old_no, int old_nt, int new_no, int new_nt,
-                                   int o_keep, int g_keep, const int* vl0, const int* vrev0, const int* vn0,
+                                   int o_keep, int g_keep, const int* vl0, const short* vrev0, const int* vn0,
                                    const double* x0_0, DevWork& w, hipStream_t s);
 // One finished request for launch_serve_extract: its owned slots, the
 // offset of its block in the output, its placement translation and its box.

@@ -641,8 +641,8 @@ __global__ __launch_bounds__(256) void k_verlet_reverse(const int* __restrict__ 
     for (int u = 0; u < kRevBatch; ++u) {
       const int p = p0 + u * kRowLanes;
       if (own[u]) {
-        w.vrev[(size_t)i * w.MV + p] = q[u];
-        if (!im.owner && q[u] >= 0) w.vrev[(size_t)ov[u] * w.MV + q[u]] = p;
+        w.vrev[(size_t)i * w.MV + p] = (short)q[u];
+        if (!im.owner && q[u] >= 0) w.vrev[(size_t)ov[u] * w.MV + q[u]] = (short)p;
       }
     }
   }

@@ -234,4 +234,51 @@ __device__ __forceinline__ void load_row4(const float* __restrict__ row, int kp,
   }
 }
 
+// sum of v over the P consecutive lanes of a lane group (every lane gets the
+// same bits: each stage adds two partners that hold each other's value), with
+// the lane permutations of the DPP adds (one instruction per stage)
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v)
+{
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v)
+{
+  return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true),
+                          __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true));
+}
+template <int P, class V>
+__device__ __forceinline__ V group_sum(V v)
+{
+  static_assert(P == 1 || P == 4 || P == 8 || P == 16, "lane groups of 4, 8 or 16");
+  if (P >= 4) {
+    v += dpp_move<0xB1>(v);  // quad_perm [1,0,3,2]
+    v += dpp_move<0x4E>(v);  // quad_perm [2,3,0,1]
+  }
+  if (P >= 8) v += dpp_move<0x141>(v);   // row_half_mirror
+  if (P >= 16) v += dpp_move<0x140>(v);  // row_mirror
+  return v;
+}
+
+// multi-type models with at most this many types keep their coefficient
+// blocks (descriptor) and adjoint rows (gather) in LDS
+constexpr int kTypesLds = 4;
+
+// orders this wavefront's LDS writes before its later LDS reads (each
+// wavefront works in its own LDS region, so no workgroup barrier is needed)
+__device__ __forceinline__ void wave_lds_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// the value of lane L of the quad
+template <int L>
+__device__ __forceinline__ int quad_lane(int v)
+{
+  return __builtin_amdgcn_mov_dpp(v, L * 0x55, 0xf, 0xf, true);
+}
+
 }  // namespace dmgx

@@ -196,7 +196,8 @@ struct Server::Lane {
   DBuf<double> home, home2;  // owned slots' positions where their request's shell was built
   // the previous layout's Verlet rows (and the displacement references of its
   // slots), copied out of the engine at a relayout for the continuing requests
-  DBuf<int> vl0, vrev0, vn0;
+  DBuf<int> vl0, vn0;
+  DBuf<short> vrev0;
   DBuf<double> x00;
   DBuf<int> req_flag;        // active request -> 1 once an atom drifted past the shell's budget
   DBuf<int> req_moved;       // layout request -> 1 once an atom moved skin/2 since its rows were built
@@ -258,8 +259,9 @@ struct Server::Lane {
                             &g_shift2, &out, &home, &home2, &x00})
       b->release();
     for (DBuf<int>* b : {&type, &type2, &atom_req, &req_md, &owner, &owner2, &image, &image2, &gstart, &gstart2,
-                         &req_flag, &req_moved, &req_off, &lists, &vl0, &vrev0, &vn0})
+                         &req_flag, &req_moved, &req_off, &lists, &vl0, &vn0})
       b->release();
+    vrev0.release();
     if (h_drift) (void)hipHostFree(h_drift);
     h_drift = nullptr;
     h_drift_cap = 0;
@@ -286,7 +288,7 @@ double Server::slot_bytes(int model, bool owned) const
   // reverse slots copied at a relayout for the continuing requests
   const NepEngine& e = *lanes_[(size_t)model]->nep;
   if (!owned) return e.bytes_per_slot(false) + kLayoutSlotBytes;
-  return e.bytes_per_slot(true) + kLayoutSlotBytes + 2.0 * 4.0 * std::max(e.work().MV, 1);
+  return e.bytes_per_slot(true) + kLayoutSlotBytes + (4.0 + 2.0) * std::max(e.work().MV, 1);
 }
 
 void Server::pin_put(void* p, size_t cap)
@@ -844,7 +846,7 @@ void Server::relayout(Lane& L)
     L.vn0.need(old_no, "serve carried row lengths");
     L.x00.need(3LL * old_nt, "serve carried references");
     check(hipMemcpyAsync(L.vl0.p, ew.vl, rows * 4, hipMemcpyDeviceToDevice, L.stream), "serve carry rows");
-    check(hipMemcpyAsync(L.vrev0.p, ew.vrev, rows * 4, hipMemcpyDeviceToDevice, L.stream), "serve carry reverse");
+    check(hipMemcpyAsync(L.vrev0.p, ew.vrev, rows * sizeof(short), hipMemcpyDeviceToDevice, L.stream), "serve carry reverse");
     check(hipMemcpyAsync(L.vn0.p, ew.vn, (size_t)old_no * 4, hipMemcpyDeviceToDevice, L.stream), "serve carry lengths");
     check(hipMemcpyAsync(L.x00.p, ew.x0, (size_t)old_nt * 24, hipMemcpyDeviceToDevice, L.stream),
           "serve carry references");
