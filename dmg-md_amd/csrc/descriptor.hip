@@ -54,7 +54,7 @@ extern template void run_generic<kMaxL>(const DescriptorCall&);
 hipError_t launch_descriptor(const DevBox& b, const DevModel& m, int N, int c1, int c2, const int* type, double* pe,
                              bool acc, int ann, DevWork& w, hipStream_t s, hipEvent_t e0, hipEvent_t e1, int lanes)
 {
-  if (lanes != 1 && lanes != 4) return hipErrorInvalidValue;
+  if (lanes != 1 && lanes != 4 && lanes != 16) return hipErrorInvalidValue;
   if (c2 <= c1) return hipSuccess;
   const DescriptorCall a{b, m, N, c1, c2, type, pe, acc ? 1 : 0, ann, lanes, w, s, e0, e1};
   auto is = [&](int nr, int kr, int na, int ka, bool q2, bool q1, bool one) {

@@ -39,10 +39,6 @@ struct Cfg {
   // registers that leave two wavefronts per SIMD; through LDS (ann_mfma) else
   static constexpr bool ann_rows =
       ANN == kAnnMfma32 && ONE && EXACT && NA * nabc + 4 * ((dim + 3) / 4) + 16 * ((dim + 15) / 16) <= 216;
-  // wavefronts per SIMD the registers are allocated for: two for the
-  // single-type matrix-core instances (120 moments of 256 registers), one for
-  // the wider ones, which would spill
-  static constexpr int waves = EXACT && ONE && ANN != kAnnValu && NA * nabc <= 128 ? 2 : 1;
 };
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -56,10 +52,10 @@ __device__ __forceinline__ short to_bf16(float x)
   return (short)(u >> 16);
 }
 
-// LDS floats per wavefront of the matrix-core ANN: 64 rows of DMAX+1 (odd
-// stride), then 64 energies
+// LDS floats per wavefront of the matrix-core ANN: 64 rows of an odd
+// stride, then 64 energies
 template <int DMAX>
-constexpr int ann_lds_floats() { return 64 * (DMAX + 1) + 128; }
+constexpr int ann_lds_floats() { return 64 * (DMAX | 1) + 128; }
 
 // ANN of the 64 atoms of a wavefront on the matrix cores (single-type
 // model, H <= 64).  Lane l holds atom l's scaled descriptor q[0..D).
@@ -77,7 +73,7 @@ constexpr int ann_lds_floats() { return 64 * (DMAX + 1) + 128; }
 // padded to 64 hidden units with an odd row stride (no bank conflicts), then
 // b0 and w1 (zero past H)
 template <int DMAX>
-constexpr int ann_w_stride() { return DMAX + 1; }
+constexpr int ann_w_stride() { return DMAX | 1; }
 // floats of W0 rows: 64 x WS floats, or with SPLIT three bfloat16 parts of
 // 64 x WS shorts each (96 x WS floats); then b0 and w1
 template <int DMAX, bool SPLIT = false>
@@ -148,7 +144,7 @@ __device__ __forceinline__ void ann_mfma(const DevModel& m, int D, const float* 
   // method of Henry, Tang and Heinecke (ARITH 2019)
   constexpr bool BF16 = MODE == kAnnMfmaBf16;
   constexpr bool X3 = MODE == kAnnMfmaSplit;
-  constexpr int DS = DMAX + 1;
+  constexpr int DS = DMAX | 1;
   constexpr int DT = (DMAX + 15) / 16;
   const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
   float* Qs = lds;
@@ -460,6 +456,20 @@ constexpr int desc_lds_bytes()
   return 4 * (pcut + ctab + annw + annl);
 }
 
+// Wavefronts per SIMD an instance's registers are allocated for.  Two (256
+// registers) for the single-type instances with up to 128 moments, and for the
+// several-type matrix-core ones whose LDS lets two workgroups share a CU (606
+// -> 461 us on 192,000 water atoms, with 84 bytes of spills per lane; four
+// lanes per atom on 21,952 carbon atoms 63 -> 44).  One for the wider ones,
+// which would spill hundreds of bytes.
+template <class C, int P>
+constexpr int desc_waves()
+{
+  if (!C::exact) return 1;
+  if (C::one) return C::na * C::nabc <= 128 ? 2 : 1;
+  return P == 1 && C::ann == kAnnMfma32 && desc_lds_bytes<C>() <= 80 * 1024 ? 2 : 1;
+}
+
 template <int NR, int KR, int NA, int KA, bool Q2, bool Q1, bool ONE, int ANN = kAnnMfma32>
 constexpr bool mfma_ann_fits()
 {
@@ -492,7 +502,8 @@ constexpr bool mfma_ann_fits()
 // sums are combined across the group, so every lane holds the atom's
 // descriptor, moments and derivatives.
 template <class C, bool CAND, int P = 1>
-__global__ __launch_bounds__(kDescBlock, C::waves) void k_descriptor(DevBox b, DevModel m, int N, int c1, int c2, int nblocks,
+__global__ __launch_bounds__(kDescBlock, (desc_waves<C, P>())) void k_descriptor(
+                                                       DevBox b, DevModel m, int N, int c1, int c2, int nblocks,
                                                        const int* __restrict__ type, double* __restrict__ pe,
                                                        float4* __restrict__ edge, int* __restrict__ vsa,
                                                        short* __restrict__ eq, int accumulate, DevWork w)
@@ -630,19 +641,20 @@ __global__ __launch_bounds__(kDescBlock, C::waves) void k_descriptor(DevBox b, D
     // radial-only edges, stored from the row's end downward; kAhead records
     // in flight (the work per edge is short).  The angular edges' radial terms
     // are summed in the loop over the angular moments.
-    constexpr int kAhead = 12;
+    constexpr int kAhead = P == 1 ? 12 : 3;
+    const float4* const first = erow + (size_t)(w.MR - 1) * kTile;
     const int nro = nr - na;
     float4 ring[kAhead];
 #pragma unroll
     for (int u = 0; u < kAhead; ++u)
-      ring[u] = u * P + lr < nro ? erow[(size_t)(w.MR - 1 - (u * P + lr)) * kTile] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      ring[u] = u * P + lr < nro ? first[-(ptrdiff_t)(u * P + lr) * kTile] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     for (int e0 = lr; e0 < nro; e0 += kAhead * P)
 #pragma unroll
       for (int u = 0; u < kAhead; ++u) {
         const int e = e0 + u * P;
         if (e >= nro) break;
         const float4 r = ring[u];
-        if (e + kAhead * P < nro) ring[u] = erow[(size_t)(w.MR - 1 - (e + kAhead * P)) * kTile];
+        if (e + kAhead * P < nro) ring[u] = first[-(ptrdiff_t)(e + kAhead * P) * kTile];
         const float d2 = r.x * r.x + r.y * r.y + r.z * r.z;
         radial_edge(d2 * __builtin_amdgcn_rsqf(d2), type_of(r));
       }
@@ -728,7 +740,7 @@ __global__ __launch_bounds__(kDescBlock, C::waves) void k_descriptor(DevBox b, D
   // each lane takes every P-th edge with kRing records in flight: a record
   // comes from beyond L1, and an edge's arithmetic covers a fraction of that
   // (one ahead: 171 us on 256,000 Cu atoms, four: 165)
-  constexpr int kRing = 4;
+  constexpr int kRing = P == 1 ? 4 : 1;
   auto edge_at = [&](int e) { return erow[(size_t)e * kTile]; };
   float4 ring[kRing];
   auto fill_ring = [&]() {
@@ -1109,6 +1121,7 @@ void run_descriptor(const DescriptorCall& a)
 {
   if constexpr (C::ann == kAnnValu) {
     if (a.lanes == 4 && !a.w.split) return launch_instance<C, false, 4>(a);
+    if (a.lanes == 16 && !a.w.split) return launch_instance<C, false, 16>(a);
   }
   if (a.w.split) launch_instance<C, true, 1>(a);
   else launch_instance<C, false, 1>(a);

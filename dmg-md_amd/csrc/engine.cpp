@@ -429,6 +429,7 @@ void NepEngine::set_desc_lanes(int lanes)
 {
   if (lanes != 0 && lanes != 1 && lanes != 4) throw std::invalid_argument("descriptor lanes per atom are 0, 1 or 4");
   tune_.desc_lanes = lanes;
+  tune_.desc_pinned = lanes != 0;
   tune_.tuned = true;
 }
 
@@ -631,7 +632,7 @@ void NepEngine::launch_key(std::vector<long long>& k) const
                         (const void*)w.flags, (const void*)w.partial, (const void*)w.thermo})
     p(q);
   for (int v : {tune_.filter_lanes, tune_.gather_lanes, tune_.row_layout, tune_.overlap, tune_.split,
-                tune_.desc_lanes})
+                tune_.desc_lanes, (int)tune_.desc_pinned})
     k.push_back(v);
 }
 
@@ -787,15 +788,31 @@ void NepEngine::compute(const Box& box, int N, int n1, int n2, int nd1, int nd2,
 // Smallest centre range split for the overlapped schedule: each half keeps
 // at least this many centres (below it the launches are too short to gain)
 constexpr int kOverlapMinCentres = 16384;
-// Below this many centres one lane per atom leaves most SIMDs idle (256 CUs x
-// 4 SIMDs x 64 lanes): the untuned descriptor then takes four lanes per atom
-constexpr int kLaneGroupCentres = 65536;
-
-int NepEngine::desc_lanes(int n, int ann) const
+// Lanes per atom of the untuned descriptor, by the wavefronts that fill the
+// GPU's 1,024 SIMDs.  Its time steps up with each further wavefront per SIMD, so
+// a small system gains from more lanes per atom until they need another.
+// Narrow instances (one type, at most five angular functions) hold two
+// wavefronts per SIMD: sixteen lanes up to 8,192 centres (4,096 carbon atoms:
+// 23 us against 32 with four; 10,648: 39 against 34), four up to 36,864 (32,000
+// Cu atoms: 50 us against 54 with one lane; 48,668: 79 against 56).  The others
+// hold one: sixteen up to 6,144 (5,832 atoms of a 100-neuron model: 110 us
+// against 131; 10,125 water atoms: 88 against 62), four up to 57,344 (46,875
+// water atoms: 165 us against 200; 65,856: 262 against 225).
+struct LaneRule {
+  int wide, group;
+};
+LaneRule lane_rule(const DevModel& m)
 {
-  if (w_.split || (ann != 1 && ann != 0)) return 1;  // candidate rows, or BF16 operands asked for
-  if (tune_.desc_lanes) return tune_.desc_lanes;
-  return n < kLaneGroupCentres ? 4 : 1;
+  return m.T == 1 && m.nA <= 5 && m.L <= kPadL ? LaneRule{8192, 36864} : LaneRule{6144, 57344};
+}
+
+int NepEngine::desc_lanes(int n, int ann, bool split) const
+{
+  if (split || (ann != 1 && ann != 0)) return 1;  // candidate rows, or BF16 operands asked for
+  if (tune_.desc_pinned) return tune_.desc_lanes;
+  const LaneRule rule = lane_rule(dmd_);
+  const int lanes = tune_.desc_lanes ? tune_.desc_lanes : n < rule.group ? 4 : 1;
+  return lanes == 4 && n <= rule.wide ? 16 : lanes;
 }
 
 void NepEngine::launch_filter_descriptor(const DevBox& b, int N, int c1, int c2, const int* type, double* pe,
@@ -816,7 +833,7 @@ void NepEngine::launch_filter_descriptor(const DevBox& b, int N, int c1, int c2,
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     const bool attached = profile && prof_.attach(kProfDescriptor, &ev0, &ev1);
     if (profile && !attached) prof_.begin(kProfDescriptor, s);
-    check(launch_descriptor(b, dmd_, N, c1, c2, type, pe, acc, ann, w_, s, ev0, ev1, desc_lanes(n, ann)),
+    check(launch_descriptor(b, dmd_, N, c1, c2, type, pe, acc, ann, w_, s, ev0, ev1, desc_lanes(n, ann, w_.split != 0)),
           "descriptor");
     if (profile && !attached) prof_.end(s);
     return;
@@ -835,7 +852,7 @@ void NepEngine::launch_filter_descriptor(const DevBox& b, int N, int c1, int c2,
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     if (profile) prof_.attach(kProfDescriptor, &ev0, &ev1);
     check(launch_descriptor(b, dmd_, N, h ? mid : c1, h ? c2 : mid, type, pe, acc, ann, w_, s, ev0, ev1,
-                            desc_lanes(n, ann)),
+                            desc_lanes(n, ann, w_.split != 0)),
           "descriptor");
   }
 }
@@ -953,7 +970,8 @@ const NepEngine::Tuning& NepEngine::autotune(const Box& box, int N, int nc, cons
     }
     tune_.overlap = t[1] < t[0] ? 1 : 0;
   }
-  // one or four lanes per atom in the descriptor (FP32 requests only)
+  // one lane per atom in the descriptor or a group (FP32 requests only)
+  tune_.desc_pinned = false;
   {
     const int ann = ann_mode(flags);
     if (ann == 0 || ann == 1) {
@@ -1145,8 +1163,7 @@ void NepEngine::compute_in(void* ws, size_t ws_bytes, const Box& box, int N, int
   else check(launch_filter(b, dm_, nd1, nd2, w, s, tune_.filter_lanes), "filter");
   const bool acc = (flags & 1u) != 0;
   const int ann = ann_mode(flags);
-  const int lanes = (split || (ann != 1 && ann != 0)) ? 1
-                    : tune_.desc_lanes ? tune_.desc_lanes : (nd2 - nd1 < kLaneGroupCentres ? 4 : 1);
+  const int lanes = desc_lanes(nd2 - nd1, ann, split);
   check(launch_descriptor(b, dmd_, N, nd1, nd2, type, pe, acc, ann, w, s, nullptr, nullptr, lanes), "descriptor");
   check(launch_gather(b, dm_, N, n1, n2, nd1, nd2, type, force, virial, acc, w, s, tune_.gather_lanes), "gather");
   check(hipMemcpyAsync(hflags_, w.flags, kNumFlags * sizeof(int), hipMemcpyDeviceToHost, s), "read status words");

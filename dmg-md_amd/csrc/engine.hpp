@@ -151,11 +151,14 @@ class NepEngine {
     // packed positions, and the descriptor writes the step's angular edges
     int split = 0;
     double split_ms[2] = {0, 0};        // the step's force kernels with the filter / with candidate rows
-    // lanes per atom of the descriptor: 1, 4 (a group of four lanes shares an
+    // lanes per atom of the descriptor: 1, 4 (a group of lanes shares an
     // atom's edges and hidden neurons, the ANN on the vector ALUs in FP32), or
-    // 0 before tuning: four below kLaneGroupCentres centres, else one.  BF16
-    // and split-BF16 ANN requests keep one lane per atom.
+    // 0 before tuning: a group for small systems, else one lane (lane_rule).  A
+    // group is four lanes, or sixteen for the smallest unless set_desc_lanes
+    // asked for four.  BF16 and split-BF16 ANN requests keep one
+    // lane per atom.
     int desc_lanes = 0;
+    bool desc_pinned = false;           // desc_lanes was set, not tuned
     double desc_ms[2] = {0, 0};         // the step's force kernels with 1 / 4 lanes per atom
     bool tuned = false;
   };
@@ -254,7 +257,7 @@ class NepEngine {
   void launch_filter_descriptor(const DevBox& b, int N, int c1, int c2, const int* type, double* pe, bool acc,
                                 int ann, bool close, hipStream_t s, bool profile);
   // lanes per atom of the descriptor for n centres in ANN mode ann
-  int desc_lanes(int n, int ann) const;
+  int desc_lanes(int n, int ann, bool split) const;
   DevBox last_box_{};  // box of the last evaluation (the filter of copy_pair_rows)
   hipStream_t side_ = nullptr;  // the overlapped filter's stream
   hipEvent_t fork_ = nullptr, join_ = nullptr;

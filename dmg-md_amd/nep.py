@@ -193,7 +193,7 @@ class NEP:
 
     def set_desc_lanes(self, lanes: int) -> None:
         """Lanes per atom of the descriptor kernel: 1, 4, or 0 (by system
-        size: four below 65,536 centres)."""
+        size: sixteen or four in small systems)."""
         check(lib().dmgx_nep_set_desc_lanes(self._h, int(lanes)))
 
     def autotune(self, box: Box, type, position, potential, force, virial, *, ann_bf16=False,

@@ -177,9 +177,10 @@ typedef struct dmgx_tuning {
                            entry within its pair's rc + skin) and the step has no filter
                            pass: the descriptor and gather form the distances themselves */
   double split_ms[2];   /* the step's force kernels with the filter / with the split rows */
-  int desc_lanes;       /* lanes per atom of the descriptor: 1, 4 (a group of four lanes shares
-                           an atom's edges and hidden neurons; FP32 ANN on the vector ALUs),
-                           0 before tuning (four below 65,536 centres, else one); BF16 ANN
+  int desc_lanes;       /* lanes per atom of the descriptor: 1, 4 (a group of lanes shares
+                           an atom's edges and hidden neurons, four or, in the smallest
+                           systems unless set, sixteen; FP32 ANN on the vector ALUs), 0
+                           before tuning (a group in small systems, else one); BF16 ANN
                            requests keep one */
   double desc_ms[2];    /* the step's force kernels with 1 / 4 lanes per atom */
 } dmgx_tuning;
@@ -192,7 +193,7 @@ int dmgx_nep_set_tiles(dmgx_nep* nep, int filter_lanes, int gather_lanes);
  * rebuild, with the distance test at the point of use.  The next evaluation
  * rebuilds the rows; a server bound to the handle keeps the choice. */
 int dmgx_nep_set_split(dmgx_nep* nep, int split);
-/* Sets the descriptor's lanes per atom (0: by system size, 1 or 4; no
+/* Sets the descriptor's lanes per atom (0: by system size, 1 or exactly 4; no
  * counterpart in the reference, whose launch shape is fixed); a server bound
  * to the handle keeps the choice. */
 int dmgx_nep_set_desc_lanes(dmgx_nep* nep, int lanes);
