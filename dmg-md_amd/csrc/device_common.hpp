@@ -60,9 +60,11 @@ __device__ __forceinline__ double dist2(double x, double y, double z)
   return (x * x + y * y) + z * z;
 }
 
-// cell coordinates of a position; returns false when a non-periodic
-// coordinate lies outside the box
-__device__ __forceinline__ bool cell_coords(const DevBox& b, double x, double y, double z, int* c)
+// cell coordinates of a position (and with f the position inside the cell,
+// in cell edges); returns false when a non-periodic coordinate lies outside
+// the box
+__device__ __forceinline__ bool cell_coords(const DevBox& b, double x, double y, double z, int* c,
+                                            float* f = nullptr)
 {
   const double s[3] = {b.hi[0] * x + b.hi[1] * y + b.hi[2] * z, b.hi[3] * x + b.hi[4] * y + b.hi[5] * z,
                        b.hi[6] * x + b.hi[7] * y + b.hi[8] * z};
@@ -78,6 +80,7 @@ __device__ __forceinline__ bool cell_coords(const DevBox& b, double x, double y,
     }
     int k = (int)(u * b.nc[d]);
     c[d] = k < 0 ? 0 : (k >= b.nc[d] ? b.nc[d] - 1 : k);
+    if (f) f[d] = (float)(u * b.nc[d] - c[d]);
   }
   return ok;
 }

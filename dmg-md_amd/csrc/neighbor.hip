@@ -15,7 +15,10 @@
 // works on one centre reads and writes contiguous memory.  Build, sort and
 // reverse search run with kRowLanes lanes per centre (4 centres per wave).
 #include <algorithm>
+#include <limits>
+#include <type_traits>
 #include "device_common.hpp"
+#include "nep_math.hpp"
 
 namespace dmgx {
 
@@ -341,12 +344,157 @@ __device__ __forceinline__ bool key_less(const uint64_t* gid, int a, int b)
 constexpr int kRanges = 64;
 constexpr int kRangesPerLane = kRanges / kRowLanes;
 constexpr size_t kRangeLds = 2 * kRanges * sizeof(int);  // starts + prefix, per centre
+// rows of at most this many entries are sorted in registers
+constexpr int kSortMax = 16 * kRowLanes;
 
-// LDS bytes of one centre's row buffers: 64-bit keys (rows keyed by global
-// id only), the accepted slots and the sorted row; a multiple of 8
+// LDS bytes of one centre's row buffers: the accepted slots, with their
+// 64-bit keys where rows are keyed by global id, and the sorted row where
+// the register sort may not hold it; a multiple of 8
 __host__ __device__ inline size_t build_row_lds(int mv, bool keyed)
 {
-  return (keyed ? 16 : 8) * (size_t)mv;
+  return (keyed ? 16 : mv > kSortMax ? 8 : 4) * (size_t)mv;
+}
+
+// Bitonic sort of kRowLanes * E keys held E to a lane (ascending, key
+// lane * E + r in register r): in-lane exchanges, and between lanes the
+// mirrors and swaps that the DPP lane permutations offer.
+template <class K>
+__device__ __forceinline__ void exchange(K& a, K& b)
+{
+  const bool swap = b < a;
+  const K lo = swap ? b : a, hi = swap ? a : b;
+  a = lo;
+  b = hi;
+}
+__device__ __forceinline__ void exchange(int& a, int& b)
+{
+  const int lo = min(a, b), hi = max(a, b);
+  a = lo;
+  b = hi;
+}
+__device__ __forceinline__ int keep(int a, int b, bool upper) { return upper ? max(a, b) : min(a, b); }
+__device__ __forceinline__ uint64_t keep(uint64_t a, uint64_t b, bool upper) { return (b < a) == upper ? a : b; }
+
+// in-lane: merge the halves of each block of S keys, the first step mirrored
+template <int S, bool FLIP, int E, class K>
+__device__ __forceinline__ void merge_in_lane(K (&v)[E])
+{
+#pragma unroll
+  for (int r = 0; r < E; ++r) {
+    const int o = FLIP ? r ^ (S - 1) : r ^ (S / 2);
+    if (o > r) exchange(v[r], v[o]);
+  }
+  if constexpr (S > 2) merge_in_lane<S / 2, false>(v);
+}
+template <int S, int E, class K>
+__device__ __forceinline__ void sort_in_lane(K (&v)[E])
+{
+  if constexpr (S > 2) sort_in_lane<S / 2>(v);
+  if constexpr (S >= 2) merge_in_lane<S, true>(v);
+}
+// between lanes: key r of a lane against key r of its partner lane ...
+template <int CTRL, int E, class K>
+__device__ __forceinline__ void swap_step(K (&v)[E], bool upper)
+{
+#pragma unroll
+  for (int r = 0; r < E; ++r) {
+    K p = dpp_move<CTRL>(v[r]);
+    v[r] = keep(v[r], p, upper);
+  }
+}
+// ... or against key E - 1 - r of the mirrored lane
+template <int CTRL, int E, class K>
+__device__ __forceinline__ void mirror_step(K (&v)[E], bool upper)
+{
+#pragma unroll
+  for (int r = 0; r < E / 2; ++r) {
+    const K a = dpp_move<CTRL>(v[E - 1 - r]), b = dpp_move<CTRL>(v[r]);
+    v[r] = keep(v[r], a, upper);
+    v[E - 1 - r] = keep(v[E - 1 - r], b, upper);
+  }
+}
+template <int E, class K>
+__device__ __forceinline__ void sort_row(K (&v)[E], int lg)
+{
+  const bool b0 = lg & 1, b1 = lg & 2, b2 = lg & 4, b3 = lg & 8;
+  constexpr int kX1 = 0xB1, kX2 = 0x4E, kX3 = 0x1B, kX7 = 0x141, kX15 = 0x140;  // lane ^ 1, 2, 3, 7, 15
+  sort_in_lane<E>(v);
+  mirror_step<kX1>(v, b0);  // two lanes
+  merge_in_lane<E, false>(v);
+  mirror_step<kX3>(v, b1);  // four
+  swap_step<kX1>(v, b0);
+  merge_in_lane<E, false>(v);
+  mirror_step<kX7>(v, b2);  // eight
+  swap_step<kX2>(v, b1);
+  swap_step<kX1>(v, b0);
+  merge_in_lane<E, false>(v);
+  mirror_step<kX15>(v, b3);  // sixteen
+#pragma unroll
+  for (int r = 0; r < E; ++r) {
+    const K p = dpp_move<kX3>(dpp_move<kX7>(v[r]));  // lane ^ 4
+    v[r] = keep(v[r], p, b2);
+  }
+  swap_step<kX2>(v, b1);
+  swap_step<kX1>(v, b0);
+  merge_in_lane<E, false>(v);
+}
+
+// sorts the n <= kRowLanes * E entries of a row and writes them out, four to
+// a store (entries past n within the row's last four are not read by anyone)
+template <bool KEYED, int E>
+__device__ __forceinline__ void write_sorted(const int* row, const uint64_t* key, int n, int lg, bool active,
+                                             int* __restrict__ out)
+{
+  using K = std::conditional_t<KEYED, uint64_t, int>;
+  K v[E];
+#pragma unroll
+  for (int r = 0; r < E; ++r) {
+    const int k = r * kRowLanes + lg;
+    v[r] = std::numeric_limits<K>::max();
+    if (k < n) {
+      if constexpr (KEYED) v[r] = key[k] << 32 | (uint32_t)row[k];
+      else v[r] = row[k];
+    }
+  }
+  sort_row(v, lg);
+#pragma unroll
+  for (int r = 0; r < E; r += 4) {
+    const int k = lg * E + r;
+    if (active && k < n)
+      *reinterpret_cast<int4*>(out + k) = make_int4((int)v[r], (int)v[r + 1], (int)v[r + 2], (int)v[r + 3]);
+  }
+}
+
+// the general form for longer rows and for keys that need all their bits:
+// the rank of every entry among all n, then the row from its sorted copy
+template <bool KEYED>
+__device__ __forceinline__ void write_ranked(const int* row, const uint64_t* key, int* sorted, int n, int lg,
+                                             bool active, int* __restrict__ out)
+{
+  for (int k = lg; k < n; k += kRowLanes) {
+    const int v = row[k];
+    int r = 0;
+    if constexpr (KEYED) {
+      const uint64_t kv = key[k];
+      for (int t = 0; t < n; ++t) {
+        const uint64_t kt = key[t];
+        r += (kt < kv || (kt == kv && row[t] < v)) ? 1 : 0;
+      }
+    } else {
+      // four entries per LDS read (row is 16-byte aligned: MV is a multiple of 4)
+      const int4* row4 = reinterpret_cast<const int4*>(row);
+      const int n4 = n >> 2;
+      for (int t = 0; t < n4; ++t) {
+        const int4 x = row4[t];
+        r += (x.x < v) + (x.y < v) + (x.z < v) + (x.w < v);
+      }
+      for (int t = n4 * 4; t < n; ++t) r += row[t] < v ? 1 : 0;
+    }
+    sorted[r] = v;
+  }
+  wave_lds_sync();
+  if (active)
+    for (int k = lg; k < n; k += kRowLanes) out[k] = sorted[k];
 }
 
 // One kRowLanes group per centre.  The group first reads the bounds of all
@@ -355,11 +503,20 @@ __host__ __device__ inline size_t build_row_lds(int mv, bool keyed)
 // cell_atoms / xs (the cell-ordered copy of the positions), so a candidate
 // costs two independent contiguous loads; each step tests two candidates
 // per lane whose loads were issued a step earlier.  Accepted slots are compacted into LDS
-// with a ballot, rank-sorted there on (key, slot) and written out as one
-// contiguous row.  Rows past the capacity MV are counted but not stored;
-// the count is reported through the flags.
-template <bool LISTED>
-__global__ __launch_bounds__(256) void k_verlet_build(const int* __restrict__ go, DevBox b, int c1, int c2,
+// with a ballot, sorted on (key, slot) and written out as one contiguous
+// row.  Rows past the capacity MV are counted but not stored; the count is
+// reported through the flags.  A group lives inside one wavefront, so there
+// is no workgroup barrier.
+//
+// Bound by vector instructions.  In an orthogonal box a range holds only the
+// cells that a sphere of rc+skin around the centre reaches (84 of the 125 on
+// average), and rows of up to kSortMax entries are sorted in registers: 192,000
+// water atoms (143 entries a row) 316 us against 886 with every cell and rank
+// sorts in LDS, 60,001 keyed rows of 90 92 against 276, 2.3 million rows of 90
+// 1,570 against 2,410.  Four wavefronts per SIMD hold the sort's registers
+// (five: 335, 124 and 1,480 us; six: 389, 199 and 1,950).
+template <bool LISTED, bool KEYED, bool PLAIN>
+__global__ __launch_bounds__(256, 4) void k_verlet_build(const int* __restrict__ go, DevBox b, int c1, int c2,
                                                       int groups, const double4* __restrict__ xq, double rv2,
                                                       const uint64_t* __restrict__ gid, DevWork w)
 {
@@ -369,179 +526,199 @@ __global__ __launch_bounds__(256) void k_verlet_build(const int* __restrict__ go
   const int g = threadIdx.x / kRowLanes, lg = threadIdx.x % kRowLanes;
   const int gw = g % (64 / kRowLanes);  // group inside the wavefront
   // per centre: [keys (with gid only) | row | sorted row], then the ranges
-  const size_t per = build_row_lds(w.MV, gid != nullptr) / sizeof(uint64_t);
+  const size_t per = build_row_lds(w.MV, KEYED) / sizeof(uint64_t);
   uint64_t* key = shk + (size_t)g * per;
-  int* row = reinterpret_cast<int*>(gid ? key + w.MV : key);
+  int* row = reinterpret_cast<int*>(KEYED ? key + w.MV : key);
   int* sorted = row + w.MV;
   int* rs = reinterpret_cast<int*>(shk + (size_t)groups * per) + g * 2 * kRanges;
   int* rp = rs + kRanges;
+  // PLAIN: orthogonal with positive edges.  Cell edges for the trim (0: this
+  // direction is not trimmed, where five periodic cells make the +-2 rows
+  // reach the same atoms from both sides).  kTrim cells of slack cover the
+  // rounding of the cell coordinates.
+  constexpr float kTrim = 1e-3f;
+  const float reach2 = (float)rv2 * (1.0f + kTrim);
+  float edge[3];
+  double len[3], half[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    edge[d] = b.pbc[d] && b.nc[d] < 6 ? 0.0f : (float)(b.thick[d] / b.nc[d]) * (1.0f - kTrim);
+    len[d] = b.h[4 * d];
+    half[d] = b.pbc[d] ? len[d] * 0.5 : std::numeric_limits<double>::infinity();
+  }
+  const float inv_edge_x = 1.0f / edge[0];
   // centres c1 + k, or with compacted lists the listed centres (of the
   // requests this rebuild remakes) inside [c1, c2): a pass per group of
   // `groups` centres, the grid striding over the groups
   const int ncent = LISTED ? w.map.req_off[2 * w.map.n_req] : c2 - c1;
-  for (int pass = 0;; ++pass) {
-  const int base = (blockIdx.x + pass * gridDim.x) * groups;
-  if (base >= ncent) break;
-  const int kc = base + g;
-  const int i = LISTED ? (kc < ncent ? w.map.lists[kc] : -1) : c1 + kc;
-  const bool active = LISTED ? (i >= c1 && i < c2) : (i < c2 && slot_rebuilt(w.map, go_word, i));
-  if (!__syncthreads_or(active)) continue;  // no centre of this pass is rebuilt
-  double4 pi = make_double4(0, 0, 0, 0);
-  int c[3] = {0, 0, 0};
-  if (active) {
-    pi = xq[i];
-    cell_coords(b, pi.x, pi.y, pi.z, c);
-  }
-  // ranges q = 2 * (5 (dz+2) + dy+2) + part, lane lg holding q in
-  // [lg*kRangesPerLane, (lg+1)*kRangesPerLane)
-  int len[kRangesPerLane];
-  int tot = 0;
+  for (int base = blockIdx.x * groups; base < ncent; base += gridDim.x * groups) {
+    const int kc = base + g;
+    const int i = LISTED ? (kc < ncent ? w.map.lists[kc] : -1) : c1 + kc;
+    const bool active = LISTED ? (i >= c1 && i < c2) : (i < c2 && slot_rebuilt(w.map, go_word, i));
+    if (!__any(active)) continue;  // no centre of this wavefront is rebuilt
+    double4 pi = make_double4(0, 0, 0, 0);
+    int c[3] = {0, 0, 0};
+    float f[3] = {0, 0, 0};
+    if (active) {
+      pi = xq[i];
+      cell_coords(b, pi.x, pi.y, pi.z, c, f);
+    }
+    // ranges q = 2 * (5 (dz+2) + dy+2) + part, lane lg holding q in
+    // [lg*kRangesPerLane, (lg+1)*kRangesPerLane); the empty ones are dropped
+    int start[kRangesPerLane], count[kRangesPerLane];
+    int tot = 0, some = 0;
 #pragma unroll
-  for (int u = 0; u < kRangesPerLane; ++u) {
-    const int q = lg * kRangesPerLane + u;
-    int s = 0, e = 0;
-    if (active && q < 50) {
-      const int r = q >> 1, part = q & 1;
-      int cz = c[2] + r / 5 - 2, cy = c[1] + r % 5 - 2;
-      bool ok = true;
-      if (b.pbc[2]) cz = (cz + b.nc[2]) % b.nc[2];
-      else ok = ok && cz >= 0 && cz < b.nc[2];
-      if (b.pbc[1]) cy = (cy + b.nc[1]) % b.nc[1];
-      else ok = ok && cy >= 0 && cy < b.nc[1];
-      int lo0 = c[0] - 2, hi0 = c[0] + 2, lo1 = 0, hi1 = -1;
-      if (b.pbc[0]) {
-        if (lo0 < 0) {
-          lo1 = lo0 + b.nc[0];
-          hi1 = b.nc[0] - 1;
-          lo0 = 0;
-        } else if (hi0 >= b.nc[0]) {
-          lo1 = 0;
-          hi1 = hi0 - b.nc[0];
-          hi0 = b.nc[0] - 1;
+    for (int u = 0; u < kRangesPerLane; ++u) {
+      const int q = lg * kRangesPerLane + u;
+      int s = 0, e = 0;
+      if (active && q < 50) {
+        const int r = q >> 1, part = q & 1;
+        const int dz = r / 5 - 2, dy = r % 5 - 2;
+        int cz = c[2] + dz, cy = c[1] + dy;
+        bool ok = true;
+        if (b.pbc[2]) cz = (cz + b.nc[2]) % b.nc[2];
+        else ok = ok && cz >= 0 && cz < b.nc[2];
+        if (b.pbc[1]) cy = (cy + b.nc[1]) % b.nc[1];
+        else ok = ok && cy >= 0 && cy < b.nc[1];
+        int lo0 = c[0] - 2, hi0 = c[0] + 2;
+        if constexpr (PLAIN) {
+          // what the row's distance in y and z leaves of the reach in x
+          const float gy = fmaxf(fmaxf(dy - f[1], f[1] - dy - 1.0f) - kTrim, 0.0f) * edge[1];
+          const float gz = fmaxf(fmaxf(dz - f[2], f[2] - dz - 1.0f) - kTrim, 0.0f) * edge[2];
+          const float left = reach2 - gy * gy - gz * gz;
+          ok = ok && left > 0.0f;
+          if (edge[0] > 0.0f) {
+            const float wx = sqrtf(fmaxf(left, 0.0f)) * inv_edge_x + kTrim;
+            lo0 = c[0] + (int)fmaxf(floorf(f[0] - wx), -2.0f);
+            hi0 = c[0] + (int)fminf(floorf(f[0] + wx), 2.0f);
+          }
         }
-      } else {
-        lo0 = max(lo0, 0);
-        hi0 = min(hi0, b.nc[0] - 1);
+        int lo1 = 0, hi1 = -1;
+        if (b.pbc[0]) {
+          if (lo0 < 0) {
+            lo1 = lo0 + b.nc[0];
+            hi1 = b.nc[0] - 1;
+            lo0 = 0;
+          } else if (hi0 >= b.nc[0]) {
+            lo1 = 0;
+            hi1 = hi0 - b.nc[0];
+            hi0 = b.nc[0] - 1;
+          }
+        } else {
+          lo0 = max(lo0, 0);
+          hi0 = min(hi0, b.nc[0] - 1);
+        }
+        const int lo = part ? lo1 : lo0, hi = part ? hi1 : hi0;
+        if (ok && hi >= lo) {
+          const int at = b.nc[0] * (cy + b.nc[1] * cz);
+          s = w.cell_start[at + lo];
+          e = w.cell_start[at + hi + 1];
+        }
       }
-      const int lo = part ? lo1 : lo0, hi = part ? hi1 : hi0;
-      if (ok && hi >= lo) {
-        const int base = b.nc[0] * (cy + b.nc[1] * cz);
-        s = w.cell_start[base + lo];
-        e = w.cell_start[base + hi + 1];
+      start[u] = s;
+      count[u] = e - s;
+      tot += e - s;
+      some += e > s ? 1 : 0;
+    }
+    int off = tot, at = some;
+    auto scan_step = [&](int a, int t) {
+      off += a;
+      at += t;
+    };
+    scan_step(dpp_move<0x111>(off), dpp_move<0x111>(at));  // row_shr 1, 2, 4, 8: zeros come in
+    scan_step(dpp_move<0x112>(off), dpp_move<0x112>(at));
+    scan_step(dpp_move<0x114>(off), dpp_move<0x114>(at));
+    scan_step(dpp_move<0x118>(off), dpp_move<0x118>(at));
+    const int total = __shfl(off, kRowLanes - 1, kRowLanes);
+    if (lg == kRowLanes - 1) rp[at] = total;
+    off -= tot;
+    at -= some;
+#pragma unroll
+    for (int u = 0; u < kRangesPerLane; ++u)
+      if (count[u] > 0) {
+        rs[at] = start[u] - off;
+        rp[at] = off;
+        off += count[u];
+        ++at;
       }
-    }
-    rs[q] = s;
-    len[u] = e - s;
-    tot += e - s;
-  }
-  int incl = tot;
-#pragma unroll
-  for (int d = 1; d < kRowLanes; d <<= 1) {
-    const int v = __shfl_up(incl, d, kRowLanes);
-    if (lg >= d) incl += v;
-  }
-  int off = incl - tot;
-#pragma unroll
-  for (int u = 0; u < kRangesPerLane; ++u) {
-    rp[lg * kRangesPerLane + u] = off;
-    off += len[u];
-  }
-  const int total = __shfl(incl, kRowLanes - 1, kRowLanes);
-  __syncthreads();
-  // k < total lies in range q with rp[q] <= k < rp[q+1] (q < 50, and
-  // rp[50] = total); a lane's k only grows, so q only moves forward
-  int q = 0;
-  auto slot_of = [&](int k) {
-    while (rp[q + 1] <= k) ++q;
-    return rs[q] + (k - rp[q]);
-  };
-  // each step tests candidates k and k + kRowLanes of every lane, whose
-  // loads were issued in the step before
-  constexpr int kStep = 2 * kRowLanes;
-  int jn[2] = {0, 0};
-  double4 pn[2] = {make_double4(0, 0, 0, 0), make_double4(0, 0, 0, 0)};
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int k = lg + h * kRowLanes;
-    if (k < total) {
-      const int sl = slot_of(k);
-      jn[h] = w.cell_atoms[sl];
-      pn[h] = w.xs[sl];
-    }
-  }
-  int found = 0;
-  for (int k0 = 0; __any(k0 < total); k0 += kStep) {
-    int jc[2];
-    double4 pc[2];
+    wave_lds_sync();
+    // k < total lies in range q with rp[q] <= k < rp[q+1] (the last range
+    // ends at total); a lane's k only grows, so q only moves forward
+    int q = 0;
+    auto slot_of = [&](int k) {
+      while (rp[q + 1] <= k) ++q;
+      return rs[q] + k;
+    };
+    // each step tests candidates k and k + kRowLanes of every lane, whose
+    // loads were issued in the step before
+    constexpr int kStep = 2 * kRowLanes;
+    int jn[2] = {0, 0};
+    double4 pn[2] = {make_double4(0, 0, 0, 0), make_double4(0, 0, 0, 0)};
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      jc[h] = jn[h];
-      pc[h] = pn[h];
-      const int k = k0 + kStep + lg + h * kRowLanes;
+      const int k = lg + h * kRowLanes;
       if (k < total) {
         const int sl = slot_of(k);
         jn[h] = w.cell_atoms[sl];
         pn[h] = w.xs[sl];
       }
     }
+    int found = 0;
+    bool wide = false;  // a key of this row needs more than 32 bits
+    for (int k0 = 0; __any(k0 < total); k0 += kStep) {
+      int jc[2];
+      double4 pc[2];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int k = k0 + lg + h * kRowLanes;
-      const int j = jc[h];
-      bool take = false;
-      if (k < total && j != i) {
-        double x = pc[h].x - pi.x, y = pc[h].y - pi.y, z = pc[h].z - pi.z;
-        mic(b, x, y, z);
-        take = dist2(x, y, z) < rv2;
-      }
-      const unsigned gm = (unsigned)(__ballot(take) >> (gw * kRowLanes)) & ((1u << kRowLanes) - 1u);
-      if (take) {
-        const int at = found + __popc(gm & ((1u << lg) - 1u));
-        if (at < w.MV) {
-          row[at] = j;
-          if (gid) key[at] = gid[j];
+      for (int h = 0; h < 2; ++h) {
+        jc[h] = jn[h];
+        pc[h] = pn[h];
+        const int k = k0 + kStep + lg + h * kRowLanes;
+        if (k < total) {
+          const int sl = slot_of(k);
+          jn[h] = w.cell_atoms[sl];
+          pn[h] = w.xs[sl];
         }
       }
-      found += __popc(gm);
-    }
-  }
-  __syncthreads();
-  const int n = min(found, w.MV);
-  if (gid) {
-    for (int k = lg; k < n; k += kRowLanes) {
-      const uint64_t kv = key[k];
-      const int v = row[k];
-      int r = 0;
-      for (int t = 0; t < n; ++t) {
-        const uint64_t kt = key[t];
-        r += (kt < kv || (kt == kv && row[t] < v)) ? 1 : 0;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int k = k0 + lg + h * kRowLanes;
+        const int j = jc[h];
+        double x = pc[h].x - pi.x, y = pc[h].y - pi.y, z = pc[h].z - pi.z;
+        if constexpr (PLAIN) {  // the minimum image as mic() forms it
+          x -= fabs(x) > half[0] ? copysign(len[0], x) : 0.0;
+          y -= fabs(y) > half[1] ? copysign(len[1], y) : 0.0;
+          z -= fabs(z) > half[2] ? copysign(len[2], z) : 0.0;
+        } else {
+          mic(b, x, y, z);
+        }
+        const bool take = k < total && j != i && dist2(x, y, z) < rv2;
+        const unsigned gm = (unsigned)(__ballot(take) >> (gw * kRowLanes)) & ((1u << kRowLanes) - 1u);
+        if (take) {
+          const int to = found + __popc(gm & ((1u << lg) - 1u));
+          if (to < w.MV) {
+            row[to] = j;
+            if constexpr (KEYED) {
+              const uint64_t kj = gid[j];
+              key[to] = kj;
+              wide = wide || (kj >> 32) != 0;
+            }
+          }
+        }
+        found += __popc(gm);
       }
-      sorted[r] = v;
     }
-  } else {
-    // four entries per LDS read (row is 16-byte aligned: MV is a multiple of 4)
-    const int4* row4 = reinterpret_cast<const int4*>(row);
-    const int n4 = n >> 2;
-    for (int k = lg; k < n; k += kRowLanes) {
-      const int v = row[k];
-      int r = 0;
-      for (int t = 0; t < n4; ++t) {
-        const int4 x = row4[t];
-        r += (x.x < v) + (x.y < v) + (x.z < v) + (x.w < v);
-      }
-      for (int t = n4 * 4; t < n; ++t) r += row[t] < v ? 1 : 0;
-      sorted[r] = v;
-    }
-  }
-  __syncthreads();
-  if (active) {
-    for (int k = lg; k < n; k += kRowLanes) w.vl[(size_t)i * w.MV + k] = sorted[k];
-    if (lg == 0) {
+    wave_lds_sync();
+    const int n = min(found, w.MV);
+    int* out = w.vl + (size_t)max(i, 0) * w.MV;
+    if (__any(n > kSortMax) || (KEYED && __any(wide))) write_ranked<KEYED>(row, key, sorted, n, lg, active, out);
+    else if (__any(n > 8 * kRowLanes)) write_sorted<KEYED, 16>(row, key, n, lg, active, out);
+    else if (__any(n > 4 * kRowLanes)) write_sorted<KEYED, 8>(row, key, n, lg, active, out);
+    else write_sorted<KEYED, 4>(row, key, n, lg, active, out);
+    if (active && lg == 0) {
       w.vn[i] = found;
       if (found > w.MV) atomicMax(&w.flags[kFlagVerletOverflow], found);
     }
-  }
-  __syncthreads();  // the next pass reuses the LDS
+    wave_lds_sync();  // the next pass reuses the LDS
   }
 }
 
@@ -737,8 +914,14 @@ hipError_t launch_rebuild(const DevBox& b, int N, int c1, int c2, double rv2, co
       nr = std::min(nr, kListBlocks);
     }
     const size_t lds = build_lds_per_centre(w.MV, keyed) * groups;
-    if (listed) k_verlet_build<true><<<nb, groups * kRowLanes, lds, s>>>(go, b, c1, c2, groups, w.xq, rv2, gid, w);
-    else k_verlet_build<false><<<nb, groups * kRowLanes, lds, s>>>(go, b, c1, c2, groups, w.xq, rv2, gid, w);
+    const bool plain = b.ortho && b.h[0] > 0.0 && b.h[4] > 0.0 && b.h[8] > 0.0;
+    const auto pick = [](auto keyed, bool listed, bool plain) {
+      constexpr bool K = decltype(keyed)::value;
+      return listed ? (plain ? k_verlet_build<true, K, true> : k_verlet_build<true, K, false>)
+                    : (plain ? k_verlet_build<false, K, true> : k_verlet_build<false, K, false>);
+    };
+    const auto build = keyed ? pick(std::true_type{}, listed, plain) : pick(std::false_type{}, listed, plain);
+    build<<<nb, groups * kRowLanes, lds, s>>>(go, b, c1, c2, groups, w.xq, rv2, gid, w);
     k_verlet_reverse<<<nr, 256, 0, s>>>(go, c1, c2, gid, w);
   }
   // the request marks of this rebuild are spent

@@ -248,6 +248,16 @@ __device__ __forceinline__ double dpp_move(double v)
   return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true),
                           __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true));
 }
+template <int CTRL>
+__device__ __forceinline__ int dpp_move(int v)
+{
+  return __builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ uint64_t dpp_move(uint64_t v)
+{
+  return (uint64_t)(uint32_t)dpp_move<CTRL>((int)(v >> 32)) << 32 | (uint32_t)dpp_move<CTRL>((int)v);
+}
 template <int P, class V>
 __device__ __forceinline__ V group_sum(V v)
 {
@@ -272,13 +282,6 @@ __device__ __forceinline__ void wave_lds_sync()
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// the value of lane L of the quad
-template <int L>
-__device__ __forceinline__ int quad_lane(int v)
-{
-  return __builtin_amdgcn_mov_dpp(v, L * 0x55, 0xf, 0xf, true);
 }
 
 }  // namespace dmgx
