@@ -349,7 +349,6 @@ void NepEngine::free_all()
   dfree(&w_.nac);
   dfree(&w_.cell_count);
   dfree(&w_.cell_start);
-  dfree(&w_.cell_tiles);
   w_.cap = w_.rcap = 0;
   w_.ncell_cap = 0;
   have_list_ = false;
@@ -467,8 +466,7 @@ void NepEngine::ensure_cells(int ncell)
 {
   if (ncell <= w_.ncell_cap) return;
   dalloc(&w_.cell_count, (size_t)ncell, "cell counts");
-  dalloc(&w_.cell_start, (size_t)ncell + 1, "cell starts");
-  dalloc(&w_.cell_tiles, 2 * ((size_t)ncell / 4096 + 2) + 8, "cell scan tiles");
+  dalloc(&w_.cell_start, cell_start_entries(ncell), "cell starts");
   check(hipMemset(w_.cell_count, 0, sizeof(int) * ncell), "clear cell counts");
   w_.ncell_cap = ncell;
 }
@@ -621,7 +619,7 @@ void NepEngine::launch_key(std::vector<long long>& k) const
     k.push_back(v);
   for (const void* q : {(const void*)w.xq, (const void*)w.cell_of, (const void*)w.cell_rank,
                         (const void*)w.cell_count, (const void*)w.cell_start, (const void*)w.cell_atoms,
-                        (const void*)w.xs, (const void*)w.cell_tiles, (const void*)w.vn, (const void*)w.vl,
+                        (const void*)w.xs, (const void*)w.vn, (const void*)w.vl,
                         (const void*)w.vrev, (const void*)w.x0, (const void*)w.nr, (const void*)w.na,
                         (const void*)w.edge, (const void*)w.eq, (const void*)w.vsa, (const void*)w.amask,
                         (const void*)w.bR,
@@ -1075,8 +1073,7 @@ DevWork carve_work(char* base, int cap, int mv, long long ncell, int T, int kRp,
   const size_t n = (size_t)cap, rows = n * (size_t)mv, tiles = row_entries(n, mv);
   w.flags = c.take<int>(kNumFlags);
   w.cell_count = c.take<int>((size_t)ncell);
-  w.cell_start = c.take<int>((size_t)ncell + 1);
-  w.cell_tiles = c.take<int>(2 * ((size_t)ncell / 4096 + 2) + 8);
+  w.cell_start = c.take<int>(cell_start_entries(ncell));
   w.xq = c.take<double4>(n);
   w.xs = c.take<double4>(n);
   w.cell_of = c.take<int>(n);

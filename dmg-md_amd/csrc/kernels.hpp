@@ -113,6 +113,9 @@ static_assert(sizeof(float3) == 12, "angular partials are packed");
 __host__ __device__ inline size_t row_begin(int i, int M) { return (size_t)(i >> 6) * M * kTile + (i & 63); }
 // entries of an interleaved row array for rc centres
 inline size_t row_entries(size_t rc, int M) { return (rc + kTile - 1) / kTile * kTile * (size_t)M; }
+// starts of ncell cells: an end for each tile of the scan (at most one per 2,048
+// cells and one more), and the scan's cursor
+inline size_t cell_start_entries(long long ncell) { return (size_t)ncell + 1 + 2 * ((size_t)ncell / 4096 + 2) + 8; }
 // (Every field is part of NepEngine::launch_key: a captured launch takes
 // the struct by value.)
 struct DevWork {
@@ -124,10 +127,9 @@ struct DevWork {
   int* cell_of = nullptr;      // [cap]
   int* cell_rank = nullptr;    // [cap] rank of the atom inside its cell
   int* cell_count = nullptr;   // [ncell] zero between rebuilds
-  int* cell_start = nullptr;   // [ncell+1]
+  int* cell_start = nullptr;   // [cell_start_entries(ncell)] the starts, an end per tile of the scan, its cursor
   int* cell_atoms = nullptr;   // [cap]
   double4* xs = nullptr;       // [cap] xq in cell_atoms order (rebuild only)
-  int* cell_tiles = nullptr;   // [2 (ncell/4096 + 2) + 8] tile sums, then (16-byte aligned) offsets, of the multi-block scan
   int* vn = nullptr;           // [cap] Verlet row length
   int* vl = nullptr;           // [cap*MV] Verlet rows
   short* vrev = nullptr;       // [cap*MV] position of the centre in the neighbour's row (rows hold

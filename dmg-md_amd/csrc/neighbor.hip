@@ -25,7 +25,7 @@ namespace dmgx {
 namespace {
 
 constexpr int kRowLanes = 16;  // lanes cooperating on one Verlet row
-constexpr int kScanOneBlock = 262144;  // larger cell grids are scanned by many workgroups
+constexpr int kScanCells = 4096;  // cells per workgroup of the scan (one row of cells at least)
 
 __global__ void k_set_flag(int* __restrict__ flag, int value) { *flag = value; }
 
@@ -79,12 +79,13 @@ __global__ __launch_bounds__(kBlock) void k_pack(DevBox b, int N, int T, const d
 // listed slots enter the cell list: every row it makes holds slots of its
 // own request only.
 __global__ void k_cell_count(const int* __restrict__ go, DevBox b, int N, const double4* __restrict__ xq,
-                             int* __restrict__ cell_of, int* __restrict__ rank, int* __restrict__ count,
-                             double* __restrict__ x0, int a1, int b1, int a2, int b2, int* __restrict__ flags,
-                             ImageMap m)
+                             int row_shift, int* __restrict__ cell_of, int* __restrict__ rank,
+                             int* __restrict__ count, int* __restrict__ cursor, double* __restrict__ x0, int a1, int b1,
+                             int a2, int b2, int* __restrict__ flags, ImageMap m)
 {
   const int g = *go;
   if (!g) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *cursor = 0;
   const bool listed = rebuild_listed(m);
   const int n = listed ? m.req_off[2 * m.n_req + 1] : N;
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
@@ -92,8 +93,8 @@ __global__ void k_cell_count(const int* __restrict__ go, DevBox b, int N, const 
     const double4 p = xq[i];
     int c[3];
     if (!cell_coords(b, p.x, p.y, p.z, c)) atomicOr(&flags[kFlagOutOfBox], 1);
-    const int id = c[0] + b.nc[0] * (c[1] + b.nc[1] * c[2]);
-    cell_of[i] = id;
+    const int row = c[1] + b.nc[1] * c[2], id = c[0] + b.nc[0] * row;
+    cell_of[i] = id + (row >> row_shift);  // where the scan keeps the cell's start
     rank[i] = atomicAdd(&count[id], 1);
     if (((i >= a1 && i < b1) || (i >= a2 && i < b2)) && (listed || slot_rebuilt(m, g, i))) {
       x0[i] = p.x;
@@ -103,107 +104,121 @@ __global__ void k_cell_count(const int* __restrict__ go, DevBox b, int N, const 
   }
 }
 
-// Exclusive scan of the cell counts by one workgroup, which also clears the
-// counts for the next rebuild; start[ncell] = total.  Each pass covers 4
-// sub-tiles of 4096 cells, 4 consecutive cells per thread in each (one
-// 16-byte access per thread, contiguous across the wavefront), scanned
-// together; the next pass's counts are loaded before this pass is scanned.
-__global__ __launch_bounds__(1024) void k_scan_cells(const int* __restrict__ go, int ncell,
-                                                     int* __restrict__ count, int* __restrict__ start)
+// Starts of the cells in cell_atoms.  A range of candidates runs along one row
+// of cells, so only the cells of a row need consecutive atoms: each workgroup
+// scans 2^row_shift whole rows (tile_cells cells) by itself, takes its place
+// in cell_atoms from the cursor, and clears the counts for the next rebuild.
+// A tile's starts are followed by its end: cell c of row r has its start at
+// c + (r >> row_shift), and the next entry is the cell's end.  Bound by its
+// own latency: 213,000 cells 49 -> 6.1 us against passes of one workgroup.
+__global__ __launch_bounds__(1024) void k_cell_starts(const int* __restrict__ go, int ncell, int tile_cells,
+                                                      int* __restrict__ count, int* __restrict__ start,
+                                                      int* __restrict__ cursor)
 {
   if (!*go) return;
-  constexpr int kSub = 4096, kChunks = 4, kTile = kSub * kChunks;
-  __shared__ int wsum[kChunks][16];
+  __shared__ int wsum[2][16];
+  __shared__ int place;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  auto load = [&](int base, int4* v) {
+  const int n = min(tile_cells, ncell - (int)blockIdx.x * tile_cells);
+  int* in = count + (size_t)blockIdx.x * tile_cells;
+  int* out = start + (size_t)blockIdx.x * (tile_cells + 1);
+  int v[4], sum = 0;
+  auto load = [&](int base) {
+    sum = 0;
 #pragma unroll
-    for (int c = 0; c < kChunks; ++c) {
-      const int k = base + c * kSub + threadIdx.x * 4;
-      if (k + 3 < ncell) {
-        v[c] = *reinterpret_cast<const int4*>(count + k);
-      } else {
-        v[c].x = k < ncell ? count[k] : 0;
-        v[c].y = k + 1 < ncell ? count[k + 1] : 0;
-        v[c].z = k + 2 < ncell ? count[k + 2] : 0;
-        v[c].w = 0;
-      }
+    for (int q = 0; q < 4; ++q) {
+      const int k = base + 4 * threadIdx.x + q;
+      v[q] = k < n ? in[k] : 0;
+      sum += v[q];
     }
   };
-  int4 v[kChunks], nv[kChunks];
-  load(0, v);
-  int carry = 0;
-  for (int base = 0; base < ncell; base += kTile) {
-    if (base + kTile < ncell) load(base + kTile, nv);
-    int s[kChunks], x[kChunks];
-#pragma unroll
-    for (int c = 0; c < kChunks; ++c) {
-      s[c] = v[c].x + v[c].y + v[c].z + v[c].w;
-      x[c] = s[c];
-    }
+  // sum before this thread, and of the workgroup
+  int flip = 0;
+  auto scan = [&](int* total) {
+    int x = sum;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
-#pragma unroll
-      for (int c = 0; c < kChunks; ++c) {
-        const int y = __shfl_up(x[c], off, 64);
-        if (lane >= off) x[c] += y;
-      }
+      const int y = __shfl_up(x, off, 64);
+      if (lane >= off) x += y;
     }
-    if (lane == 63) {
-#pragma unroll
-      for (int c = 0; c < kChunks; ++c) wsum[c][wave] = x[c];
-    }
+    flip ^= 1;
+    if (lane == 63) wsum[flip][wave] = x;
     __syncthreads();
-    int run_base = carry;
-#pragma unroll
-    for (int c = 0; c < kChunks; ++c) {
-      int before = 0, total = 0;
-      for (int q = 0; q < 16; ++q) {
-        const int t = wsum[c][q];
-        if (q < wave) before += t;
-        total += t;
-      }
-      const int k = base + c * kSub + threadIdx.x * 4;
-      int4 o;
-      o.x = run_base + before + x[c] - s[c];
-      o.y = o.x + v[c].x;
-      o.z = o.y + v[c].y;
-      o.w = o.z + v[c].z;
-      if (k + 3 < ncell) {
-        *reinterpret_cast<int4*>(start + k) = o;
-        *reinterpret_cast<int4*>(count + k) = make_int4(0, 0, 0, 0);
-      } else {
-        if (k < ncell) start[k] = o.x, count[k] = 0;
-        if (k + 1 < ncell) start[k + 1] = o.y, count[k + 1] = 0;
-        if (k + 2 < ncell) start[k + 2] = o.z, count[k + 2] = 0;
-      }
-      run_base += total;
+    int before = x - sum;
+    *total = 0;
+    for (int q = 0; q < 16; ++q) {
+      if (q < wave) before += wsum[flip][q];
+      *total += wsum[flip][q];
     }
-    carry = run_base;
-#pragma unroll
-    for (int c = 0; c < kChunks; ++c) v[c] = nv[c];
-    __syncthreads();
+    return before;
+  };
+  int all = 0, before = 0;
+  for (int base = 0; base < n; base += kScanCells) {
+    load(base);
+    int t;
+    before = scan(&t);
+    all += t;
   }
-  if (threadIdx.x == 0) start[ncell] = carry;
+  if (threadIdx.x == 0) place = atomicAdd(cursor, all);
+  __syncthreads();
+  int run = place;
+  for (int base = 0; base < n; base += kScanCells) {
+    if (n > kScanCells) {  // a row longer than the tile: its counts again
+      int t;
+      load(base);
+      before = scan(&t);
+      before += run;
+      run += t;
+    } else {
+      before += run;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int k = base + 4 * threadIdx.x + q;
+      if (k < n) {
+        out[k] = before;
+        in[k] = 0;
+      }
+      before += v[q];
+    }
+  }
+  if (threadIdx.x == 0) out[n] = place + all;
 }
 
-// Multi-block form of the same scan for large grids: each workgroup scans
-// one tile of 4096 cells (and clears its counts) and stores the tile total;
-// k_scan_cells then scans the tile totals into offsets and k_scan_offsets
-// adds each tile's offset.
-__global__ __launch_bounds__(1024) void k_scan_tiles(const int* __restrict__ go, int ncell, int* __restrict__ count,
-                                                     int* __restrict__ start, int* __restrict__ tile_sum)
+// Count, scan and fill of a small system by one workgroup, with the cells in
+// LDS: one launch instead of three, in a rebuild and in every step without
+// one.  Bound by what one CU loads and stores (2.4 us per 1,000 atoms).
+constexpr int kOneBlockIdBits = 14;
+__global__ __launch_bounds__(1024) void k_cells_one_block(const int* __restrict__ go, DevBox b, int N, int ncell,
+                                                          const double4* __restrict__ xq, int* __restrict__ cell_of,
+                                                          int* __restrict__ start, double* __restrict__ x0, int a1,
+                                                          int b1, int a2, int b2, int* __restrict__ flags,
+                                                          int* __restrict__ atoms, double4* __restrict__ xs, ImageMap m)
 {
-  if (!*go) return;
+  const int g = *go;
+  if (!g) return;
+  extern __shared__ int cells[];
   __shared__ int wsum[16];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int k0 = blockIdx.x * 4096 + threadIdx.x * 4;
-  int v[4], s = 0;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    v[k] = k0 + k < ncell ? count[k0 + k] : 0;
-    s += v[k];
+  for (int k = threadIdx.x; k < ncell; k += 1024) cells[k] = 0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < N; i += 1024) {
+    const double4 p = xq[i];
+    int c[3];
+    if (!cell_coords(b, p.x, p.y, p.z, c)) atomicOr(&flags[kFlagOutOfBox], 1);
+    const int id = c[0] + b.nc[0] * (c[1] + b.nc[1] * c[2]);
+    cell_of[i] = id | atomicAdd(&cells[id], 1) << kOneBlockIdBits;
+    if (((i >= a1 && i < b1) || (i >= a2 && i < b2)) && slot_rebuilt(m, g, i)) {
+      x0[i] = p.x;
+      x0[N + i] = p.y;
+      x0[2 * N + i] = p.z;
+    }
   }
-  int x = s;
+  __syncthreads();
+  const int per = (ncell + 1023) >> 10, c0 = min((int)threadIdx.x * per, ncell), c1 = min(c0 + per, ncell);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int sum = 0;
+  for (int k = c0; k < c1; ++k) sum += cells[k];
+  int x = sum;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
     const int y = __shfl_up(x, off, 64);
@@ -211,30 +226,22 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(const int* __restrict__ go,
   }
   if (lane == 63) wsum[wave] = x;
   __syncthreads();
-  int before = 0, total = 0;
-  for (int q = 0; q < 16; ++q) {
-    if (q < wave) before += wsum[q];
-    total += wsum[q];
+  int run = x - sum;
+  for (int q = 0; q < wave; ++q) run += wsum[q];
+  for (int k = c0; k < c1; ++k) {
+    const int v = cells[k];
+    cells[k] = run;
+    start[k] = run;
+    run += v;
   }
-  int run = before + x - s;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (k0 + k < ncell) {
-      start[k0 + k] = run;
-      count[k0 + k] = 0;
-    }
-    run += v[k];
+  if (threadIdx.x == 0) start[ncell] = N;
+  __syncthreads();
+  for (int i = threadIdx.x; i < N; i += 1024) {
+    const int w = cell_of[i];
+    const int at = cells[w & ((1 << kOneBlockIdBits) - 1)] + (w >> kOneBlockIdBits);
+    atoms[at] = i;
+    xs[at] = xq[i];
   }
-  if (threadIdx.x == 0) tile_sum[blockIdx.x] = total;
-}
-
-__global__ void k_scan_offsets(const int* __restrict__ go, int ncell, const int* __restrict__ tile_off,
-                               int* __restrict__ start)
-{
-  if (!*go) return;
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < ncell) start[k] += tile_off[k / 4096];
-  if (k == 0) start[ncell] = tile_off[(ncell + 4095) / 4096];
 }
 
 __global__ void k_cell_fill(const int* __restrict__ go, int N, const int* __restrict__ cell_of,
@@ -517,8 +524,8 @@ __device__ __forceinline__ void write_ranked(const int* row, const uint64_t* key
 // (five: 335, 124 and 1,480 us; six: 389, 199 and 1,950).
 template <bool LISTED, bool KEYED, bool PLAIN>
 __global__ __launch_bounds__(256, 4) void k_verlet_build(const int* __restrict__ go, DevBox b, int c1, int c2,
-                                                      int groups, const double4* __restrict__ xq, double rv2,
-                                                      const uint64_t* __restrict__ gid, DevWork w)
+                                                      int groups, int row_shift, const double4* __restrict__ xq,
+                                                      double rv2, const uint64_t* __restrict__ gid, DevWork w)
 {
   const int go_word = *go;
   if (!go_word) return;
@@ -610,7 +617,7 @@ __global__ __launch_bounds__(256, 4) void k_verlet_build(const int* __restrict__
         }
         const int lo = part ? lo1 : lo0, hi = part ? hi1 : hi0;
         if (ok && hi >= lo) {
-          const int at = b.nc[0] * (cy + b.nc[1] * cz);
+          const int row = cy + b.nc[1] * cz, at = b.nc[0] * row + (row >> row_shift);
           s = w.cell_start[at + lo];
           e = w.cell_start[at + hi + 1];
         }
@@ -832,6 +839,13 @@ inline int nblk(int n) { return (n + kBlock - 1) / kBlock; }
 // launch that finds no rebuild asked returns in about a microsecond
 constexpr int kListBlocks = 2048;
 
+// Systems up to kOneBlockAtoms atoms and kOneBlockCells cells (60 KiB of LDS)
+// have their cells made by one workgroup: 4,096 atoms 11.9 us against 10.6 in
+// three launches and the 4 us between them, 5,832 18 us, 11,000 29 us against
+// 13; and a step without a rebuild is two launches (7 us) shorter, 82 -> 74 us
+// a step of 4,096 carbon atoms.
+constexpr int kOneBlockAtoms = 6144, kOneBlockCells = 15 * 1024;
+
 // LDS of one centre of the build: its row buffers and candidate ranges
 size_t build_lds_per_centre(int mv, bool keyed) { return build_row_lds(mv, keyed) + kRangeLds; }
 
@@ -886,22 +900,22 @@ hipError_t launch_rebuild(const DevBox& b, int N, int c1, int c2, double rv2, co
   }
   const bool cap = capped || listed;
   const int slot_blocks = cap ? std::min(nblk(N), kListBlocks) : nblk(N);
-  if (N > 0)
-    k_cell_count<<<slot_blocks, kBlock, 0, s>>>(go, b, N, w.xq, w.cell_of, w.cell_rank, w.cell_count, w.x0, r[0],
-                                                r[1], r[2], r[3], w.flags, w.map);
-  if (ncell <= kScanOneBlock) {
-    k_scan_cells<<<1, 1024, 0, s>>>(go, ncell, w.cell_count, w.cell_start);
-  } else {
-    const int tiles = (ncell + 4095) / 4096;
-    int* tile_sum = w.cell_tiles;
-    int* tile_off = w.cell_tiles + ((tiles + 4) & ~3);  // 16-byte aligned for the scan's vector stores
-    k_scan_tiles<<<tiles, 1024, 0, s>>>(go, ncell, w.cell_count, w.cell_start, tile_sum);
-    k_scan_cells<<<1, 1024, 0, s>>>(go, tiles, tile_sum, tile_off);
-    k_scan_offsets<<<nblk(ncell), kBlock, 0, s>>>(go, ncell, tile_off, w.cell_start);
-  }
-  if (N > 0)
+  // the cells of small systems by one workgroup, whose LDS holds them
+  int row_shift = 31;
+  if (!listed && N > 0 && N <= kOneBlockAtoms && ncell <= kOneBlockCells) {
+    k_cells_one_block<<<1, 1024, ncell * sizeof(int), s>>>(go, b, N, ncell, w.xq, w.cell_of, w.cell_start, w.x0, r[0],
+                                                           r[1], r[2], r[3], w.flags, w.cell_atoms, w.xs, w.map);
+  } else if (N > 0) {
+    row_shift = 0;
+    while (((long long)b.nc[0] << (row_shift + 1)) <= kScanCells) ++row_shift;
+    const int rows = b.nc[1] * b.nc[2], tiles = (int)(((long long)rows + (1LL << row_shift) - 1) >> row_shift);
+    int* cursor = w.cell_start + (size_t)ncell + tiles;
+    k_cell_count<<<slot_blocks, kBlock, 0, s>>>(go, b, N, w.xq, row_shift, w.cell_of, w.cell_rank, w.cell_count, cursor,
+                                                w.x0, r[0], r[1], r[2], r[3], w.flags, w.map);
+    k_cell_starts<<<tiles, 1024, 0, s>>>(go, ncell, b.nc[0] << row_shift, w.cell_count, w.cell_start, cursor);
     k_cell_fill<<<slot_blocks, kBlock, 0, s>>>(go, N, w.cell_of, w.cell_rank, w.cell_start, w.xq, w.cell_atoms, w.xs,
                                                w.map);
+  }
   if (c2 > c1) {
     const bool keyed = gid != nullptr;
     const int groups = build_groups(w.MV, keyed);
@@ -921,7 +935,7 @@ hipError_t launch_rebuild(const DevBox& b, int N, int c1, int c2, double rv2, co
                     : (plain ? k_verlet_build<false, K, true> : k_verlet_build<false, K, false>);
     };
     const auto build = keyed ? pick(std::true_type{}, listed, plain) : pick(std::false_type{}, listed, plain);
-    build<<<nb, groups * kRowLanes, lds, s>>>(go, b, c1, c2, groups, w.xq, rv2, gid, w);
+    build<<<nb, groups * kRowLanes, lds, s>>>(go, b, c1, c2, groups, row_shift, w.xq, rv2, gid, w);
     k_verlet_reverse<<<nr, 256, 0, s>>>(go, c1, c2, gid, w);
   }
   // the request marks of this rebuild are spent

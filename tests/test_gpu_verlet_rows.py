@@ -1,8 +1,9 @@
 """Verlet rows as the device stores them, against brute force: row lengths on
 both sides of each register sort (64, 128 and 256 entries) and beyond it, boxes
 of five cells and more per direction, open and mixed directions, a skewed box,
-atoms a little outside their periodic box, and rows ordered by global ids that
-fit 32 bits, that do not, and that repeat."""
+atoms a little outside their periodic box, rows ordered by global ids that
+fit 32 bits, that do not, and that repeat, and the cell grids of each way the
+cells are made."""
 import os
 
 import numpy as np
@@ -60,3 +61,29 @@ def test_rows_match_brute_force(dmgx, name, density, ids):
         if gid is not None:
             want = want[np.lexsort((want, gid[want]))]
         assert np.array_equal(rows[i], want), (i, len(rows[i]), len(want))
+
+
+def _elongated(n, edges, seed):
+    rng = np.random.default_rng(seed)
+    return np.ascontiguousarray(rng.uniform(0.02, 0.98, (n, 3)).T * np.asarray(edges)[:, None])
+
+
+# (atoms, box, directions): either side of the size up to which one workgroup
+# makes the cells, more cells than its LDS holds, several tiles of the scan
+# with a rest, rows of cells longer than a tile, and rows of a single cell
+CELLS = [(1, (40.0, 40.0, 40.0), (0, 0, 0)), (6144, (38.0, 38.0, 38.0), (1, 1, 1)),
+         (6145, (38.0, 38.0, 38.0), (1, 1, 1)), (3000, (80.0, 90.0, 70.0), (1, 0, 1)),
+         (4000, (110.0, 30.0, 141.0), (0, 1, 0)), (7000, (61.0, 59.0, 83.0), (1, 1, 1)),
+         (6500, (23000.0, 14.0, 14.0), (0, 0, 0)), (6500, (5.0, 60.0, 61.0), (0, 1, 1))]
+
+
+@pytest.mark.parametrize("n,edges,pbc", CELLS)
+def test_rows_over_cell_grids(dmgx, n, edges, pbc):
+    nep = dmgx.NEP(os.path.join(POTENTIALS, "nep_carbon.txt"))
+    h, pos = np.diag(edges), _elongated(n, edges, n)
+    for _ in range(2):  # the second rebuild starts from the counts the first one left
+        gpu_compute(dmgx, nep, dmgx.Box(h, pbc), np.zeros(n, np.int32), pos, force_rebuild=True)
+        rows = nep.verlet_rows(0, n)
+    ref = neighbor_rows(h, pbc, pos, nep.info.rc_radial_max + 1.0, max_nb=1024)
+    for i in range(n):
+        assert np.array_equal(rows[i], np.sort(np.asarray(ref[i]))), i
