@@ -1566,16 +1566,18 @@ void MdState::checkpoint(bool save)
   struct {
     double* live;
     double** copy;
-    size_t n;
-  } buf[6] = {{pos_, &ck_pos_, 3}, {vel_, &ck_vel_, 3}, {force_, &ck_force_, 3}, {pe_, &ck_pe_, 1},
-              {vir_, &ck_vir_, 9}, {unwrapped_, &ck_unwrapped_, 3}};
-  for (auto& e : buf) {
-    if (!e.live) continue;
-    const size_t bytes = e.n * (size_t)N_ * sizeof(double);
-    if (!*e.copy) dalloc(e.copy, e.n * (size_t)N_, "checkpoint");
-    if (save) check(hipMemcpyAsync(*e.copy, e.live, bytes, hipMemcpyDeviceToDevice, stream_), "checkpoint");
-    else check(hipMemcpyAsync(e.live, *e.copy, bytes, hipMemcpyDeviceToDevice, stream_), "restore");
+    int n;
+  } buf[kMaxCopies] = {{pos_, &ck_pos_, 3}, {vel_, &ck_vel_, 3}, {force_, &ck_force_, 3}, {pe_, &ck_pe_, 1},
+                       {vir_, &ck_vir_, 9}, {unwrapped_, &ck_unwrapped_, 3}};
+  ArrayCopies c{};
+  for (int a = 0; a < kMaxCopies; ++a) {
+    if (!buf[a].live) continue;
+    c.n[a] = (long long)buf[a].n * N_;
+    if (!*buf[a].copy) dalloc(buf[a].copy, (size_t)c.n[a], "checkpoint");
+    c.to[a] = save ? *buf[a].copy : buf[a].live;
+    c.from[a] = save ? buf[a].live : *buf[a].copy;
   }
+  check(launch_copy_arrays(c, stream_), save ? "checkpoint" : "restore");
 }
 
 void MdState::run(int steps, double dt_fs, const EnsembleConfig& ens, unsigned flags, double* thermo_out, int every,
@@ -1699,7 +1701,12 @@ void MdState::run(int steps, double dt_fs, const EnsembleConfig& ens, unsigned f
     checkpoint(true);
     bool redo = false;
     for (int attempt = 0; attempt < 4; ++attempt) {
-      if (kind != 0) {
+      // a barostat step takes its draws and target as launch arguments
+      double draws[2] = {0.0, 0.0}, target = 0.0;
+      if (kind != 0 && baro) {
+        if (kind == 2) ctl.draw_bdp(&draws[0], &draws[1]);
+        target = ctl.target_temperature(c0, steps);
+      } else if (kind != 0) {
         // the staging buffer is free: every chunk (and every attempt) ends
         // with the status read's synchronisation, after its upload
         for (int k = 0; k < n; ++k) {
@@ -1715,7 +1722,7 @@ void MdState::run(int steps, double dt_fs, const EnsembleConfig& ens, unsigned f
       // displacement test), force, fused second half (+ thermo partials),
       // and the thermo reduction that also forms the next factor
       const double volume = box_volume(box_.h);
-      double* const fac = kind != 0 ? factor_ : nullptr;
+      double* const fac = kind != 0 && !baro ? factor_ : nullptr;  // a barostat step leaves none pending
       if (graphs && n > 0) {
         const NepEngine::Plan plan =
             nep_->plan(box_, N_, 0, N_, 0, N_, type_, pos_, nullptr, pe_, force_, vir_, flags & ~1u);
@@ -1740,18 +1747,18 @@ void MdState::run(int steps, double dt_fs, const EnsembleConfig& ens, unsigned f
         p.end(stream_);
         if (thermo_on) {
           p.begin(kProfThermo, stream_);
-          check(launch_thermo_final(N_, volume, kind, coupling, 0.0, rand_, factor_, tw_, stream_, targets,
-                                    kind != 0 ? kstep_ : nullptr),
+          // a barostat step's thermo (before the thermostat rescale) is read
+          // by the host after the status words' synchronisation
+          check(baro ? launch_thermo_final(N_, volume, kind, coupling, target, nullptr, factor_, tw_, stream_, nullptr,
+                                           nullptr, draws, hth)
+                     : launch_thermo_final(N_, volume, kind, coupling, 0.0, rand_, factor_, tw_, stream_, targets,
+                                           kind != 0 ? kstep_ : nullptr),
                 "thermostat");
           p.end(stream_);
         }
       }
       const bool pending = kind != 0 && n > 0;
       if (pending) check(launch_scale_by(3 * N_, factor_, vel_, stream_), "thermostat scale");
-      // a barostat step's thermo (before the thermostat rescale) comes back
-      // with the status words, in the same synchronisation
-      if (baro)
-        check(hipMemcpyAsync(hth, tw_.thermo, 8 * sizeof(double), hipMemcpyDeviceToHost, stream_), "thermo copy");
       redo = nep_->settle(stream_);
       if (!redo) break;
       checkpoint(false);

@@ -871,6 +871,8 @@ __global__ __launch_bounds__(kThermoThreads) void k_md_second(int N, double dt, 
 // With step_index, the step's target temperature and draws are
 // targets[k] and rand2[2k .. 2k+1] for k = *step_index, which the kernel then
 // advances: the same launch serves every step of a chunk (a replayed graph).
+// Without rand2 the draws are d0 and d1.  With report (pinned host memory)
+// the thermo goes there too: a step that the host waits for needs no copy.
 __global__ __launch_bounds__(kThermoThreads) void k_thermo_final(int nb, int N, double volume,
                                                                  const double* __restrict__ partial,
                                                                  double* __restrict__ thermo, int kind,
@@ -878,7 +880,8 @@ __global__ __launch_bounds__(kThermoThreads) void k_thermo_final(int nb, int N, 
                                                                  const double* __restrict__ rand2,
                                                                  double* __restrict__ factor,
                                                                  const double* __restrict__ targets,
-                                                                 int* __restrict__ step_index)
+                                                                 int* __restrict__ step_index, double d0, double d1,
+                                                                 double* __restrict__ report)
 {
   KSum acc[8];
 #pragma unroll
@@ -894,13 +897,15 @@ __global__ __launch_bounds__(kThermoThreads) void k_thermo_final(int nb, int N, 
       rand2 += 2 * k;
       *step_index = k + 1;
     }
+    const double draws[2] = {d0, d1};
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
       double v = acc[q].s + acc[q].c;
       if (q == 0) v /= 3.0 * N * 8.617343e-5;
       else if (q >= 2) v /= volume;
       thermo[q] = v;
-      if (q == 0 && factor) factor[0] = ensemble_factor(kind, N, coupling, t_target, rand2, v);
+      if (report) report[q] = v;
+      if (q == 0 && factor) factor[0] = ensemble_factor(kind, N, coupling, t_target, rand2 ? rand2 : draws, v);
     }
   }
 }
@@ -909,6 +914,21 @@ __global__ void k_chunk_start(double* __restrict__ factor, int* __restrict__ ste
 {
   factor[0] = 1.0;
   *step_index = 0;
+}
+
+// Several arrays copied by one launch (a chunk's checkpoint; up to six copies
+// of a few microseconds each otherwise).  Bound by memory: 19 doubles an atom
+// read and written.
+__global__ __launch_bounds__(kBlock) void k_copy_arrays(ArrayCopies c)
+{
+  const long long t = blockIdx.x * (long long)kBlock + threadIdx.x, stride = (long long)gridDim.x * kBlock;
+#pragma unroll
+  for (int a = 0; a < kMaxCopies; ++a) {
+    const long long pairs = c.n[a] >> 1;
+    for (long long k = t; k < pairs; k += stride)
+      reinterpret_cast<double2*>(c.to[a])[k] = reinterpret_cast<const double2*>(c.from[a])[k];
+    if (t == 0 && (c.n[a] & 1)) c.to[a][c.n[a] - 1] = c.from[a][c.n[a] - 1];
+  }
 }
 
 __global__ void k_ensemble_factor(int kind, int N, double coupling, double t_target,
@@ -1043,7 +1063,7 @@ hipError_t launch_thermo(int N, double volume, const double* mass, const double*
   const int nb = thermo_blocks(N);
   k_thermo_partial<<<nb, kThermoThreads, 0, s>>>(N, mass, pe, vel, virial, w.partial);
   k_thermo_final<<<1, kThermoThreads, 0, s>>>(nb, N, volume, w.partial, w.thermo, 0, 0.0, 0.0, nullptr, nullptr,
-                                              nullptr, nullptr);
+                                              nullptr, nullptr, 0.0, 0.0, nullptr);
   return hipGetLastError();
 }
 
@@ -1086,10 +1106,19 @@ hipError_t launch_md_second(int N, double dt, const double* mass, double* vel, c
 
 hipError_t launch_thermo_final(int N, double volume, int kind, double coupling, double t_target,
                                const double* rand2, double* factor, DevWork& tw, hipStream_t s,
-                               const double* targets, int* step_index)
+                               const double* targets, int* step_index, const double* draws, double* report)
 {
   k_thermo_final<<<1, kThermoThreads, 0, s>>>(thermo_blocks(N), N, volume, tw.partial, tw.thermo, kind, coupling,
-                                                t_target, rand2, kind ? factor : nullptr, targets, step_index);
+                                              t_target, rand2, kind ? factor : nullptr, targets, step_index,
+                                              draws ? draws[0] : 0.0, draws ? draws[1] : 0.0, report);
+  return hipGetLastError();
+}
+
+hipError_t launch_copy_arrays(const ArrayCopies& c, hipStream_t s)
+{
+  long long most = 0;
+  for (long long n : c.n) most = std::max(most, n);
+  if (most > 0) k_copy_arrays<<<(int)std::min<long long>((most / 2 + kBlock) / kBlock, 4096), kBlock, 0, s>>>(c);
   return hipGetLastError();
 }
 

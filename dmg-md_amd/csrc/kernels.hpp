@@ -280,10 +280,21 @@ hipError_t launch_md_first(const DevBox& b, int N, int T, double dt, const doubl
 hipError_t launch_md_second(int N, double dt, const double* mass, double* vel, const double* force, const double* pe,
                             const double* virial, bool thermo, DevWork& tw, hipStream_t s);
 // With step_index (device), the step's target and draws are targets[k] and
-// rand2[2k..] for k = *step_index, advanced by the kernel (t_target unused).
+// rand2[2k..] for k = *step_index, advanced by the kernel (t_target unused);
+// without rand2 they are t_target and draws[0], draws[1] (host).  The thermo
+// goes to report (pinned host memory) too when given.
 hipError_t launch_thermo_final(int N, double volume, int kind, double coupling, double t_target,
                                const double* rand2, double* factor, DevWork& tw, hipStream_t s,
-                               const double* targets = nullptr, int* step_index = nullptr);
+                               const double* targets = nullptr, int* step_index = nullptr,
+                               const double* draws = nullptr, double* report = nullptr);
+// to[a][0 .. n[a]) = from[a][0 .. n[a]), 16-byte aligned arrays
+constexpr int kMaxCopies = 6;
+struct ArrayCopies {
+  double* to[kMaxCopies];
+  const double* from[kMaxCopies];
+  long long n[kMaxCopies];  // 0: none
+};
+hipError_t launch_copy_arrays(const ArrayCopies& c, hipStream_t s);
 // factor[0] = 1 and *step_index = 0: a chunk's first step applies no
 // pending factor and takes the chunk's first target and draws
 hipError_t launch_chunk_start(double* factor, int* step_index, hipStream_t s);
