@@ -572,14 +572,15 @@ void NepEngine::launch_force(const Plan& p, int N, int n1, int n2, int nd1, int 
   ++evaluations_;
   check(launch_rebuild(p.box, N, nd1, nd2, rv * rv, by_gid ? gid : nullptr, w_, s, nullptr, rare_rebuilds_),
         "rebuild");
-  if (w_.split) check(launch_split(p.box, dm_, nd1, nd2, w_, s, tune_.filter_lanes), "candidate rows");
+  if (w_.split) check(launch_split(p.box, dm_, nd1, nd2, w_, s, filter_lanes(nd2 - nd1)), "candidate rows");
   prof_.end(s);
   const bool acc = (flags & 1u) != 0;
   // ANN: FP32 on the matrix cores unless BF16 operands or the vector path are asked for
   const int ann = ann_mode(flags);
   launch_filter_descriptor(p.box, N, nd1, nd2, type, pe, acc, ann, true, s, true);
   prof_.begin(kProfGather, s);
-  check(launch_gather(p.box, dm_, N, n1, n2, nd1, nd2, type, force, virial, acc, w_, s, tune_.gather_lanes),
+  check(launch_gather(p.box, dm_, N, n1, n2, nd1, nd2, type, force, virial, acc, w_, s,
+                      gather_lanes(n2 - n1)),
         "gather");
   prof_.end(s);
   last_box_ = p.box;
@@ -630,7 +631,7 @@ void NepEngine::launch_key(std::vector<long long>& k) const
                         (const void*)w.flags, (const void*)w.partial, (const void*)w.thermo})
     p(q);
   for (int v : {tune_.filter_lanes, tune_.gather_lanes, tune_.row_layout, tune_.overlap, tune_.split,
-                tune_.desc_lanes, (int)tune_.desc_pinned})
+                tune_.desc_lanes, (int)tune_.desc_pinned, (int)tune_.lanes_set})
     k.push_back(v);
 }
 
@@ -804,6 +805,26 @@ LaneRule lane_rule(const DevModel& m)
   return m.T == 1 && m.nA <= 5 && m.L <= kPadL ? LaneRule{8192, 36864} : LaneRule{6144, 57344};
 }
 
+// Lanes of the untuned filter and gather.  Up to these sizes the wavefronts of
+// sixteen and eight lanes per centre leave SIMDs empty or a few long rows
+// set the time: filter with 32 lanes, 4,096 carbon atoms 9.4 us against 11.6,
+// 5,832 of a 130-neighbour model 20 against 27, 3,000 water atoms 11.3 against
+// 13.5 (6,912 Cu atoms 10.4 against 10.2, 10,125 water atoms 19.4 against 17.2);
+// gather with 16 lanes, 4,096 carbon atoms 10.3 us against 13.7, 10,125 water
+// atoms 17.9 against 23.6, 10,976 Cu atoms 12.4 against 12.4 (13,824 carbon
+// atoms 17.2 against 17.5, 16,384 Cu atoms 14.2 against 12.5).
+constexpr int kWideFilterCentres = 6144, kWideGatherAtoms = 12288;
+
+int NepEngine::filter_lanes(int n) const
+{
+  return !tune_.lanes_set && n <= kWideFilterCentres ? 32 : tune_.filter_lanes;
+}
+
+int NepEngine::gather_lanes(int n) const
+{
+  return !tune_.lanes_set && n <= kWideGatherAtoms ? 16 : tune_.gather_lanes;
+}
+
 int NepEngine::desc_lanes(int n, int ann, bool split) const
 {
   if (split || (ann != 1 && ann != 0)) return 1;  // candidate rows, or BF16 operands asked for
@@ -825,7 +846,7 @@ void NepEngine::launch_filter_descriptor(const DevBox& b, int N, int c1, int c2,
   if (!split) {
     if (!w_.split) {
       if (profile) prof_.begin(kProfFilter, s);
-      check(launch_filter(b, dm_, c1, c2, w_, s, tune_.filter_lanes, close), "filter");
+      check(launch_filter(b, dm_, c1, c2, w_, s, filter_lanes(n), close), "filter");
       if (profile) prof_.end(s);
     }
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -838,12 +859,12 @@ void NepEngine::launch_filter_descriptor(const DevBox& b, int N, int c1, int c2,
   }
   // halves on workgroup boundaries of the descriptor (256 centres)
   const int mid = c1 + ((n / 2 + 255) & ~255);
-  check(launch_filter(b, dm_, c1, mid, w_, s, tune_.filter_lanes, close), "filter");
+  check(launch_filter(b, dm_, c1, mid, w_, s, filter_lanes(n), close), "filter");
   // the side stream starts after the first filter (and the rebuild before
   // it): the second filter overlaps the first descriptor
   check(hipEventRecord(fork_, s), "fork");
   check(hipStreamWaitEvent(side_, fork_, 0), "fork wait");
-  check(launch_filter(b, dm_, mid, c2, w_, side_, tune_.filter_lanes, false), "filter");
+  check(launch_filter(b, dm_, mid, c2, w_, side_, filter_lanes(n), false), "filter");
   check(hipEventRecord(join_, side_), "join");
   for (int h = 0; h < 2; ++h) {
     if (h == 1) check(hipStreamWaitEvent(s, join_, 0), "join wait");
@@ -860,7 +881,7 @@ void NepEngine::launch_step_kernels(const DevBox& b, int N, int nc, const int* t
 {
   const int ann = ann_mode(flags);
   launch_filter_descriptor(b, N, 0, nc, type, pe, false, ann, true, s, false);
-  check(launch_gather(b, dm_, N, 0, nc, 0, nc, type, force, virial, false, w_, s, tune_.gather_lanes), "gather");
+  check(launch_gather(b, dm_, N, 0, nc, 0, nc, type, force, virial, false, w_, s, gather_lanes(nc)), "gather");
 }
 
 const NepEngine::Tuning& NepEngine::autotune(const Box& box, int N, int nc, const int* type, const double* pos,
@@ -870,6 +891,7 @@ const NepEngine::Tuning& NepEngine::autotune(const Box& box, int N, int nc, cons
   int reps[3];
   if (N <= 0 || nc <= 0 || nc > N || small_box(box, reps)) return tune_;  // small boxes keep the defaults
   flags &= ~1u;
+  tune_.lanes_set = true;  // every candidate below is what it says
   // the filter's shapes first, then the candidate rows against them
   if (w_.split) set_split(0);
   compute(box, N, 0, nc, 0, nc, type, pos, nullptr, pe, force, virial, flags, s, map);
@@ -1044,6 +1066,7 @@ void NepEngine::set_tiles(int filter_lanes, int gather_lanes)
     throw std::invalid_argument("gather lanes per atom are 4, 8 or 16");
   tune_.filter_lanes = filter_lanes;
   tune_.gather_lanes = gather_lanes;
+  tune_.lanes_set = true;
   tune_.tuned = true;
 }
 
@@ -1156,13 +1179,14 @@ void NepEngine::compute_in(void* ws, size_t ws_bytes, const Box& box, int N, int
   check(launch_pack(b, N, model_.num_types, pos, type, true, w, s), "pack");
   const double rv = model_.rcR_max + kSkin;
   check(launch_rebuild(b, N, nd1, nd2, rv * rv, by_gid ? gid : nullptr, w, s), "rebuild");
-  if (split) check(launch_split(b, dm_, nd1, nd2, w, s, tune_.filter_lanes), "candidate rows");
-  else check(launch_filter(b, dm_, nd1, nd2, w, s, tune_.filter_lanes), "filter");
+  if (split) check(launch_split(b, dm_, nd1, nd2, w, s, filter_lanes(nd2 - nd1)), "candidate rows");
+  else check(launch_filter(b, dm_, nd1, nd2, w, s, filter_lanes(nd2 - nd1)), "filter");
   const bool acc = (flags & 1u) != 0;
   const int ann = ann_mode(flags);
   const int lanes = desc_lanes(nd2 - nd1, ann, split);
   check(launch_descriptor(b, dmd_, N, nd1, nd2, type, pe, acc, ann, w, s, nullptr, nullptr, lanes), "descriptor");
-  check(launch_gather(b, dm_, N, n1, n2, nd1, nd2, type, force, virial, acc, w, s, tune_.gather_lanes), "gather");
+  check(launch_gather(b, dm_, N, n1, n2, nd1, nd2, type, force, virial, acc, w, s, gather_lanes(n2 - n1)),
+        "gather");
   check(hipMemcpyAsync(hflags_, w.flags, kNumFlags * sizeof(int), hipMemcpyDeviceToHost, s), "read status words");
   check(hipStreamSynchronize(s), "synchronise");
   if (hflags_[kFlagBadType]) throw std::invalid_argument("an atom type lies outside [0, num_types)");

@@ -136,6 +136,7 @@ class NepEngine {
   // shapes writes them.
   struct Tuning {
     int filter_lanes = 16, gather_lanes = 8;
+    bool lanes_set = false;             // tuned or set; else small systems take 32 and 16
     double filter_ms[3] = {0, 0, 0}, gather_ms[3] = {0, 0, 0};  // per candidate, in the order above
     int row_layout = -1;                // -1 before tuning (the default rule), else 0 or 1
     int row_capacity = 0;               // entries per row now allocated
@@ -258,6 +259,9 @@ class NepEngine {
                                 int ann, bool close, hipStream_t s, bool profile);
   // lanes per atom of the descriptor for n centres in ANN mode ann
   int desc_lanes(int n, int ann, bool split) const;
+  // lanes per centre of the filter and per atom of the gather for n of them
+  int filter_lanes(int n) const;
+  int gather_lanes(int n) const;
   DevBox last_box_{};  // box of the last evaluation (the filter of copy_pair_rows)
   hipStream_t side_ = nullptr;  // the overlapped filter's stream
   hipEvent_t fork_ = nullptr, join_ = nullptr;

@@ -78,3 +78,19 @@ def test_lane_rule_sizes(dmgx, workloads, material, cells):
     one = gpu_compute(dmgx, nep, s["box"], s["types"], s["pos"])
     for a, b, tol in zip(auto, one, (TOL_EA, TOL_F, TOL_V)):
         assert np.abs(a - b).max() <= tol
+
+
+@pytest.mark.parametrize("n", [6144, 6145, 12288, 12289])
+def test_untuned_lanes_give_the_set_lanes_results(dmgx, n):
+    """The filter's and gather's lanes by size, on both sides of each limit: the edges of the rows exactly those of
+    16 and 8 lanes, and the forces to the rounding of their FP64 sums (1e-12 of the largest term of about 10)."""
+    pos, edge = _cluster(n, n)
+    types = np.zeros(n, np.int32)
+    box = dmgx.Box.orthogonal(edge, edge, edge, pbc=(0, 0, 0))
+    path = os.path.join(POTENTIALS, "nep_carbon.txt")
+    by_size, as_set = dmgx.NEP(path), dmgx.NEP(path)
+    as_set.set_tiles(16, 8)
+    a = gpu_compute(dmgx, by_size, box, types, pos.T)
+    b = gpu_compute(dmgx, as_set, box, types, pos.T)
+    assert np.array_equal(a[0], b[0])
+    assert np.abs(a[1] - b[1]).max() <= 1e-11 and np.abs(a[2] - b[2]).max() <= 1e-11
