@@ -409,69 +409,54 @@ void Server::make_pack(Request& rq, const int* type, const double* mass, const d
     K[d] = box.pbc[d] ? (int)std::ceil(d1 / th[d]) : 0;
     if (K[d] > kImageMax) throw std::invalid_argument("request box too thin for its periodic image shell");
   }
-  std::vector<double> frac(3 * (size_t)N);
-  for (int i = 0; i < N; ++i) {
-    double x[3] = {pos[i], pos[N + i], pos[2 * N + i]}, s[3];
-    to_frac(r->hi, x, s);
-    for (int d = 0; d < 3; ++d) {
-      if (!std::isfinite(s[d])) throw std::invalid_argument("non-finite position");
-      if (box.pbc[d]) s[d] -= std::floor(s[d]);
-      frac[3 * i + d] = s[d];
-    }
-    to_cart(box.h, s, x);
-    for (int d = 0; d < 3; ++d) wpos[(size_t)d * N + i] = x[d];
-  }
-  std::vector<int> g_owner, g_image;
-  std::vector<double> g_shift;
   // every image within d1 of the box (per face pair: a lower bound of the
   // Euclidean distance, so the shell is a superset of what the rows need);
   // an owned atom's Verlet neighbours at any rebuild lie within
   // rc + skin of the box plus the request's motion, covered by the margin
   // (an atom's images in increasing image code, c then b then a: the
-  // reverse search of the Verlet build looks them up by bisection)
-  for (int i = 0; i < N; ++i)
-    for (int ic = -K[2]; ic <= K[2]; ++ic)
-      for (int ib = -K[1]; ib <= K[1]; ++ib)
-        for (int ia = -K[0]; ia <= K[0]; ++ia) {
-          if (ia == 0 && ib == 0 && ic == 0) continue;
-          const int img[3] = {ia, ib, ic};
-          double far = 0.0;
-          for (int d = 0; d < 3; ++d) {
-            const double u = frac[3 * i + d] + img[d];
-            const double e = std::max(0.0, std::max(-u, u - 1.0)) * th[d];
-            far = std::max(far, e);
-          }
-          if (far > d1) continue;
-          const double sh[3] = {box.h[0] * ia + box.h[1] * ib + box.h[2] * ic,
-                                box.h[3] * ia + box.h[4] * ib + box.h[5] * ic,
-                                box.h[6] * ia + box.h[7] * ib + box.h[8] * ic};
-          g_owner.push_back(i);
-          g_image.push_back(image_code(ia, ib, ic));
-          g_shift.insert(g_shift.end(), sh, sh + 3);
-        }
-  if (g_owner.size() >= (1u << 30)) throw std::invalid_argument("request has too many periodic images");
-  r->ng = (int)g_owner.size();
-  const int NG = r->ng;
-  for (int d = 0; d < 3; ++d) {
-    r->lo[d] = 1e300;
-    r->hi_ext[d] = -1e300;
-  }
-  auto extend = [&](const double* x) {
-    for (int d = 0; d < 3; ++d) {
-      r->lo[d] = std::min(r->lo[d], x[d]);
-      r->hi_ext[d] = std::max(r->hi_ext[d], x[d]);
-    }
-  };
+  // reverse search of the Verlet build looks them up by bisection).
+  // The distance bounds a direction at a time, so an atom's images are the
+  // product of the offsets that each direction admits (bit k + kImageMax of
+  // admit); they are counted first and then written straight into the pack.
+  std::vector<unsigned> admit(3 * (size_t)N);
+  std::vector<int> g_first((size_t)N + 1);
+  long long images = 0;
   for (int i = 0; i < N; ++i) {
-    const double x[3] = {wpos[i], wpos[(size_t)N + i], wpos[2 * (size_t)N + i]};
-    extend(x);
+    double x[3] = {pos[i], pos[N + i], pos[2 * N + i]}, s[3];
+    to_frac(r->hi, x, s);
+    long long count = 1;
+    bool self = true;  // the atom itself is no image of its own
+    for (int d = 0; d < 3; ++d) {
+      if (!std::isfinite(s[d])) throw std::invalid_argument("non-finite position");
+      if (box.pbc[d] && !(s[d] > 0.0 && s[d] < 1.0)) s[d] -= std::floor(s[d]);
+      // the distance grows with |k|, so the first offset out of reach ends a side
+      unsigned bits = std::max(0.0, std::max(-s[d], s[d] - 1.0)) * th[d] > d1 ? 0u : 1u << kImageMax;
+      self = self && bits;
+      for (int k = 1; k <= K[d]; ++k) {
+        if ((s[d] + k - 1.0) * th[d] > d1) break;
+        bits |= 1u << (kImageMax + k);
+      }
+      for (int k = 1; k <= K[d]; ++k) {
+        if (-(s[d] - k) * th[d] > d1) break;
+        bits |= 1u << (kImageMax - k);
+      }
+      admit[3 * (size_t)i + d] = bits;
+      count *= __builtin_popcount(bits);
+    }
+    g_first[i] = (int)images;
+    images += count - (self ? 1 : 0);
+    if (images >= (1LL << 30)) throw std::invalid_argument("request has too many periodic images");
+    to_cart(box.h, s, x);
+    for (int d = 0; d < 3; ++d) wpos[(size_t)d * N + i] = x[d];
   }
-  for (int g = 0; g < NG; ++g) {
-    const int o = g_owner[g];
-    const double x[3] = {wpos[o] + g_shift[3 * g], wpos[(size_t)N + o] + g_shift[3 * g + 1],
-                         wpos[2 * (size_t)N + o] + g_shift[3 * g + 2]};
-    extend(x);
-  }
+  const int NG = (int)images;
+  r->ng = g_first[N] = NG;
+  double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+  for (int d = 0; d < 3; ++d)
+    for (int i = 0; i < N; ++i) {
+      lo[d] = std::min(lo[d], wpos[(size_t)d * N + i]);
+      hi[d] = std::max(hi[d], wpos[(size_t)d * N + i]);
+    }
   const size_t doff = serve_pack_double_offset(N, NG), bytes = serve_pack_bytes(N, NG);
   r->bytes = (long long)std::ceil(N * slot_bytes(model, true) + NG * slot_bytes(model, false)) + (long long)bytes;
   if (r->footprint() > cfg_.max_atoms)
@@ -486,20 +471,53 @@ void Server::make_pack(Request& rq, const int* type, const double* mass, const d
   int* pi = reinterpret_cast<int*>(host);
   double* pd = reinterpret_cast<double*>(host + doff);
   std::copy(type, type + N, pi);
-  for (int g = 0, a = 0; a < N; ++a) {
-    pi[N + a] = g;
-    while (g < NG && g_owner[g] == a) ++g;
-  }
-  std::copy(g_owner.begin(), g_owner.end(), pi + 2 * (size_t)N);
-  std::copy(g_image.begin(), g_image.end(), pi + 2 * (size_t)N + NG);
+  std::copy(g_first.begin(), g_first.begin() + N, pi + N);
   std::copy(mass, mass + N, pd);
-  for (int a = 0; a < N; ++a)
-    for (int d = 0; d < 3; ++d) {
-      pd[N + 3 * (size_t)a + d] = wpos[(size_t)d * N + a];
-      pd[4 * (size_t)N + 3 * (size_t)a + d] = vel ? vel[(size_t)d * N + a] : 0.0;
-      pd[7 * (size_t)N + 3 * (size_t)a + d] = force ? force[(size_t)d * N + a] : 0.0;
+  auto interleave = [N](const double* from, double* to) {
+    if (!from) {
+      std::fill(to, to + 3 * (size_t)N, 0.0);
+      return;
     }
-  std::copy(g_shift.begin(), g_shift.end(), pd + 10 * (size_t)N);
+    for (size_t a = 0; a < (size_t)N; ++a) {
+      to[3 * a] = from[a];
+      to[3 * a + 1] = from[(size_t)N + a];
+      to[3 * a + 2] = from[2 * (size_t)N + a];
+    }
+  };
+  interleave(wpos.data(), pd + N);
+  interleave(vel, pd + 4 * (size_t)N);
+  interleave(force, pd + 7 * (size_t)N);
+  int* g_owner = pi + 2 * (size_t)N;
+  int* g_image = g_owner + NG;
+  double* g_shift = pd + 10 * (size_t)N;
+  size_t g = 0;
+  for (int i = 0; i < N; ++i) {
+    if (g_first[i] == g_first[i + 1]) continue;
+    const unsigned* in = &admit[3 * (size_t)i];
+    const double at[3] = {wpos[i], wpos[(size_t)N + i], wpos[2 * (size_t)N + i]};
+    for (unsigned mc = in[2]; mc; mc &= mc - 1)
+      for (unsigned mb = in[1]; mb; mb &= mb - 1)
+        for (unsigned ma = in[0]; ma; ma &= ma - 1) {
+          const int ia = __builtin_ctz(ma) - kImageMax, ib = __builtin_ctz(mb) - kImageMax,
+                    ic = __builtin_ctz(mc) - kImageMax;
+          if (ia == 0 && ib == 0 && ic == 0) continue;
+          const double sh[3] = {box.h[0] * ia + box.h[1] * ib + box.h[2] * ic,
+                                box.h[3] * ia + box.h[4] * ib + box.h[5] * ic,
+                                box.h[6] * ia + box.h[7] * ib + box.h[8] * ic};
+          g_owner[g] = i;
+          g_image[g] = image_code(ia, ib, ic);
+          for (int d = 0; d < 3; ++d) {
+            g_shift[3 * g + d] = sh[d];
+            lo[d] = std::min(lo[d], at[d] + sh[d]);
+            hi[d] = std::max(hi[d], at[d] + sh[d]);
+          }
+          ++g;
+        }
+  }
+  for (int d = 0; d < 3; ++d) {
+    r->lo[d] = lo[d];
+    r->hi_ext[d] = hi[d];
+  }
   // asynchronous upload: the lane's stream waits for `ready` before it
   // places the request
   r->pack = pack_get(bytes, &r->pack_cap);
