@@ -656,13 +656,13 @@ __global__ __launch_bounds__(256, 4) void k_verlet_build(const int* __restrict__
       while (rp[q + 1] <= k) ++q;
       return rs[q] + k;
     };
-    // each step tests candidates k and k + kRowLanes of every lane, whose
-    // loads were issued in the step before
-    constexpr int kStep = 2 * kRowLanes;
-    int jn[2] = {0, 0};
-    double4 pn[2] = {make_double4(0, 0, 0, 0), make_double4(0, 0, 0, 0)};
+    // each step tests kBatch candidates of every lane, whose loads were issued
+    // in the step before
+    constexpr int kBatch = 2, kStep = kBatch * kRowLanes;
+    int jn[kBatch] = {};
+    double4 pn[kBatch] = {};
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < kBatch; ++h) {
       const int k = lg + h * kRowLanes;
       if (k < total) {
         const int sl = slot_of(k);
@@ -673,10 +673,10 @@ __global__ __launch_bounds__(256, 4) void k_verlet_build(const int* __restrict__
     int found = 0;
     bool wide = false;  // a key of this row needs more than 32 bits
     for (int k0 = 0; __any(k0 < total); k0 += kStep) {
-      int jc[2];
-      double4 pc[2];
+      int jc[kBatch];
+      double4 pc[kBatch];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
+      for (int h = 0; h < kBatch; ++h) {
         jc[h] = jn[h];
         pc[h] = pn[h];
         const int k = k0 + kStep + lg + h * kRowLanes;
@@ -687,7 +687,7 @@ __global__ __launch_bounds__(256, 4) void k_verlet_build(const int* __restrict__
         }
       }
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
+      for (int h = 0; h < kBatch; ++h) {
         const int k = k0 + lg + h * kRowLanes;
         const int j = jc[h];
         double x = pc[h].x - pi.x, y = pc[h].y - pi.y, z = pc[h].z - pi.z;
@@ -738,6 +738,7 @@ __global__ __launch_bounds__(256, 4) void k_verlet_build(const int* __restrict__
 // lane searches kRevBatch edges of its centre in lockstep.
 constexpr int kRevBatch = 4;
 
+template <int G>
 __global__ __launch_bounds__(256) void k_verlet_reverse(const int* __restrict__ go, int c1, int c2,
                                                         const uint64_t* __restrict__ gid, DevWork w)
 {
@@ -745,21 +746,21 @@ __global__ __launch_bounds__(256) void k_verlet_reverse(const int* __restrict__ 
   if (!go_word) return;
   const bool listed = rebuild_listed(w.map);
   const int ncent = listed ? w.map.req_off[2 * w.map.n_req] : c2 - c1;
-  const int lg = threadIdx.x % kRowLanes;
-  for (int kc = (blockIdx.x * blockDim.x + threadIdx.x) / kRowLanes; kc < ncent;
-       kc += gridDim.x * (blockDim.x / kRowLanes)) {
+  const int lg = threadIdx.x % G;
+  for (int kc = (blockIdx.x * blockDim.x + threadIdx.x) / G; kc < ncent;
+       kc += gridDim.x * (blockDim.x / G)) {
   const int i = listed ? w.map.lists[kc] : c1 + kc;
   if (i < c1 || i >= c2 || (!listed && !slot_rebuilt(w.map, go_word, i))) continue;
   const int n = min(w.vn[i], w.MV);
   const int* ri = w.vl + (size_t)i * w.MV;
   const ImageMap& im = w.map;
-  for (int p0 = lg; p0 < n; p0 += kRevBatch * kRowLanes) {
+  for (int p0 = lg; p0 < n; p0 += kRevBatch * G) {
     int t[kRevBatch], lo[kRevBatch], hi[kRevBatch], q[kRevBatch], ov[kRevBatch];
     bool own[kRevBatch];
     const int* ro[kRevBatch];
 #pragma unroll
     for (int u = 0; u < kRevBatch; ++u) {
-      const int p = p0 + u * kRowLanes;
+      const int p = p0 + u * G;
       // the reverse of i -> j is found in the row of j; with an image map, j
       // stands for its owner o = owner[j] shifted by S, and the reverse entry
       // is o -> (the image of i shifted by -S), one of i's own ghost slots
@@ -823,7 +824,7 @@ __global__ __launch_bounds__(256) void k_verlet_reverse(const int* __restrict__ 
     }
 #pragma unroll
     for (int u = 0; u < kRevBatch; ++u) {
-      const int p = p0 + u * kRowLanes;
+      const int p = p0 + u * G;
       if (own[u]) {
         w.vrev[(size_t)i * w.MV + p] = (short)q[u];
         if (!im.owner && q[u] >= 0) w.vrev[(size_t)ov[u] * w.MV + q[u]] = (short)p;
@@ -845,6 +846,13 @@ constexpr int kListBlocks = 2048;
 // 13; and a step without a rebuild is two launches (7 us) shorter, 82 -> 74 us
 // a step of 4,096 carbon atoms.
 constexpr int kOneBlockAtoms = 6144, kOneBlockCells = 15 * 1024;
+
+// A wavefront per centre searches the reverse entries of small systems, whose
+// searches are latency: 64-atom box 8.1 us against 16.5 with kRowLanes, Cu with
+// vacancies 7.2 against 10.3, 4,096 carbon atoms 11.0 against 17.3, 5,832 of a
+// 130-neighbour model 49 against 66 (11,000 BaTiO3 atoms 21.9 against 21.7, 60,001
+// keyed rows 103 against 89).
+constexpr int kWideReverse = 8192;
 
 // LDS of one centre of the build: its row buffers and candidate ranges
 size_t build_lds_per_centre(int mv, bool keyed) { return build_row_lds(mv, keyed) + kRangeLds; }
@@ -922,7 +930,9 @@ hipError_t launch_rebuild(const DevBox& b, int N, int c1, int c2, double rv2, co
     constexpr int rows_per_block = 256 / kRowLanes;
     // build workgroups hold groups * kRowLanes lanes
     int nb = (c2 - c1 + groups - 1) / groups;
-    int nr = (c2 - c1 + rows_per_block - 1) / rows_per_block;
+    const bool wide = c2 - c1 <= kWideReverse;
+    const int reverses_per_block = wide ? 256 / 64 : rows_per_block;
+    int nr = (c2 - c1 + reverses_per_block - 1) / reverses_per_block;
     if (cap) {
       nb = std::min(nb, kListBlocks * (rows_per_block / groups));
       nr = std::min(nr, kListBlocks);
@@ -936,7 +946,8 @@ hipError_t launch_rebuild(const DevBox& b, int N, int c1, int c2, double rv2, co
     };
     const auto build = keyed ? pick(std::true_type{}, listed, plain) : pick(std::false_type{}, listed, plain);
     build<<<nb, groups * kRowLanes, lds, s>>>(go, b, c1, c2, groups, row_shift, w.xq, rv2, gid, w);
-    k_verlet_reverse<<<nr, 256, 0, s>>>(go, c1, c2, gid, w);
+    if (wide) k_verlet_reverse<64><<<nr, 256, 0, s>>>(go, c1, c2, gid, w);
+    else k_verlet_reverse<kRowLanes><<<nr, 256, 0, s>>>(go, c1, c2, gid, w);
   }
   // the request marks of this rebuild are spent
   if (w.map.slot_req && w.map.n_req > 0) k_clear_moved<<<nblk(w.map.n_req), kBlock, 0, s>>>(go, w.map);

@@ -10,8 +10,8 @@ import numpy as np
 import pytest
 
 from conftest import POTENTIALS
-from gpu_helpers import gpu_compute, to_dev
-from oracle import neighbor_rows
+from gpu_helpers import errors, gpu_compute, to_dev
+from oracle import OracleNEP, neighbor_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -87,3 +87,19 @@ def test_rows_over_cell_grids(dmgx, n, edges, pbc):
     ref = neighbor_rows(h, pbc, pos, nep.info.rc_radial_max + 1.0, max_nb=1024)
     for i in range(n):
         assert np.array_equal(rows[i], np.sort(np.asarray(ref[i]))), i
+
+
+@pytest.mark.parametrize("n", [8192, 8193])
+def test_reverse_entries_around_the_wide_search(dmgx, n):
+    """Forces (which read every edge's reverse entry) against the oracle on both sides of the size up to which a
+    wavefront searches a centre's reverse entries, at the parity tests' bars."""
+    rng = np.random.default_rng(n)
+    m = int(np.ceil(n ** (1 / 3)))
+    g = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)[rng.permutation(m ** 3)[:n]]
+    pos = np.ascontiguousarray((5.0 + 2.3 * g + rng.uniform(-0.15, 0.15, (n, 3))).T)
+    edge = 10.0 + 2.3 * m
+    path = os.path.join(POTENTIALS, "nep_carbon.txt")
+    h, pbc, types = np.diag([edge] * 3), (0, 0, 0), np.zeros(n, np.int32)
+    ref = OracleNEP(path, round_params_to_float=True).compute(h, pbc, types, pos)
+    e = errors(gpu_compute(dmgx, dmgx.NEP(path), dmgx.Box(h, pbc), types, pos), ref)
+    assert e["force"] <= 1e-4 and e["energy_atom_max"] <= 2e-5 and e["virial"] <= 2e-4, e
