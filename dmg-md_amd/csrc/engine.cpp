@@ -1761,14 +1761,17 @@ void MdState::run(int steps, double dt_fs, const EnsembleConfig& ens, unsigned f
         p.begin(kProfIntegrate, stream_);
         // the displacement test honours what box rescales have used of the skin
         check(launch_md_first(plan.box, N_, nep_->model().num_types, dt, mass_, pos_, vel_, force_, fac, type_,
-                              plan.forced, nep_->work(), stream_, unwrapped_, nep_->half_skin()),
+                              plan.forced, nep_->work(), stream_, unwrapped_, nep_->half_skin(), !thermo_on && k > 0),
               "velocity Verlet (first half)");
         p.end(stream_);
         nep_->launch_force(plan, N_, 0, N_, 0, N_, type_, nullptr, pe_, force_, vir_, flags & ~1u, stream_);
-        p.begin(kProfIntegrate, stream_);
-        check(launch_md_second(N_, dt, mass_, vel_, force_, pe_, vir_, thermo_on, tw_, stream_),
-              "velocity Verlet (second half)");
-        p.end(stream_);
+        // without a thermostat the next step's first half takes this kick along
+        if (thermo_on || k + 1 == n) {
+          p.begin(kProfIntegrate, stream_);
+          check(launch_md_second(N_, dt, mass_, vel_, force_, pe_, vir_, thermo_on, tw_, stream_),
+                "velocity Verlet (second half)");
+          p.end(stream_);
+        }
         if (thermo_on) {
           p.begin(kProfThermo, stream_);
           // a barostat step's thermo (before the thermostat rescale) is read

@@ -268,15 +268,15 @@ hipError_t launch_ensemble_scale(int kind, int N, double coupling, double t_targ
                                  double* factor, const double* thermo, double* vel, hipStream_t s);
 hipError_t launch_check_scaled(int n, double factor, const double* data, int* flag, hipStream_t s);
 
-// Fused MD-loop kernels.  launch_md_first: v *= factor[0] (if factor), half
-// kick, drift, wrap, pack (x, y, z, type) into w.xq and the displacement test
-// (or a forced rebuild request).  launch_md_second: half kick, plus the thermo
+// Fused MD-loop kernels.  launch_md_first: v *= factor[0] (if factor), the last
+// step's second half kick (if kick), half kick, drift, wrap, pack (x, y, z,
+// type) into w.xq and the displacement test (or a forced rebuild request).  launch_md_second: half kick, plus the thermo
 // partial sums into tw.partial when `thermo`.  launch_thermo_final: tw.thermo
 // from the partials and, when kind != 0, the velocity factor of that
 // thermostat into factor[0] (see launch_ensemble_scale for kind).
 hipError_t launch_md_first(const DevBox& b, int N, int T, double dt, const double* mass, double* pos, double* vel,
                            const double* force, const double* factor, const int* type, bool forced, DevWork& w,
-                           hipStream_t s, double* unwrapped = nullptr, double half_skin = -1.0);
+                           hipStream_t s, double* unwrapped = nullptr, double half_skin = -1.0, bool kick = false);
 hipError_t launch_md_second(int N, double dt, const double* mass, double* vel, const double* force, const double* pe,
                             const double* virial, bool thermo, DevWork& tw, hipStream_t s);
 // With step_index (device), the step's target and draws are targets[k] and
