@@ -4,17 +4,18 @@
 //  * Verlet list with a 1 A skin, rebuilt only when an atom moved more than
 //    skin/2 (neighbor.cu:446-582); rows hold slot indices, sorted ascending
 //    (or by global id), with a precomputed reverse position per entry.
-//  * Every step a filter pass (16 lanes per centre, ballot compaction) turns
+//  * Every step a filter pass (16 or 32 lanes per centre, ballot compaction) turns
 //    each Verlet row into one compact edge row: angular edges first (slots
 //    0..na-1, ascending), radial-only edges from the end of the row
 //    downward, each edge a float4 (FP64 minimum-image r_ij rounded to float,
 //    neighbour slot).  Later kernels stream these rows instead of
-//    re-gathering positions.  All rows are row-major ([i*M + slot]).
+//    re-gathering positions.  The edge rows are interleaved by tiles of 64
+//    centres (row_begin), the others row-major ([i*M + slot]).
 //  * One fused per-atom kernel does descriptor -> ANN -> adjoints -> angular
 //    partial forces: the angular moments s[n][lm] stay in registers, are
 //    turned in place into the adjoint dE/ds, and each angular edge's
 //    dE_i/dr_ij is written at i's slot.
-//  * The gather kernel (8 lanes per atom) forms the radial pair force from
+//  * The gather kernel (8 or 16 lanes per atom) forms the radial pair force from
 //    both centres' basis-space adjoints, adds the angular partials of both
 //    directions (dE_j/dr_ji read from j's row through the reverse index) and
 //    ZBL, and writes FP64 force/virial.  No floating-point atomics anywhere:
@@ -32,8 +33,8 @@ namespace dmgx {
 
 // kFilterLanes lanes per centre walk its Verlet row kFilterLanes entries per
 // round; the kept entries of each round are compacted with a wavefront
-// ballot, so every store of the kernel is contiguous inside the row.  The
-// loads of kFilterBatch rounds (row entries, their reverse positions, then
+// ballot and staged in LDS, from where the workgroup stores whole lines of the
+// interleaved rows.  The loads of kFilterBatch rounds (row entries, their reverse positions, then
 // the neighbours' packed positions) are issued before any of them is used,
 // so a wave waits for two memory latencies per batch instead of two per
 // round.  Types were validated when the step's positions were packed; here
@@ -967,8 +968,6 @@ __global__ void k_check_scaled(int n, double factor, const double* __restrict__ 
 
 static inline int nblk(int n) { return (n + kBlock - 1) / kBlock; }
 
-// lanes per centre (8, 16 or 32) and the Verlet entries each lane loads
-// per pass (7, 7 or 4)
 // closes a rebuild request as the filter does, for an evaluation whose
 // first filter launch has no centres
 __global__ void k_close_request(int* __restrict__ flags)
@@ -979,6 +978,8 @@ __global__ void k_close_request(int* __restrict__ flags)
   }
 }
 
+// lanes per centre (8, 16 or 32) and the Verlet entries each lane loads
+// per pass (7, 5 or 4)
 template <int G, int RB, bool CAND = false>
 static void run_filter(const DevBox& b, const DevModel& m, int c1, int c2, int close, DevWork& w, hipStream_t s)
 {

@@ -12,8 +12,9 @@
 // position of the centre inside each neighbour's row.
 //
 // Layout: rows are row-major (vl[i*MV + p]) so that a group of lanes that
-// works on one centre reads and writes contiguous memory.  Build, sort and
-// reverse search run with kRowLanes lanes per centre (4 centres per wave).
+// works on one centre reads and writes contiguous memory.  Build and sort run
+// with kRowLanes lanes per centre (4 centres per wave), the reverse search
+// with kRowLanes or, in small systems, a wavefront.
 #include <algorithm>
 #include <limits>
 #include <type_traits>
