@@ -928,20 +928,16 @@ const NepEngine::Tuning& NepEngine::autotune(const Box& box, int N, int nc, cons
   // whole force sequence with them
   auto tune_lanes = [&](int layout) {
     const int fl[3] = {8, 16, 32}, gl[3] = {4, 8, 16};
-    int best = 1;
-    for (int k = 0; k < 3; ++k) {
+    for (int k = 0; k < 3; ++k)
       tune_.filter_ms[k] = time_median([&] { check(launch_filter(b, dm_, 0, nc, w_, s, fl[k]), "tune filter"); });
-      if (tune_.filter_ms[k] < tune_.filter_ms[best]) best = k;
-    }
-    tune_.filter_lanes = fl[best];
-    best = 1;
-    for (int k = 0; k < 3; ++k) {
+    tune_.filter_lanes = fl[std::min_element(tune_.filter_ms, tune_.filter_ms + 3) - tune_.filter_ms];
+    for (int k = 0; k < 3; ++k)
       tune_.gather_ms[k] = time_median([&] {
         check(launch_gather(b, dm_, N, 0, nc, 0, nc, type, force, virial, false, w_, s, gl[k]), "tune gather");
       });
-      if (tune_.gather_ms[k] < tune_.gather_ms[best]) best = k;
-    }
-    tune_.gather_lanes = gl[best];
+    // (after all three are timed: 256,000 Cu atoms 104 us with four lanes
+    // against 110 with eight, 192,000 water atoms 216 against 213)
+    tune_.gather_lanes = gl[std::min_element(tune_.gather_ms, tune_.gather_ms + 3) - tune_.gather_ms];
     tune_.force_ms[layout] = time_median([&] { launch_step_kernels(b, N, nc, type, pe, force, virial, flags, s); });
   };
   const int layout0 = (w_.MV == padded_rows(mv_base_, 1)) ? 1 : 0;
