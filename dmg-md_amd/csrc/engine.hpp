@@ -136,7 +136,7 @@ class NepEngine {
   // shapes writes them.
   struct Tuning {
     int filter_lanes = 16, gather_lanes = 8;
-    bool lanes_set = false;             // tuned or set; else small systems take 32 and 16
+    bool lanes_set = false;             // tuned or set; else by size (filter_lanes, gather_lanes)
     double filter_ms[3] = {0, 0, 0}, gather_ms[3] = {0, 0, 0};  // per candidate, in the order above
     int row_layout = -1;                // -1 before tuning (the default rule), else 0 or 1
     int row_capacity = 0;               // entries per row now allocated

@@ -80,7 +80,7 @@ def test_lane_rule_sizes(dmgx, workloads, material, cells):
         assert np.abs(a - b).max() <= tol
 
 
-@pytest.mark.parametrize("n", [6144, 6145, 12288, 12289])
+@pytest.mark.parametrize("n", [6144, 6145, 12288, 12289, 36864, 36865])
 def test_untuned_lanes_give_the_set_lanes_results(dmgx, n):
     """The filter's and gather's lanes by size, on both sides of each limit: the edges of the rows exactly those of
     16 and 8 lanes, and the forces to the rounding of their FP64 sums (1e-12 of the largest term of about 10)."""
