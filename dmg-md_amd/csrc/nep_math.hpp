@@ -139,10 +139,12 @@ __device__ __forceinline__ void harmonics(float ux, float uy, float uz, float* Y
 // r = 1 / (e^{2|v|} + 1): |x| = 1 - 2 r and s = 4 e^{2|v|} r^2 above |v| = 0.6
 // (the second free of the cancellation in 1 - x^2), an odd polynomial (a
 // minimax fit of the relative error, below 2 ulp) below it.  No branches.  The
-// library's tanh is about twice as long.
+// library's tanh is about twice as long.  The clamp is the minimum that passes
+// NaN on (one v_minimum3_f32; fminf would return 20 and make it +-1): a NaN
+// descriptor, of two atoms at the same place, stays one in the energy.
 __device__ __forceinline__ void tanh_sech2(float v, float& x, float& s)
 {
-  const float av = fminf(fabsf(v), 20.0f), z = v * v;
+  const float av = __builtin_elementwise_minimum(fabsf(v), 20.0f), z = v * v;
   const float e = __builtin_amdgcn_exp2f(2.88539008f * av), e1 = e + 1.0f;
   float r = __builtin_amdgcn_rcpf(e1);
   r = fmaf(r, fmaf(-e1, r, 1.0f), r);
