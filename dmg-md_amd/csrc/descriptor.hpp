@@ -479,6 +479,68 @@ constexpr bool mfma_ann_fits()
          (ONE ? 64 * 1024 : kDescLdsMax);
 }
 
+// The angular edges' second pass of the generic instance, whose moments (240 or
+// 800 a lane) lie in scratch: the basis first and then a function at a time,
+// and the adjoint contracted degree by degree, in the order the moments lie
+// in.  The form by order of the exact instances, their shared loop for the
+// radial terms and their four records in flight cost it registers and code
+// without an access less: 110,592 atoms with 10 radial functions 3,040 us
+// against 3,876, 32,768 with a basis of 16 1,229 against 1,391, 110,592 at
+// order 6 8,031 against 10,471.
+template <int NA, int KA>
+__device__ __forceinline__ void basis_by_function(int nA, int kA, const float* __restrict__ c, float rcinv, float d,
+                                                  float fc, float fcp, float* g, float* gp)
+{
+  float f[KA], fp[KA];
+  cheb_d<KA>(kA, rcinv, d, fc, fcp, f, fp);
+#pragma unroll
+  for (int n = 0; n < NA; ++n) {
+    g[n] = 0.0f;
+    gp[n] = 0.0f;
+    if (n < nA) {
+#pragma unroll
+      for (int k = 0; k < KA; ++k)
+        if (k < kA) {
+          g[n] += c[n * kA + k] * f[k];
+          gp[n] += c[n * kA + k] * fp[k];
+        }
+    }
+  }
+}
+template <int NA, int LM, int NABC>
+__device__ __forceinline__ void contract_by_degree(const float (&s)[NA][NABC], const float* g, const float* gp,
+                                                   const DirectionPowers<LM>& pw, float& Pr, float& Gx, float& Gy,
+                                                   float& Gz)
+{
+  static_for<1, LM>([&](auto l) {
+    constexpr int L = decltype(l)::value, b = L * L - 1;
+    float A = 0.0f, B = 0.0f;
+#pragma unroll
+    for (int n = 0; n < NA; ++n) {
+      A += s[n][b] * g[n];
+      B += s[n][b] * gp[n];
+    }
+    Pr += B * harmonic_z<L, 0>(pw.zp);
+    Gz += A * harmonic_dz<L, 0>(pw.zp);
+    static_for<1, L>([&](auto mm) {
+      constexpr int M = decltype(mm)::value, ir = b + 2 * M - 1, ii = ir + 1;
+      float Ar = 0.0f, Ai = 0.0f, Br = 0.0f, Bi = 0.0f;
+#pragma unroll
+      for (int n = 0; n < NA; ++n) {
+        Ar += s[n][ir] * g[n];
+        Ai += s[n][ii] * g[n];
+        Br += s[n][ir] * gp[n];
+        Bi += s[n][ii] * gp[n];
+      }
+      const float Z = harmonic_z<L, M>(pw.zp), dZ = harmonic_dz<L, M>(pw.zp), mz = (float)M * Z;
+      Pr += Z * (Br * pw.re[M] + Bi * pw.im[M]);
+      Gx += mz * (Ar * pw.re[M - 1] + Ai * pw.im[M - 1]);
+      Gy += mz * (Ai * pw.re[M - 1] - Ar * pw.im[M - 1]);
+      Gz += dZ * (Ar * pw.re[M] + Ai * pw.im[M]);
+    });
+  });
+}
+
 // What bounds it: vector instruction issue, most of it in the two loops over
 // the angular edges (about 240 and 500 instructions per edge and wavefront at
 // n_max 4, basis 8, order 4).  The angular coefficients are literals, the
@@ -600,6 +662,8 @@ __global__ __launch_bounds__(kDescBlock, (desc_waves<C, P>())) void k_descriptor
   for (int t = 0; t < (C::cl ? C::ltypes : 1); ++t)
 #pragma unroll
     for (int k = 0; k < KR; ++k) Ft[t][k] = 0.0f;
+  // the angular edges' radial terms in the loop over their moments
+  constexpr bool kOneLoop = C::exact;
   auto radial_edge = [&](const float d, const int tj) {
     const float rc = C::one ? rcRf[0] : pcut[ti * T + tj];
     const float rcinv = C::one ? 1.0f / rc : pcut[kPairs + ti * T + tj];
@@ -640,21 +704,25 @@ __global__ __launch_bounds__(kDescBlock, (desc_waves<C, P>())) void k_descriptor
   if (!CAND) {
     // radial-only edges, stored from the row's end downward; kAhead records
     // in flight (the work per edge is short).  The angular edges' radial terms
-    // are summed in the loop over the angular moments.
-    constexpr int kAhead = P == 1 ? 12 : 3;
+    // are summed in the loop over the angular moments, or here as well.
+    constexpr int kAhead = !C::exact ? 8 : P == 1 ? 12 : 3;
     const float4* const first = erow + (size_t)(w.MR - 1) * kTile;
-    const int nro = nr - na;
+    const int nro = kOneLoop ? nr - na : nr;
+    auto record = [&](int e) {
+      if (!kOneLoop && e < na) return erow[(size_t)e * kTile];
+      return first[-(ptrdiff_t)(kOneLoop ? e : e - na) * kTile];
+    };
     float4 ring[kAhead];
 #pragma unroll
     for (int u = 0; u < kAhead; ++u)
-      ring[u] = u * P + lr < nro ? first[-(ptrdiff_t)(u * P + lr) * kTile] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      ring[u] = u * P + lr < nro ? record(u * P + lr) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     for (int e0 = lr; e0 < nro; e0 += kAhead * P)
 #pragma unroll
       for (int u = 0; u < kAhead; ++u) {
         const int e = e0 + u * P;
         if (e >= nro) break;
         const float4 r = ring[u];
-        if (e + kAhead * P < nro) ring[u] = first[-(ptrdiff_t)(e + kAhead * P) * kTile];
+        if (e + kAhead * P < nro) ring[u] = record(e + kAhead * P);
         const float d2 = r.x * r.x + r.y * r.y + r.z * r.z;
         radial_edge(d2 * __builtin_amdgcn_rsqf(d2), type_of(r));
       }
@@ -740,7 +808,7 @@ __global__ __launch_bounds__(kDescBlock, (desc_waves<C, P>())) void k_descriptor
   // each lane takes every P-th edge with kRing records in flight: a record
   // comes from beyond L1, and an edge's arithmetic covers a fraction of that
   // (one ahead: 171 us on 256,000 Cu atoms, four: 165)
-  constexpr int kRing = P == 1 ? 4 : 1;
+  constexpr int kRing = P == 1 && C::exact ? 4 : 1;
   auto edge_at = [&](int e) { return erow[(size_t)e * kTile]; };
   float4 ring[kRing];
   auto fill_ring = [&]() {
@@ -760,7 +828,7 @@ __global__ __launch_bounds__(kDescBlock, (desc_waves<C, P>())) void k_descriptor
     const float d2 = r.x * r.x + r.y * r.y + r.z * r.z;
     const float dinv = __builtin_amdgcn_rsqf(d2);  // hardware 1/sqrt (1 ulp); edges have d > 0
     const float d = d2 * dinv;
-    if (!CAND) radial_edge(d, tj);
+    if (!CAND && kOneLoop) radial_edge(d, tj);
     const float rc = C::one ? rcAf[0] : pcut[2 * kPairs + ti * T + tj];
     const float rcinv = C::one ? 1.0f / rc : pcut[3 * kPairs + ti * T + tj];
     if (m.zbl) {
@@ -993,7 +1061,9 @@ __global__ __launch_bounds__(kDescBlock, (desc_waves<C, P>())) void k_descriptor
     // with S_n = sum c_nk (T_k(x) + 1) and D_n = sum c_nk T_k'(x):
     // g_n = (fc/2) S_n, g'_n = (fc/2) x' D_n + (fc'/2) S_n
     float g[NA], gp[NA];
-    {
+    if constexpr (!C::exact) {
+      basis_by_function<NA, KA>(nA, kA, c, rcinv, d, fc, fcp, g, gp);
+    } else {
       const float t = d * rcinv - 1.0f, x = 2.0f * t * t - 1.0f;
       const float hfc = 0.5f * fc, hfcp = 0.5f * fcp, hx = hfc * (4.0f * t * rcinv);
       float T1 = x, T0 = 1.0f, U1 = 1.0f, U0 = 0.0f;  // U1 = U_{k-1}, T_k' = k U_{k-1}
@@ -1032,56 +1102,60 @@ __global__ __launch_bounds__(kDescBlock, (desc_waves<C, P>())) void k_descriptor
     // dY/du (Y = Z(uz) Re/Im (ux + i uy)^m)
     const DirectionPowers<LM> pw(ux, uy, uz);
     float Pr = 0.0f, Gx = 0.0f, Gy = 0.0f, Gz = 0.0f;
-    static_for<1, LM>([&](auto l) {
-      constexpr int L = decltype(l)::value, a = L * L - 1;
-      float A = 0.0f, B = 0.0f;
-#pragma unroll
-      for (int n = 0; n < NA; ++n) {
-        A += s[n][a] * g[n];
-        B += s[n][a] * gp[n];
-      }
-      Pr += B * harmonic_z<L, 0>(pw.zp);
-      Gz += A * harmonic_dz<L, 0>(pw.zp);
-    });
-    static_for<1, LM>([&](auto mm) {
-      constexpr int M = decltype(mm)::value;
-      float R = 0.0f, I = 0.0f, dR = 0.0f, dI = 0.0f, RB = 0.0f, IB = 0.0f;
-      static_for<M, LM>([&](auto l) {
-        constexpr int L = decltype(l)::value, ir = L * L - 1 + 2 * M - 1, ii = ir + 1;
-        float Ar = 0.0f, Ai = 0.0f, Br = 0.0f, Bi = 0.0f;
+    if constexpr (!C::exact) {
+      contract_by_degree(s, g, gp, pw, Pr, Gx, Gy, Gz);
+    } else {
+      static_for<1, LM>([&](auto l) {
+        constexpr int L = decltype(l)::value, a = L * L - 1;
+        float A = 0.0f, B = 0.0f;
 #pragma unroll
         for (int n = 0; n < NA; ++n) {
-          Ar += s[n][ir] * g[n];
-          Ai += s[n][ii] * g[n];
-          Br += s[n][ir] * gp[n];
-          Bi += s[n][ii] * gp[n];
+          A += s[n][a] * g[n];
+          B += s[n][a] * gp[n];
         }
-        if constexpr (L == M) {  // Z = 1
-          R = Ar;
-          I = Ai;
-          RB = Br;
-          IB = Bi;
-        } else {
-          const float Z = harmonic_z<L, M>(pw.zp), dZ = harmonic_dz<L, M>(pw.zp);
-          R += Z * Ar;
-          I += Z * Ai;
-          RB += Z * Br;
-          IB += Z * Bi;
-          dR += dZ * Ar;
-          dI += dZ * Ai;
-        }
+        Pr += B * harmonic_z<L, 0>(pw.zp);
+        Gz += A * harmonic_dz<L, 0>(pw.zp);
       });
-      Pr += RB * pw.re[M] + IB * pw.im[M];
-      constexpr float fm = (float)M;
-      if constexpr (M == 1) {
-        Gx += R;
-        Gy += I;
-      } else {
-        Gx += fm * (R * pw.re[M - 1] + I * pw.im[M - 1]);
-        Gy += fm * (I * pw.re[M - 1] - R * pw.im[M - 1]);
-      }
-      if constexpr (M < LM) Gz += dR * pw.re[M] + dI * pw.im[M];
-    });
+      static_for<1, LM>([&](auto mm) {
+        constexpr int M = decltype(mm)::value;
+        float R = 0.0f, I = 0.0f, dR = 0.0f, dI = 0.0f, RB = 0.0f, IB = 0.0f;
+        static_for<M, LM>([&](auto l) {
+          constexpr int L = decltype(l)::value, ir = L * L - 1 + 2 * M - 1, ii = ir + 1;
+          float Ar = 0.0f, Ai = 0.0f, Br = 0.0f, Bi = 0.0f;
+#pragma unroll
+          for (int n = 0; n < NA; ++n) {
+            Ar += s[n][ir] * g[n];
+            Ai += s[n][ii] * g[n];
+            Br += s[n][ir] * gp[n];
+            Bi += s[n][ii] * gp[n];
+          }
+          if constexpr (L == M) {  // Z = 1
+            R = Ar;
+            I = Ai;
+            RB = Br;
+            IB = Bi;
+          } else {
+            const float Z = harmonic_z<L, M>(pw.zp), dZ = harmonic_dz<L, M>(pw.zp);
+            R += Z * Ar;
+            I += Z * Ai;
+            RB += Z * Br;
+            IB += Z * Bi;
+            dR += dZ * Ar;
+            dI += dZ * Ai;
+          }
+        });
+        Pr += RB * pw.re[M] + IB * pw.im[M];
+        constexpr float fm = (float)M;
+        if constexpr (M == 1) {
+          Gx += R;
+          Gy += I;
+        } else {
+          Gx += fm * (R * pw.re[M - 1] + I * pw.im[M - 1]);
+          Gy += fm * (I * pw.re[M - 1] - R * pw.im[M - 1]);
+        }
+        if constexpr (M < LM) Gz += dR * pw.re[M] + dI * pw.im[M];
+      });
+    }
     const float gu = Gx * ux + Gy * uy + Gz * uz;
     const float3 fo = make_float3(Pr * ux + (Gx - gu * ux) * dinv, Pr * uy + (Gy - gu * uy) * dinv,
                                   Pr * uz + (Gz - gu * uz) * dinv);

@@ -66,6 +66,36 @@ __device__ __forceinline__ void cheb_scaled(float rcinv, float d, float h, float
   for (int k = 2; k < K; ++k) t[k] = x2 * t[k - 1] - t[k - 2];
 }
 
+// basis and d/dd (T_k' = k U_{k-1})
+template <int K>
+__device__ __forceinline__ void cheb_d(int kn, float rcinv, float d, float fc, float fcp, float* f, float* fp)
+{
+  const float t = d * rcinv - 1.0f;
+  const float x = 2.0f * t * t - 1.0f;
+  const float dx = 4.0f * t * rcinv;  // dx/dd
+  f[0] = fc;
+  fp[0] = fcp;
+  float tm2 = 1.0f, tm1 = x, um2 = 1.0f, um1 = 2.0f * x;
+  if (K > 1) {
+    const float v = 0.5f * (x + 1.0f);
+    f[1] = v * fc;
+    fp[1] = 0.5f * dx * fc + v * fcp;
+  }
+#pragma unroll
+  for (int k = 2; k < K; ++k) {
+    const float tk = 2.0f * x * tm1 - tm2;
+    const float v = 0.5f * (tk + 1.0f);
+    const float der = 0.5f * k * um1 * dx;  // (T_k'/2) dx/dd, T_k' = k U_{k-1}
+    f[k] = k < kn ? v * fc : 0.0f;
+    fp[k] = k < kn ? der * fc + v * fcp : 0.0f;
+    tm2 = tm1;
+    tm1 = tk;
+    const float uk = 2.0f * x * um1 - um2;
+    um2 = um1;
+    um1 = uk;
+  }
+}
+
 // Z_{L,m}(z) from the powers of z, and its derivative
 template <int L, int M, class Pow>
 __device__ __forceinline__ float harmonic_z(const Pow& zp)
