@@ -37,6 +37,14 @@ bool descriptor_bucket(const DevModel& m, int dims[4])
   return false;
 }
 
+DescriptorForm descriptor_form(const DevModel& m)
+{
+  for (const ExactCfg& c : kExact)
+    if (model_is(m, c.nr, c.kr, c.na, c.ka, 4, c.q2, c.q1, c.one))
+      return c.one && c.na * 24 <= kNarrowMoments ? DescriptorForm::narrow : DescriptorForm::wide;
+  return DescriptorForm::generic;
+}
+
 // Compiled in descriptor_instances.hip, one group per object file.
 extern template void run_exact<5, 9, 5, 9, true, true, true>(const DescriptorCall&);
 extern template void run_exact<7, 9, 5, 9, true, false, true>(const DescriptorCall&);

@@ -457,16 +457,17 @@ constexpr int desc_lds_bytes()
 }
 
 // Wavefronts per SIMD an instance's registers are allocated for.  Two (256
-// registers) for the single-type instances with up to 128 moments, and for the
+// registers) for the single-type instances with up to kNarrowMoments moments, and for the
 // several-type matrix-core ones whose LDS lets two workgroups share a CU (606
 // -> 461 us on 192,000 water atoms, with 84 bytes of spills per lane; four
 // lanes per atom on 21,952 carbon atoms 63 -> 44).  One for the wider ones,
 // which would spill hundreds of bytes.
+constexpr int kNarrowMoments = 128;
 template <class C, int P>
 constexpr int desc_waves()
 {
   if (!C::exact) return 1;
-  if (C::one) return C::na * C::nabc <= 128 ? 2 : 1;
+  if (C::one) return C::na * C::nabc <= kNarrowMoments ? 2 : 1;
   return P == 1 && C::ann == kAnnMfma32 && desc_lds_bytes<C>() <= 80 * 1024 ? 2 : 1;
 }
 

@@ -790,20 +790,28 @@ constexpr int kOverlapMinCentres = 16384;
 // Lanes per atom of the untuned descriptor, by the wavefronts that fill the
 // GPU's 1,024 SIMDs.  Its time steps up with each further wavefront per SIMD, so
 // a small system gains from more lanes per atom until they need another.
-// Narrow instances (one type, at most five angular functions) hold two
-// wavefronts per SIMD: sixteen lanes up to 8,192 centres (4,096 carbon atoms:
-// 23 us against 32 with four; 10,648: 39 against 34), four up to 36,864 (32,000
-// Cu atoms: 50 us against 54 with one lane; 48,668: 79 against 56).  The others
-// hold one: sixteen up to 6,144 (5,832 atoms of a 100-neuron model: 110 us
-// against 131; 10,125 water atoms: 88 against 62), four up to 57,344 (46,875
-// water atoms: 165 us against 200; 65,856: 262 against 225).
+// Narrow instances hold two wavefronts per SIMD: sixteen lanes up to 8,192
+// centres (4,096 carbon atoms: 23 us against 32 with four; 10,648: 39 against
+// 34), four up to 36,864 (32,000 Cu atoms: 50 us against 54 with one lane;
+// 48,668: 79 against 56).  The lane groups of the wide ones hold one: sixteen up
+// to 6,144 (5,832 atoms of a 100-neuron model: 110 us against 131; 10,125 water
+// atoms: 88 against 62), four up to 57,344 (46,875 water atoms: 165 us against
+// 200 with one lane; 65,856: 262 against 225).  The generic ones hold one and
+// wait for scratch: at order 4 sixteen up to 8,192 (8,000 atoms with a basis of
+// 16: 461 us against 603; 10,648: 669 against 613), four up to 49,152 (46,656:
+// 1,831 against 2,071 with one; 54,872: 2,388 against 2,084); above it sixteen
+// up to 5,120 (order 6, 4,096 atoms: 644 against 924; 5,832: 978 against 938),
+// four up to 36,864 (32,768: 2,853 against 3,042; 46,656: 3,968 against 3,121).
 struct LaneRule {
   int wide, group;
 };
-bool narrow(const DevModel& m) { return m.T == 1 && m.nA <= 5 && m.L <= kPadL; }
 LaneRule lane_rule(const DevModel& m)
 {
-  return narrow(m) ? LaneRule{8192, 36864} : LaneRule{6144, 57344};
+  switch (descriptor_form(m)) {
+    case DescriptorForm::narrow: return {8192, 36864};
+    case DescriptorForm::wide: return {6144, 57344};
+    default: return m.L <= kPadL ? LaneRule{8192, 49152} : LaneRule{5120, 36864};
+  }
 }
 
 // Lanes of the untuned filter and gather.  Up to these sizes the wavefronts of
@@ -821,19 +829,20 @@ int NepEngine::filter_lanes(int n) const
   return !tune_.lanes_set && n <= kWideFilterCentres ? 32 : tune_.filter_lanes;
 }
 
-// With one type and narrow adjoint rows four lanes are the faster from about as
-// many atoms as fill every SIMD's slots with eight: 32,768 carbon atoms 27.6 us
-// against 25.5, 39,304 33.4 against 35.1, 46,656 33.8 against 36.9, 42,592 Cu
-// atoms 22.9 against 24.5, 87,808 39.6 against 39.0, 256,000 103 against 112
-// (192,000 water atoms 216 against 213, 64,000 of a 130-neighbour model 274
-// against 250).
-constexpr int kNarrowGatherAtoms = 36864;
+// With one type and narrow adjoint rows (up to 12 basis functions) four lanes
+// are the faster from about as many atoms as fill every SIMD's slots with eight:
+// 32,768 carbon atoms 27.6 us against 25.5, 39,304 33.4 against 35.1, 46,656 33.8
+// against 36.9, 42,592 Cu atoms 22.9 against 24.5, 87,808 39.6 against 39.0,
+// 256,000 103 against 112; 110,592 atoms with 11 functions 70 against 74, with 13
+// 119 against 116, with 17 190 against 175 (192,000 water atoms 216 against 213).
+constexpr int kNarrowGatherAtoms = 36864, kNarrowGatherRow = 12;
 
 int NepEngine::gather_lanes(int n) const
 {
   if (tune_.lanes_set) return tune_.gather_lanes;
   if (n <= kWideGatherAtoms) return 16;
-  return n > kNarrowGatherAtoms && narrow(dmd_) ? 4 : tune_.gather_lanes;
+  const bool narrow = dm_.T == 1 && dm_.kRp <= kNarrowGatherRow;
+  return n > kNarrowGatherAtoms && narrow ? 4 : tune_.gather_lanes;
 }
 
 int NepEngine::desc_lanes(int n, int ann, bool split) const

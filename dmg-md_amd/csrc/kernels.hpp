@@ -232,6 +232,11 @@ hipError_t launch_split(const DevBox& b, const DevModel& m, int c1, int c2, DevW
 // blocks); false where the model has an exact instance, or exceeds every
 // padded size and runs on the generic instance.
 bool descriptor_bucket(const DevModel& m, int dims[4]);
+// the kind of instance the descriptor of m (its padded sizes) runs on: a
+// single-type exact one whose registers hold two wavefronts per SIMD at every
+// number of lanes per atom, another exact one, or a generic one
+enum class DescriptorForm { narrow, wide, generic };
+DescriptorForm descriptor_form(const DevModel& m);
 // ann: 0 FP32 on the vector ALUs, 1 FP32 on the matrix cores, 2 BF16 operands,
 // 3 split-BF16 operands (hi + lo, three MFMAs per product)
 // on the matrix cores; modes 1 and 2 apply to models of at most 2 types with

@@ -53,3 +53,38 @@ def test_generic_instances_against_oracle(dmgx, workloads, tmp_path, num_types, 
             assert e["force"] <= max(1e-4, 2e-6 * np.abs(ref["force"]).max()), (split, lanes, e)
             assert e["energy_atom_max"] <= max(2e-5, 2e-7 * np.abs(ref["pe"]).max()), (split, lanes, e)
             assert e["virial"] <= max(2e-4, 2e-6 * np.abs(ref["virial"]).max()), (split, lanes, e)
+
+
+def _cluster(n, seed=11, spacing=2.3):
+    rng = np.random.default_rng(seed)
+    m = int(np.ceil(n ** (1 / 3)))
+    g = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n].astype(float)
+    return np.ascontiguousarray((5.0 + g * spacing + rng.uniform(-0.15, 0.15, (n, 3))).T), 10.0 + m * spacing
+
+
+@pytest.mark.parametrize("n_max,basis,l_max,n,desc,gather", [
+    ((4, 4), (16, 12), (4, 2, 1), 8192, None, 16),  # None: sixteen lanes, which cannot be set
+    ((4, 4), (16, 12), (4, 2, 1), 8193, 4, 16), ((4, 4), (16, 12), (4, 2, 1), 36865, 4, 8),
+    ((4, 4), (16, 12), (4, 2, 1), 49151, 4, 8), ((4, 4), (16, 12), (4, 2, 1), 49152, 1, 8),
+    ((4, 4), (8, 8), (6, 2, 1), 5121, 4, 16), ((4, 4), (8, 8), (6, 2, 1), 36863, 4, 8),
+    ((4, 4), (8, 8), (6, 2, 1), 36865, 1, 4),
+    ((4, 4), (11, 8), (4, 2, 1), 36865, 4, 4), ((4, 4), (12, 8), (4, 2, 1), 36865, 4, 8)])
+def test_untuned_lanes_by_the_instance(dmgx, workloads, tmp_path, n_max, basis, l_max, n, desc, gather):
+    """The lanes of an untuned handle follow the kind of descriptor instance and the width of the gather's adjoint rows:
+    bit for bit the results of the lanes set by hand."""
+    path = write_model(tmp_path / "nep.txt", ["C"], n_max, basis, l_max, lattice(dmgx, workloads, 4, 1))
+    pos, edge = _cluster(n)
+    types = np.zeros(n, np.int32)
+    box = dmgx.Box.orthogonal(edge, edge, edge, pbc=(0, 0, 0))
+    untuned, by_hand = dmgx.NEP(path), dmgx.NEP(path)
+    a = gpu_compute(dmgx, untuned, box, types, pos)
+    by_hand.set_tiles(16, gather)
+    if desc:
+        by_hand.set_desc_lanes(desc)
+    b = gpu_compute(dmgx, by_hand, box, types, pos)
+    for x, y in zip(a, b):
+        assert np.array_equal(x, y)
+    if desc is None:  # neither of the others
+        for lanes in (1, 4):
+            by_hand.set_desc_lanes(lanes)
+            assert not np.array_equal(a[0], gpu_compute(dmgx, by_hand, box, types, pos)[0])
