@@ -911,10 +911,10 @@ const NepEngine::Tuning& NepEngine::autotune(const Box& box, int N, int nc, cons
   int reps[3];
   if (N <= 0 || nc <= 0 || nc > N || small_box(box, reps)) return tune_;  // small boxes keep the defaults
   flags &= ~1u;
-  tune_.lanes_set = true;  // every candidate below is what it says
   // the filter's shapes first, then the candidate rows against them
   if (w_.split) set_split(0);
   compute(box, N, 0, nc, 0, nc, type, pos, nullptr, pe, force, virial, flags, s, map);
+  tune_.lanes_set = true;  // every candidate below is what it says
   flags &= ~2u;
   // rows, edges, adjoints and partials are current: the filter rewrites its
   // outputs identically and the gather overwrites the forces, so every

@@ -1,0 +1,37 @@
+"""What the autotuner and the lane setters leave in a handle, seen through results: the FP32 sums of the descriptor
+and the FP64 sums of the gather differ in their last bits with the lanes that form them."""
+import os
+
+import numpy as np
+import pytest
+
+from conftest import POTENTIALS
+from gpu_helpers import gpu_compute, to_dev
+
+pytestmark = pytest.mark.gpu
+
+CARBON = os.path.join(POTENTIALS, "nep_carbon.txt")
+
+
+def _same(a, b):
+    return all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+def _autotune(nep, s, types, **kw):
+    import torch
+    n = len(types)
+    t, x = to_dev(types, torch.int32), to_dev(s["pos"], torch.float64)
+    out = [torch.zeros(k * n, dtype=torch.float64, device="cuda") for k in (1, 3, 9)]
+    return nep.autotune(s["box"], t, x, *out, **kw)
+
+
+def test_refused_autotune_leaves_the_lanes_by_size(dmgx, workloads):
+    s = workloads.carbon_diamond_4096(seed=4)
+    nep = dmgx.NEP(CARBON)
+    with pytest.raises(dmgx.DmgxError):
+        _autotune(nep, s, np.full(len(s["types"]), nep.num_types, np.int32))
+    fresh, by_hand = dmgx.NEP(CARBON), dmgx.NEP(CARBON)
+    by_hand.set_tiles(16, 8)
+    a, b, c = (gpu_compute(dmgx, h, s["box"], s["types"], s["pos"]) for h in (nep, fresh, by_hand))
+    assert not _same(b, c)
+    assert _same(a, b)
