@@ -1006,11 +1006,12 @@ const NepEngine::Tuning& NepEngine::autotune(const Box& box, int N, int nc, cons
     }
     tune_.overlap = t[1] < t[0] ? 1 : 0;
   }
-  // one lane per atom in the descriptor or a group (FP32 requests only)
-  tune_.desc_pinned = false;
+  // one lane per atom in the descriptor or a group (FP32 requests only; lanes
+  // that were set stay so in the others)
   {
     const int ann = ann_mode(flags);
     if (ann == 0 || ann == 1) {
+      tune_.desc_pinned = false;
       double t[2];
       for (int k = 0; k < 2; ++k) {
         tune_.desc_lanes = k ? 4 : 1;

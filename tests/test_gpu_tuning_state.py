@@ -35,3 +35,18 @@ def test_refused_autotune_leaves_the_lanes_by_size(dmgx, workloads):
     a, b, c = (gpu_compute(dmgx, h, s["box"], s["types"], s["pos"]) for h in (nep, fresh, by_hand))
     assert not _same(b, c)
     assert _same(a, b)
+
+
+def test_bfloat16_autotune_keeps_the_descriptor_lanes_set(dmgx, workloads):
+    """Autotuning BF16 requests does not time the descriptor's lanes, so exactly four stay exactly four."""
+    s = workloads.carbon_diamond_4096(seed=4)
+    nep, four, by_size = dmgx.NEP(CARBON), dmgx.NEP(CARBON), dmgx.NEP(CARBON)
+    nep.set_desc_lanes(4)
+    tune = _autotune(nep, s, s["types"], ann_bf16=True)
+    assert tune["desc_lanes"] == 4
+    four.set_desc_lanes(4)
+    if tune["split"]:
+        pytest.skip("candidate rows keep one lane per atom")
+    a, b, c = (gpu_compute(dmgx, h, s["box"], s["types"], s["pos"])[0] for h in (nep, four, by_size))
+    assert not np.array_equal(b, c)
+    assert np.array_equal(a, b)
