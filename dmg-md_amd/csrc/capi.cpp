@@ -223,7 +223,7 @@ int dmgx_nep_get_tuning(const dmgx_nep* nep, dmgx_tuning* out)
 {
   return guarded([&] {
     if (!nep || !out) throw std::invalid_argument("null argument");
-    fill_tuning(nep->engine.tuning(), out);
+    fill_tuning(nep->engine.launched_tuning(), out);
   });
 }
 

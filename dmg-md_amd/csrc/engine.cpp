@@ -587,6 +587,7 @@ void NepEngine::launch_force(const Plan& p, int N, int n1, int n2, int nd1, int 
   last_N_stats_ = N;
   last_c1_ = nd1;
   last_c2_ = nd2;
+  last_forces_ = n2 - n1;
 }
 
 void NepEngine::adopt_carried(const Box& box, int N, int n_owned, int c_keep, int g_keep, const int* type,
@@ -843,6 +844,14 @@ int NepEngine::gather_lanes(int n) const
   if (n <= kWideGatherAtoms) return 16;
   const bool narrow = dm_.T == 1 && dm_.kRp <= kNarrowGatherRow;
   return n > kNarrowGatherAtoms && narrow ? 4 : tune_.gather_lanes;
+}
+
+NepEngine::Tuning NepEngine::launched_tuning() const
+{
+  Tuning t = tune_;
+  if (last_c2_ > last_c1_) t.filter_lanes = filter_lanes(last_c2_ - last_c1_);
+  if (last_forces_ > 0) t.gather_lanes = gather_lanes(last_forces_);
+  return t;
 }
 
 int NepEngine::desc_lanes(int n, int ann, bool split) const

@@ -164,6 +164,8 @@ class NepEngine {
     bool tuned = false;
   };
   const Tuning& tuning() const { return tune_; }
+  // the same with the filter and gather lanes that the last evaluation launched
+  Tuning launched_tuning() const;
   // Sets the shapes directly (rejects other values); marks them tuned, so
   // a server does not re-tune them
   void set_tiles(int filter_lanes, int gather_lanes);
@@ -265,7 +267,7 @@ class NepEngine {
   DevBox last_box_{};  // box of the last evaluation (the filter of copy_pair_rows)
   hipStream_t side_ = nullptr;  // the overlapped filter's stream
   hipEvent_t fork_ = nullptr, join_ = nullptr;
-  int last_N_stats_ = 0, last_c1_ = 0, last_c2_ = 0;
+  int last_N_stats_ = 0, last_c1_ = 0, last_c2_ = 0, last_forces_ = 0;
   Profiler prof_;
   // replicated small-box system (atoms x replicas)
   long long sb_cap_ = 0;

@@ -177,7 +177,7 @@ class NEP:
         return out
 
     def tuning(self) -> dict:
-        """Tile shapes the per-step kernels use (and the autotuner's timings)."""
+        """Tile shapes the last evaluation's per-step kernels used (and the autotuner's timings)."""
         t = _lib.Tuning()
         check(lib().dmgx_nep_get_tuning(self._h, ctypes.byref(t)))
         return _tuning_dict(t)

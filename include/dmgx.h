@@ -160,9 +160,11 @@ int dmgx_nep_profile_reset(dmgx_nep* nep);
  * rounded up to a multiple of 4 (layout 0) or to a power of two (layout 1;
  * -1 before tuning, when the power of two is taken where it costs at most
  * 1.25x), with the filter + descriptor + gather time of each layout the
- * autotuner timed.  Defaults 16 and 8, taken around the middle of the sizes
- * (untuned small systems launch 32 and 16, large single-type ones 4 in the
- * gather); tuned = 1 once the autotuner has run.
+ * autotuner timed.  Untuned lanes go by system size: 16 and 8 around the
+ * middle of the sizes (and before the first evaluation), 32 and 16 in small
+ * systems, 4 in the gather of large single-type ones; dmgx_nep_get_tuning
+ * gives those of the last evaluation, which dmgx_nep_set_tiles would pin.
+ * tuned = 1 once the autotuner has run.
  * Boxes small enough to be replicated keep the defaults. */
 typedef struct dmgx_tuning {
   int filter_lanes, gather_lanes;

@@ -50,3 +50,22 @@ def test_bfloat16_autotune_keeps_the_descriptor_lanes_set(dmgx, workloads):
     a, b, c = (gpu_compute(dmgx, h, s["box"], s["types"], s["pos"])[0] for h in (nep, four, by_size))
     assert not np.array_equal(b, c)
     assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("cells,lanes", [(4, (32, 16)), (10, (16, 16)), (12, (16, 8)), (17, (16, 4))])
+def test_reported_lanes_are_those_launched(dmgx, workloads, cells, lanes):
+    """An untuned handle reports the lanes that its last evaluation launched, so that pinning what it reports changes
+    nothing."""
+    s = workloads.vacancy_lattice("carbon", cells, np.random.default_rng(3), vacancies=False)
+    nep, pinned = dmgx.NEP(CARBON), dmgx.NEP(CARBON)
+    t = nep.tuning()
+    assert (t["filter_lanes"], t["gather_lanes"]) == (16, 8)
+    a = gpu_compute(dmgx, nep, s["box"], s["types"], s["pos"])
+    t = nep.tuning()
+    assert (t["filter_lanes"], t["gather_lanes"], t["tuned"]) == (*lanes, False)
+    pinned.set_tiles(t["filter_lanes"], t["gather_lanes"])
+    assert _same(a, gpu_compute(dmgx, pinned, s["box"], s["types"], s["pos"]))
+    nep.set_tiles(8, 4)
+    gpu_compute(dmgx, nep, s["box"], s["types"], s["pos"])
+    t = nep.tuning()
+    assert (t["filter_lanes"], t["gather_lanes"]) == (8, 4)
