@@ -409,8 +409,9 @@ void Server::make_pack(Request& rq, const int* type, const double* mass, const d
     K[d] = box.pbc[d] ? (int)std::ceil(d1 / th[d]) : 0;
     if (K[d] > kImageMax) throw std::invalid_argument("request box too thin for its periodic image shell");
   }
-  // every image within d1 of the box (per face pair: a lower bound of the
-  // Euclidean distance, so the shell is a superset of what the rows need);
+  // every image within d1 of the box (per periodic face pair: a lower bound of
+  // the distance to every owned atom, which may lie anywhere along an open
+  // direction, so the shell is a superset of what the rows need);
   // an owned atom's Verlet neighbours at any rebuild lie within
   // rc + skin of the box plus the request's motion, covered by the margin
   // (an atom's images in increasing image code, c then b then a: the
@@ -425,13 +426,11 @@ void Server::make_pack(Request& rq, const int* type, const double* mass, const d
     double x[3] = {pos[i], pos[N + i], pos[2 * N + i]}, s[3];
     to_frac(r->hi, x, s);
     long long count = 1;
-    bool self = true;  // the atom itself is no image of its own
     for (int d = 0; d < 3; ++d) {
       if (!std::isfinite(s[d])) throw std::invalid_argument("non-finite position");
       if (box.pbc[d] && !(s[d] > 0.0 && s[d] < 1.0)) s[d] -= std::floor(s[d]);
       // the distance grows with |k|, so the first offset out of reach ends a side
-      unsigned bits = std::max(0.0, std::max(-s[d], s[d] - 1.0)) * th[d] > d1 ? 0u : 1u << kImageMax;
-      self = self && bits;
+      unsigned bits = 1u << kImageMax;
       for (int k = 1; k <= K[d]; ++k) {
         if ((s[d] + k - 1.0) * th[d] > d1) break;
         bits |= 1u << (kImageMax + k);
@@ -444,7 +443,7 @@ void Server::make_pack(Request& rq, const int* type, const double* mass, const d
       count *= __builtin_popcount(bits);
     }
     g_first[i] = (int)images;
-    images += count - (self ? 1 : 0);
+    images += count - 1;  // the atom itself is no image of its own
     if (images >= (1LL << 30)) throw std::invalid_argument("request has too many periodic images");
     to_cart(box.h, s, x);
     for (int d = 0; d < 3; ++d) wpos[(size_t)d * N + i] = x[d];
