@@ -1,6 +1,6 @@
 """Models beyond the padded descriptor sizes (more radial functions, wider bases or higher 3-body orders): the generic
 descriptor instances on every number of lanes per atom and on the candidate rows, against the FP64 oracle at the bars
-of the parity tests."""
+of the parity tests; and the lanes that untuned handles of each kind of instance take."""
 import numpy as np
 import pytest
 
@@ -68,7 +68,11 @@ def _cluster(n, seed=11, spacing=2.3):
     ((4, 4), (16, 12), (4, 2, 1), 49151, 4, 8), ((4, 4), (16, 12), (4, 2, 1), 49152, 1, 8),
     ((4, 4), (8, 8), (6, 2, 1), 5121, 4, 16), ((4, 4), (8, 8), (6, 2, 1), 36863, 4, 8),
     ((4, 4), (8, 8), (6, 2, 1), 36865, 1, 4),
-    ((4, 4), (11, 8), (4, 2, 1), 36865, 4, 4), ((4, 4), (12, 8), (4, 2, 1), 36865, 4, 8)])
+    ((4, 4), (11, 8), (4, 2, 1), 36865, 4, 4), ((4, 4), (12, 8), (4, 2, 1), 36865, 4, 8),
+    ((4, 4), (12, 8), (4, 2, 1), 6144, None, 16), ((4, 4), (12, 8), (4, 2, 1), 6145, 4, 16),
+    ((4, 4), (12, 8), (4, 2, 1), 57343, 4, 8), ((4, 4), (12, 8), (4, 2, 1), 57344, 1, 8),
+    ((4, 4), (8, 8), (4, 2, 1), 8192, None, 16), ((4, 4), (8, 8), (4, 2, 1), 8193, 4, 16),
+    ((4, 4), (8, 8), (4, 2, 1), 36863, 4, 8), ((4, 4), (8, 8), (4, 2, 1), 36865, 1, 4)])
 def test_untuned_lanes_by_the_instance(dmgx, workloads, tmp_path, n_max, basis, l_max, n, desc, gather):
     """The lanes of an untuned handle follow the kind of descriptor instance and the width of the gather's adjoint rows:
     bit for bit the results of the lanes set by hand."""
