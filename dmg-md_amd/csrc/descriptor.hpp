@@ -457,11 +457,12 @@ constexpr int desc_lds_bytes()
 }
 
 // Wavefronts per SIMD an instance's registers are allocated for.  Two (256
-// registers) for the single-type instances with up to kNarrowMoments moments, and for the
+// registers) for the single-type instances with up to kNarrowMoments moments
+// (four lanes per atom on 21,952 carbon atoms 63 -> 44 us), and for the
 // several-type matrix-core ones whose LDS lets two workgroups share a CU (606
-// -> 461 us on 192,000 water atoms, with 84 bytes of spills per lane; four
-// lanes per atom on 21,952 carbon atoms 63 -> 44).  One for the wider ones,
-// which would spill hundreds of bytes.
+// -> 461 us on 192,000 water atoms, with 84 bytes of spills per lane).  One for
+// the wider ones, which would spill hundreds of bytes, for the lane groups of
+// several-type models and for the generic instances.
 constexpr int kNarrowMoments = 128;
 template <class C, int P>
 constexpr int desc_waves()
@@ -475,7 +476,8 @@ template <int NR, int KR, int NA, int KA, bool Q2, bool Q1, bool ONE, int ANN = 
 constexpr bool mfma_ann_fits()
 {
   // single-type instances reach two wavefronts per SIMD, so they keep two
-  // workgroups per CU (64 KiB each); multi-type ones run one either way
+  // workgroups per CU (64 KiB each); several-type ones hold two wavefronts up to
+  // 80 KiB (desc_waves) and, on the matrix cores all the same, one beyond
   return desc_lds_bytes<Cfg<NR, KR, NA, KA, 4, Q2, Q1, ONE, true, ANN, !ONE>>() <=
          (ONE ? 64 * 1024 : kDescLdsMax);
 }
@@ -550,10 +552,14 @@ __device__ __forceinline__ void contract_by_degree(const float (&s)[NA][NABC], c
 // activations are branch-free: with the matrix-core ANN above, 228 -> 191 us on
 // 256,000 Cu atoms, 713 -> 611 us on 192,000 water atoms and 2.03 -> 1.73 ms on
 // a 2.28-million-slot carbon share; with four lanes per atom 45 -> 37 us on
-// 4,096 carbon atoms.  Errors against 64 bits are those of the longer form or
-// smaller (folding the constant column of c into one coefficient would save
-// 16 more additions per edge, but its rounding is common to all edges and
-// raised the water model's energy error by a fifth).
+// 4,096 carbon atoms (32 with the registers of two wavefronts, 22 with sixteen
+// lanes).  Against 64 bits the other order of the FP32 sums moves the errors by
+// a few percent either way (2-norms over six draws of four systems): site
+// energies 0.2 to 4% smaller, forces and virials of carbon and Cu 0.2 to 2.7%
+// smaller, of BaTiO3 1.5 and 3.6% larger; the short tanh is no part of that (the
+// library's in its place: within 1%).  Folding the constant column of c into one
+// coefficient would save 16 more additions per edge, but its rounding is common
+// to all edges and raised the water model's energy error by a fifth.
 //
 // CAND: the edges come from the candidate rows (DevWork::split).  edge, vsa
 // and eq are w.edge, w.vsa and w.eq, passed as restrict parameters: with

@@ -4,7 +4,7 @@
 //  * Verlet list with a 1 A skin, rebuilt only when an atom moved more than
 //    skin/2 (neighbor.cu:446-582); rows hold slot indices, sorted ascending
 //    (or by global id), with a precomputed reverse position per entry.
-//  * Every step a filter pass (16 or 32 lanes per centre, ballot compaction) turns
+//  * Every step a filter pass (8, 16 or 32 lanes per centre, ballot compaction) turns
 //    each Verlet row into one compact edge row: angular edges first (slots
 //    0..na-1, ascending), radial-only edges from the end of the row
 //    downward, each edge a float4 (FP64 minimum-image r_ij rounded to float,
@@ -15,7 +15,7 @@
 //    partial forces: the angular moments s[n][lm] stay in registers, are
 //    turned in place into the adjoint dE/ds, and each angular edge's
 //    dE_i/dr_ij is written at i's slot.
-//  * The gather kernel (8 or 16 lanes per atom) forms the radial pair force from
+//  * The gather kernel (4, 8 or 16 lanes per atom) forms the radial pair force from
 //    both centres' basis-space adjoints, adds the angular partials of both
 //    directions (dE_j/dr_ji read from j's row through the reverse index) and
 //    ZBL, and writes FP64 force/virial.  No floating-point atomics anywhere:

@@ -1,7 +1,7 @@
 // kernels.hpp -- device-side structures and launch wrappers of the NEP step.
 //
-// All kernels live in kernels.hip (one translation unit, so the __constant__
-// angular tables are shared); host code calls the launch_* wrappers below.
+// The kernels live in kernels.hip, descriptor.hpp (instances compiled in
+// groups) and neighbor.hip; host code calls the launch_* wrappers below.
 #pragma once
 
 #include <hip/hip_runtime.h>

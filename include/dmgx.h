@@ -165,7 +165,7 @@ int dmgx_nep_profile_reset(dmgx_nep* nep);
  * systems, 4 in the gather of large single-type ones; dmgx_nep_get_tuning
  * gives those of the last evaluation, which dmgx_nep_set_tiles would pin.
  * tuned = 1 once the autotuner has run.
- * Boxes small enough to be replicated keep the defaults. */
+ * Boxes small enough to be replicated are not tuned. */
 typedef struct dmgx_tuning {
   int filter_lanes, gather_lanes;
   double filter_ms[3]; /* candidates 8, 16, 32 */

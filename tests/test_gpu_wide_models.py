@@ -21,7 +21,8 @@ def write_model(path, symbols, n_max, basis, l_max, sample, cutoff=(4.2, 3.7), n
             f"basis_size {basis[0]} {basis[1]}", "l_max " + " ".join(map(str, l_max)), f"ANN {neurons} 0"]
 
     def save(scaler):
-        path.write_text("\n".join(head + [f"{np.float32(v):.9e}" for v in np.concatenate([weights, coeffs, scaler])]) + "\n")
+        values = np.concatenate([weights, coeffs, scaler])
+        path.write_text("\n".join(head + [f"{np.float32(v):.9e}" for v in values]) + "\n")
 
     save(np.ones(dim))
     box, types, pos = sample
