@@ -632,7 +632,8 @@ void NepEngine::launch_key(std::vector<long long>& k) const
                         (const void*)w.flags, (const void*)w.partial, (const void*)w.thermo})
     p(q);
   for (int v : {tune_.filter_lanes, tune_.gather_lanes, tune_.row_layout, tune_.overlap, tune_.split,
-                tune_.desc_lanes, (int)tune_.desc_pinned, (int)tune_.lanes_set})
+                tune_.desc_lanes, (int)tune_.desc_pinned, tune_.desc_centres,
+                (int)tune_.lanes_set})
     k.push_back(v);
 }
 
@@ -859,7 +860,12 @@ int NepEngine::desc_lanes(int n, int ann, bool split) const
   if (split || (ann != 1 && ann != 0)) return 1;  // candidate rows, or BF16 operands asked for
   if (tune_.desc_pinned) return tune_.desc_lanes;
   const LaneRule rule = lane_rule(dmd_);
-  const int lanes = tune_.desc_lanes ? tune_.desc_lanes : n < rule.group ? 4 : 1;
+  int lanes = tune_.desc_lanes ? tune_.desc_lanes : n < rule.group ? 4 : 1;
+  // a group tuned on one system is not taken for a larger one past the rule's
+  // limit: a server tunes on its first batch of 65,536 atoms, where the two are
+  // within 3%, and goes on to batches of a million (carbon lane of the serving
+  // stream 2,020 -> 915 us a launch, 3% more frames)
+  if (n > tune_.desc_centres && n >= rule.group) lanes = 1;
   return lanes == 4 && n <= rule.wide ? 16 : lanes;
 }
 
@@ -1021,6 +1027,7 @@ const NepEngine::Tuning& NepEngine::autotune(const Box& box, int N, int nc, cons
     const int ann = ann_mode(flags);
     if (ann == 0 || ann == 1) {
       tune_.desc_pinned = false;
+      tune_.desc_centres = nc;
       double t[2];
       for (int k = 0; k < 2; ++k) {
         tune_.desc_lanes = k ? 4 : 1;

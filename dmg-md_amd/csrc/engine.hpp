@@ -160,6 +160,7 @@ class NepEngine {
     // lane per atom.
     int desc_lanes = 0;
     bool desc_pinned = false;           // desc_lanes was set, not tuned
+    int desc_centres = 0;               // centres that desc_lanes was tuned on
     double desc_ms[2] = {0, 0};         // the step's force kernels with 1 / 4 lanes per atom
     bool tuned = false;
   };

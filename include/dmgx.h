@@ -184,8 +184,9 @@ typedef struct dmgx_tuning {
   int desc_lanes;       /* lanes per atom of the descriptor: 1, 4 (a group of lanes shares
                            an atom's edges and hidden neurons, four or, in the smallest
                            systems unless set, sixteen; FP32 ANN on the vector ALUs), 0
-                           before tuning (a group in small systems, else one); BF16 ANN
-                           requests keep one */
+                           before tuning (a group in small systems, else one); a tuned
+                           group is not taken for larger systems than it was tuned on
+                           past those sizes; BF16 ANN requests keep one */
   double desc_ms[2];    /* the step's force kernels with 1 / 4 lanes per atom */
 } dmgx_tuning;
 int dmgx_nep_get_tuning(const dmgx_nep* nep, dmgx_tuning* out);

@@ -69,3 +69,18 @@ def test_reported_lanes_are_those_launched(dmgx, workloads, cells, lanes):
     gpu_compute(dmgx, nep, s["box"], s["types"], s["pos"])
     t = nep.tuning()
     assert (t["filter_lanes"], t["gather_lanes"]) == (8, 4)
+
+
+def test_tuned_descriptor_group_is_not_taken_for_larger_systems(dmgx, workloads):
+    """Four lanes per atom tuned on 39,304 atoms stay for them; 110,592 atoms take one lane, as the rule by size has
+    it."""
+    small, large = (workloads.vacancy_lattice("carbon", c, np.random.default_rng(3), vacancies=False) for c in (17, 24))
+    nep = dmgx.NEP(CARBON)
+    tune = _autotune(nep, small, small["types"])
+    if tune["desc_lanes"] != 4 or tune["split"]:
+        pytest.skip("the autotuner chose no group here")
+    pinned = dmgx.NEP(CARBON)
+    for s, lanes in ((small, 4), (large, 1)):
+        pinned.set_desc_lanes(lanes)
+        a, b = (gpu_compute(dmgx, h, s["box"], s["types"], s["pos"])[0] for h in (nep, pinned))
+        assert np.array_equal(a, b), lanes
