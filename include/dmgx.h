@@ -108,7 +108,7 @@ int dmgx_nep_compute(dmgx_nep* nep, const dmgx_box* box, int N, int n1, int n2, 
  * every per-atom workspace carved from a fixed 128 MiB device array that the
  * library holds on each GPU until the process ends.  It calls no hipMalloc,
  * hipFree or allocating library routine.  Limits and differences:
- *   - the system must fit the fixed workspace (about 17,000 slots of a model
+ *   - the system must fit the fixed workspace (about 23,000 slots of a model
  *     with rows of 152 entries); larger systems get DMGX_EINVAL with the
  *     sizes in the message;
  *   - Verlet rows hold the capacity MN_radial implies (no growth): a longer
