@@ -642,13 +642,12 @@ bool NepEngine::small_box(const Box& box, int reps[3]) const
   const DevBox b = make_devbox(box);
   const double need = 2.5 * (model_.rcR_max + kSkin);
   bool any = false;
-  for (int d = 0; d < 3; ++d) {
-    reps[d] = 1;
-    if (b.pbc[d] && b.thick[d] <= need) {
-      reps[d] = (int)std::floor(need / b.thick[d]) + 1;
-      any = true;
-    }
-  }
+  for (int d = 0; d < 3; ++d) any = any || (b.pbc[d] && b.thick[d] <= need);
+  // the supercell's thickness has to exceed the need when it is computed anew,
+  // where a multiple that equals it may be rounded down
+  const double over = need * (1.0 + 1e-12);
+  for (int d = 0; d < 3; ++d)
+    reps[d] = any && b.pbc[d] && b.thick[d] <= over ? (int)std::floor(over / b.thick[d]) + 1 : 1;
   return any;
 }
 
